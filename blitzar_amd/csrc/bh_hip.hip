@@ -10,6 +10,7 @@
 #include "bh_internal.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -17,6 +18,8 @@
 #include <numeric>
 #include <random>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -24,6 +27,13 @@ namespace {
 constexpr int kDefaultWavesPerCu = 24;
 constexpr float kDefaultRelativeAlpha = 0.002f;
 constexpr size_t kStackCap = 16384;
+// copy_out: slots of the pinned ring, largest and smallest chunk, and the
+// threads that empty the ring of a large copy (the caller's own not counted)
+constexpr size_t kRingSlots = 8;
+constexpr size_t kRingChunk = 2u << 20;
+constexpr size_t kRingChunkMin = 256u << 10;
+constexpr int kCopyThreads = 4;
+constexpr size_t kCopyThreadsMin = 4u << 20;
 
 // b0 build start, s0 sort start (after AABB + keys), s1 sort end, p1 after
 // the tie fix and permutation, t1 after the tree levels, b1 build end (after
@@ -73,6 +83,10 @@ struct bh_hip_handle {
     hipEvent_t ev_sorted = nullptr, ev_topo = nullptr, ev_groups = nullptr;
     int err_carry = 0;      // error bits of this call kept across a node regrow
     int steps_done = -1;    // bh_hip_step: steps completed before an error stopped it
+    // pinned ring of copy_out (allocated at the first copy, sized for it)
+    char* pinned = nullptr;
+    size_t pinned_bytes = 0;
+    hipEvent_t ring_ev[kRingSlots] = {};
     // Test switch (environment BH_HIP_TEST_FAIL_NODE_GROWTH at creation): a
     // node regrow asks for an impossible size, so the failed-allocation path
     // runs for real.
@@ -303,6 +317,115 @@ bool zero_err(bh_hip_handle* h)
     h->err_carry = 0;
     bh::launch_fill_u32(reinterpret_cast<uint32_t*>(h->d.err), 0u, 1, h->d.stream);
     return check(h, hipGetLastError(), "error flag reset");
+}
+
+// Device memory to pageable caller memory. The runtime's own copy of pageable
+// memory drains its staging buffer with one host thread, 10 GB/s into memory
+// the caller has not touched yet (the thread takes the page faults). Here the
+// link fills a pinned ring (57 GB/s) while up to kCopyThreads host threads
+// empty it: 38 GB/s for a 100 MB array on untouched huge pages, 14 GB/s on
+// untouched 4 KB pages (4 threads; 8 are no faster on huge pages). Copies below
+// kCopyThreadsMin are emptied by the calling thread alone: starting the
+// others costs about 0.1 ms, what a 4 MB copy gains. The threads end before
+// the call returns.
+bool copy_out(bh_hip_handle* h, void* dst, const void* src, size_t bytes, const char* what)
+{
+    if (bytes == 0)
+        return true;
+    const hipStream_t st = h->d.stream;
+    const size_t chunk =
+        std::clamp((bytes / kRingSlots + 4095) & ~static_cast<size_t>(4095), kRingChunkMin,
+                   kRingChunk);
+    const size_t nchunks = (bytes + chunk - 1) / chunk;
+    const size_t ring = std::min(nchunks, kRingSlots) * chunk;
+    if (h->pinned_bytes < ring) {
+        if (h->pinned)
+            (void)hipHostFree(h->pinned);
+        h->pinned = nullptr;
+        h->pinned_bytes = 0;
+        if (!check(h, hipHostMalloc(reinterpret_cast<void**>(&h->pinned), ring,
+                                    hipHostMallocDefault),
+                   "pinned copy buffer")) {
+            (void)hipGetLastError();
+            return false;
+        }
+        h->pinned_bytes = ring;
+    }
+    for (hipEvent_t& e : h->ring_ev)
+        if (!e && !check(h, hipEventCreateWithFlags(&e, hipEventDisableTiming), "event"))
+            return false;
+
+    std::atomic<size_t> landed{0};  // chunks whose bytes are in the ring
+    std::atomic<size_t> next{0};    // next chunk to move out
+    std::atomic<bool> failed{false};
+    std::atomic<size_t> emptied[kRingSlots];  // 1 + last chunk moved out of the slot
+    for (auto& e : emptied)
+        e.store(0, std::memory_order_relaxed);
+    char* const out = static_cast<char*>(dst);
+    const auto move_out = [&](size_t k) {
+        const size_t off = k * chunk;
+        std::memcpy(out + off, h->pinned + (k % kRingSlots) * chunk, std::min(chunk, bytes - off));
+        emptied[k % kRingSlots].store(k + 1, std::memory_order_release);
+    };
+    const auto worker = [&]() {
+        for (;;) {
+            const size_t k = next.fetch_add(1);
+            if (k >= nchunks)
+                return;
+            while (landed.load(std::memory_order_acquire) <= k) {
+                if (failed.load(std::memory_order_relaxed))
+                    return;
+                std::this_thread::yield();
+            }
+            move_out(k);
+        }
+    };
+    std::thread pool[kCopyThreads];
+    int nthreads = 0;
+    if (bytes >= kCopyThreadsMin) {
+        try {
+            for (; nthreads < kCopyThreads; ++nthreads)
+                pool[nthreads] = std::thread(worker);
+        } catch (const std::system_error&) {
+            // no (more) threads: those that started do it, or the caller alone
+        }
+    }
+    bool ok = true;
+    size_t issued = 0;
+    for (size_t done = 0; ok && done < nchunks; ++done) {
+        // fill every free slot, then wait for the oldest chunk under way
+        while (ok && issued < nchunks && issued < done + kRingSlots) {
+            const size_t slot = issued % kRingSlots;
+            if (issued >= kRingSlots &&
+                emptied[slot].load(std::memory_order_acquire) != issued - kRingSlots + 1) {
+                if (issued > done)
+                    break;
+                std::this_thread::yield();
+                continue;
+            }
+            const size_t off = issued * chunk;
+            ok = check(h, hipMemcpyAsync(h->pinned + slot * chunk,
+                                         static_cast<const char*>(src) + off,
+                                         std::min(chunk, bytes - off), hipMemcpyDeviceToHost, st),
+                       what) &&
+                 check(h, hipEventRecord(h->ring_ev[slot], st), what);
+            ++issued;
+        }
+        ok = ok && check(h, hipEventSynchronize(h->ring_ev[done % kRingSlots]), what);
+        if (!ok)
+            break;
+        if (nthreads > 0)
+            landed.store(done + 1, std::memory_order_release);
+        else
+            move_out(done);
+    }
+    if (!ok)
+        failed.store(true);
+    for (int i = 0; i < nthreads; ++i)
+        pool[i].join();
+    if (!ok)
+        (void)hipStreamSynchronize(st);  // nothing may still write the ring
+    return ok;
 }
 
 // Device errors that no retry repairs (a node-capacity overflow is repaired
@@ -872,11 +995,9 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
     return r;
 }
 
-bool stage_to_device(bh_hip_handle* h, const double* src3)
+bool stage_to_device(bh_hip_handle* h, const void* src, size_t bytes)
 {
-    return check(h,
-                 hipMemcpyAsync(h->d.stage, src3, 3 * h->d.n * sizeof(double),
-                                hipMemcpyHostToDevice, h->d.stream),
+    return check(h, hipMemcpyAsync(h->d.stage, src, bytes, hipMemcpyHostToDevice, h->d.stream),
                  "stage upload");
 }
 
@@ -1012,6 +1133,11 @@ void bh_hip_destroy(bh_hip_handle_t* h)
             (void)hipEventDestroy(x);
     if (h->err_host)
         (void)hipHostFree(h->err_host);
+    for (hipEvent_t x : h->ring_ev)
+        if (x)
+            (void)hipEventDestroy(x);
+    if (h->pinned)
+        (void)hipHostFree(h->pinned);
     if (h->d.stream)
         (void)hipStreamDestroy(h->d.stream);
     if (h->side)
@@ -1068,41 +1194,25 @@ bh_hip_result_t bh_hip_upload(bh_hip_handle_t* h, const double* pos3, const doub
     if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     bh::Device& d = h->d;
-    // The store keeps its current order; rank maps caller index -> slot.
-    std::vector<float> m_sorted;
-    ensure_rank(h);
-    bool ok = zero_err(h) && stage_to_device(h, pos3);
+    // The store keeps its current order; each slot picks its caller index. One
+    // staging buffer serves the three arrays in stream order (each copy lands
+    // after the kernel that read the buffer before it); the call waits for the
+    // stream before it returns, so the caller's arrays are free then.
+    bool ok = zero_err(h) && stage_to_device(h, pos3, 3 * d.n * sizeof(double));
     if (ok) {
-        bh::launch_upload_scatter(d, 0);
+        bh::launch_from_caller(d, 0);
         bh::launch_wrap(d, h->p.periodic_box);
-        ok = check(h, hipStreamSynchronize(d.stream), "upload pos");
+        if (vel3)
+            ok = stage_to_device(h, vel3, 3 * d.n * sizeof(double));
+        else
+            bh::launch_fill_u32(reinterpret_cast<uint32_t*>(d.stage), 0u, 6 * d.n, d.stream);
     }
     if (ok) {
-        if (vel3) {
-            ok = stage_to_device(h, vel3);
-        } else {
-            ok = check(h, hipMemsetAsync(d.stage, 0, 3 * d.n * sizeof(double), d.stream),
-                       "zero velocities");
-        }
+        bh::launch_from_caller(d, 1);
+        ok = stage_to_device(h, mass, d.n * sizeof(float));
     }
-    if (ok) {
-        bh::launch_upload_scatter(d, 1);
-        ok = check(h, hipStreamSynchronize(d.stream), "upload vel");
-    }
-    if (ok) {
-        // Masses: reorder on the host by the store's id map.
-        std::vector<uint32_t> id(d.n);
-        ok = check(h, hipMemcpy(id.data(), d.id, d.n * sizeof(uint32_t), hipMemcpyDeviceToHost),
-                   "id read");
-        if (ok) {
-            m_sorted.resize(d.n);
-            for (size_t s = 0; s < d.n; ++s)
-                m_sorted[s] = mass[id[s]];
-            ok = check(h, hipMemcpy(d.mass, m_sorted.data(), d.n * sizeof(float),
-                                    hipMemcpyHostToDevice),
-                       "mass upload");
-        }
-    }
+    if (ok)
+        bh::launch_from_caller(d, 2);
     h->primed = false;
     h->ad_primed = false;
     h->have_tree = false;
@@ -1119,16 +1229,12 @@ bh_hip_result_t bh_hip_download(bh_hip_handle_t* h, double* pos3, double* vel3)
     if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     bh::Device& d = h->d;
-    ensure_rank(h);
     for (int which = 0; which < 2; ++which) {
         double* dst = which == 0 ? pos3 : vel3;
         if (!dst)
             continue;
-        bh::launch_download_gather(d, which);
-        if (!check(h, hipMemcpyAsync(dst, d.stage, 3 * d.n * sizeof(double),
-                                     hipMemcpyDeviceToHost, d.stream),
-                   "download") ||
-            !check(h, hipStreamSynchronize(d.stream), "download"))
+        bh::launch_to_caller(d, which);
+        if (!copy_out(h, dst, d.stage, 3 * d.n * sizeof(double), "download"))
             return BH_HIP_INTERNAL_ERROR;
     }
     return BH_HIP_OK;
@@ -1172,17 +1278,9 @@ bh_hip_result_t bh_hip_compute_accelerations(bh_hip_handle_t* h, float* acc3)
     end_call(h);
     if (r != BH_HIP_OK || !acc3)
         return r;
-    bh::Device& d = h->d;
-    ensure_rank(h);
-    bh::launch_download_gather(d, 2);
-    std::vector<double> tmp(3 * d.n);
-    if (!check(h, hipMemcpyAsync(tmp.data(), d.stage, tmp.size() * sizeof(double),
-                                 hipMemcpyDeviceToHost, d.stream),
-               "acc download") ||
-        !check(h, hipStreamSynchronize(d.stream), "acc download"))
+    bh::launch_to_caller(h->d, 2);
+    if (!copy_out(h, acc3, h->d.stage, 3 * h->d.n * sizeof(float), "acc download"))
         return BH_HIP_INTERNAL_ERROR;
-    for (size_t i = 0; i < tmp.size(); ++i)
-        acc3[i] = static_cast<float>(tmp[i]);
     return BH_HIP_OK;
 }
 
@@ -1905,15 +2003,8 @@ extern "C" bh_hip_result_t bh_hip_pm_accelerations(bh_hip_handle_t* h, float* ac
     bh_hip_result_t r = finish(h, "pm_accelerations");
     if (r != BH_HIP_OK)
         return r;
-    ensure_rank(h);
-    bh::launch_download_gather(d, 2);
-    std::vector<double> tmp(3 * d.n);
-    if (!check(h, hipMemcpyAsync(tmp.data(), d.stage, tmp.size() * sizeof(double),
-                                 hipMemcpyDeviceToHost, d.stream),
-               "pm download") ||
-        !check(h, hipStreamSynchronize(d.stream), "pm download"))
+    bh::launch_to_caller(d, 2);
+    if (!copy_out(h, acc3, d.stage, 3 * d.n * sizeof(float), "pm download"))
         return BH_HIP_INTERNAL_ERROR;
-    for (size_t i = 0; i < tmp.size(); ++i)
-        acc3[i] = static_cast<float>(tmp[i]);
     return BH_HIP_OK;
 }

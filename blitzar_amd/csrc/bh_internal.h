@@ -352,8 +352,10 @@ void launch_kick(Device& d, double dt_kick, double max_speed);
 void launch_kick_drift(Device& d, double dt_kick, double dt_drift, double max_speed,
                        double box = 0.0);
 void launch_wrap(Device& d, double box);
-void launch_upload_scatter(Device& d, int which);   // 0 = pos, 1 = vel
-void launch_download_gather(Device& d, int which);  // 0 = pos, 1 = vel, 2 = acc(float->double)
+// caller-ordered stage -> store (0 = pos, 1 = vel: FP64 triples; 2 = mass: FP32)
+void launch_from_caller(Device& d, int which);
+// store -> caller-ordered stage (0 = pos, 1 = vel: FP64 triples; 2 = acc: FP32 triples)
+void launch_to_caller(Device& d, int which);
 void launch_init_ids(Device& d);
 void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, double eps,
                         double min_d2, double* out_dev);

@@ -123,14 +123,14 @@ class OctreeHip:
         _check(lib().bh_hip_upload(self._h, pos, vel, mass), self._h, "upload")
 
     def download(self):
-        pos = np.zeros((self.n, 3), np.float64)
-        vel = np.zeros((self.n, 3), np.float64)
+        pos = np.empty((self.n, 3), np.float64)
+        vel = np.empty((self.n, 3), np.float64)
         _check(lib().bh_hip_download(self._h, pos, vel), self._h, "download")
         return pos, vel
 
     # -- force pass and stepping -----------------------------------------------
     def compute_accelerations(self, to_host: bool = True):
-        acc = np.zeros((self.n, 3), np.float32) if to_host else None
+        acc = np.empty((self.n, 3), np.float32) if to_host else None
         _check(lib().bh_hip_compute_accelerations(self._h, acc), self._h,
                "compute_accelerations")
         return acc
@@ -181,7 +181,7 @@ class OctreeHip:
 
     def direct_forces_fp64(self, targets) -> np.ndarray:
         t = np.ascontiguousarray(targets, np.uint32)
-        out = np.zeros((t.size, 3), np.float64)
+        out = np.empty((t.size, 3), np.float64)
         _check(lib().bh_hip_direct_forces_fp64(self._h, t, t.size, out.reshape(-1)), self._h,
                "direct_forces_fp64")
         return out
@@ -202,7 +202,7 @@ class OctreeHip:
 
     def pm_accelerations(self) -> np.ndarray:
         """Long-range (mesh) part of the periodic TreePM force (caller order)."""
-        out = np.zeros((self.n, 3), np.float32)
+        out = np.empty((self.n, 3), np.float32)
         _check(lib().bh_hip_pm_accelerations(self._h, out.reshape(-1)), self._h,
                "pm_accelerations")
         return out
