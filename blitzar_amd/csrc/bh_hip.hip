@@ -26,7 +26,6 @@ namespace {
 
 constexpr int kDefaultWavesPerCu = 24;
 constexpr float kDefaultRelativeAlpha = 0.002f;
-constexpr size_t kStackCap = 16384;
 // copy_out: slots of the pinned ring, largest and smallest chunk, and the
 // threads that empty the ring of a large copy (the caller's own not counted)
 constexpr size_t kRingSlots = 8;
@@ -304,11 +303,16 @@ bool alloc_all(bh_hip_handle* h, uint64_t n)
     if (!alloc_nodes(h, 2 * n + 4096))
         return false;
     // resident walk waves: one per group of the smallest cap (16, see
-    // group_max) up to the residency limit
-    const size_t groups = (n + 15) / 16;
+    // group_max), four where walks may give a group four, up to the residency
+    // limit
+    const size_t cus = static_cast<size_t>(h->cu_count);
+    d.walk_slots = cus * static_cast<size_t>(kDefaultWavesPerCu);
+    const size_t usual = bh::walk_groups_usual(n, 16);
+    const bool four = static_cast<float>(usual) <=
+                      bh::kWalkFourWaves * static_cast<float>(d.walk_slots);
     d.stack_waves = std::max<size_t>(
-        1, std::min(groups, static_cast<size_t>(h->cu_count) * static_cast<size_t>(h->p.waves_per_cu)));
-    d.stack_cap = std::min(kStackCap, d.node_cap + 64);
+        8, std::min(four ? 4 * usual : usual, cus * static_cast<size_t>(h->p.waves_per_cu)));
+    d.stack_cap = std::min(bh::kStackCap, d.node_cap + 64);
     return dalloc(h, &d.stack, d.stack_waves * d.stack_cap, "walk stacks");
 }
 
@@ -606,8 +610,10 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
     rec(ev ? ev->t1 : nullptr, h->side);
     (void)hipEventRecord(h->ev_topo, h->side);
     bh::launch_permute_rest(d, h->side);
-    if (h->p.key_mode == 0)
-        bh::launch_groups(d, group_max(h), h->side);
+    if (h->p.key_mode == 0) {
+        d.group_cap = group_max(h);
+        bh::launch_groups(d, d.group_cap, h->side);
+    }
     (void)hipEventRecord(h->ev_groups, h->side);
     bh::launch_permute_store(d, d.stream);
     rec(ev ? ev->p1 : nullptr, d.stream);

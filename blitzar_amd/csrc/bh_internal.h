@@ -20,6 +20,19 @@ constexpr int kInfoBig = 2 * kLevels + 3;       // large nodes of the current le
 // AABB: per-block partial extrema (6 doubles per block) in Device::diag.
 constexpr int kAabbBlocks = 1024;
 
+// Groups that n particles usually make: groups fill to 0.72 of their cap.
+inline size_t walk_groups_usual(size_t n, size_t cap) { return n * 25 / (cap * 18) + 1; }
+// COM and relative walks give each group four waves up to this many groups per
+// resident wave (walk_waves in k_walk.hip).
+constexpr float kWalkFourWaves = 0.47f;
+
+// Deepest traversal stack per wave. Entries lie on the stack in order of level,
+// deepest on top, and a step pops the top T = 64 of them: when nodes of level
+// l are opened nothing deeper stays below their children, so each of the 21
+// levels leaves at most 7 T entries behind and the last push adds 8 T. (W waves
+// that pop 64 W share W regions.)
+constexpr size_t kStackCap = 64 * (7 * 21 + 8);
+
 // Walk tickets: one counter per XCD (workgroup i runs on XCD i mod 8), each
 // on its own 256-byte line.
 constexpr int kTicketQueues = 8;
@@ -221,6 +234,8 @@ struct Device {
     int* stack = nullptr;  // per-resident-wave traversal stacks
     size_t stack_waves = 0;
     size_t stack_cap = 0;
+    size_t walk_slots = 0;          // waves a walk keeps resident on this GPU (by default)
+    uint32_t group_cap = kGroupMax;  // walk-group size of the last build
 
     // block time steps (allocated on the first adaptive step; permuted with
     // the store): acceleration of the last force evaluation, level, tick of

@@ -55,8 +55,15 @@ namespace {
 #ifndef BH_WALK_PART_CAP
 #define BH_WALK_PART_CAP 96
 #endif
-constexpr int kCellCap = BH_WALK_CELL_CAP;
-constexpr int kPartCap = BH_WALK_PART_CAP;
+// Walks of W waves per group append up to 64 W entries per step, so their
+// lists grow with W.
+template <int W>
+struct WalkCaps {
+    static constexpr int kCell = W == 1 ? BH_WALK_CELL_CAP : 64 * W + 64;
+    static constexpr int kPart = W == 1 ? BH_WALK_PART_CAP : 64 * W + 64;
+    // stack entries below this depth live in LDS (W > 1)
+    static constexpr int kLdsStack = W == 1 ? 0 : 256 * W;
+};
 
 // Group tickets. On large walks (at least kQueueMinGroupsPerWave groups per
 // resident wave) the walk order is cut into chunks of kTicketChunk
@@ -292,31 +299,31 @@ __device__ inline void eval_parts_dj(const float4* __restrict__ pl, int np, int 
     }
 }
 
-template <int ORDER, bool TPM>
+template <int ORDER, bool TPM, int W>
 __device__ inline void eval_cells(const float4* __restrict__ ca, const float4* __restrict__ cb,
                                   const float2* __restrict__ cc, int ncell, int j0, int dj,
                                   float tx, float ty, float tz, const WalkParams& P, float& ax,
                                   float& ay, float& az)
 {
     if (dj == 1)
-        eval_cells_dj<ORDER, TPM, 1>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
+        eval_cells_dj<ORDER, TPM, W>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
     else if (dj == 2)
-        eval_cells_dj<ORDER, TPM, 2>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
+        eval_cells_dj<ORDER, TPM, 2 * W>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
     else
-        eval_cells_dj<ORDER, TPM, 4>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
+        eval_cells_dj<ORDER, TPM, 4 * W>(ca, cb, cc, ncell, j0, tx, ty, tz, P, ax, ay, az);
 }
 
-template <bool TPM>
+template <bool TPM, int W>
 __device__ inline void eval_parts(const float4* __restrict__ pl, int np, int j0, int dj, float tx,
                                   float ty, float tz, const WalkParams& P, float& ax, float& ay,
                                   float& az)
 {
     if (dj == 1)
-        eval_parts_dj<TPM, 1>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+        eval_parts_dj<TPM, W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
     else if (dj == 2)
-        eval_parts_dj<TPM, 2>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+        eval_parts_dj<TPM, 2 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
     else
-        eval_parts_dj<TPM, 4>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+        eval_parts_dj<TPM, 4 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
 }
 
 // Group far field: the local (Taylor) expansion about the group centre of an
@@ -433,13 +440,22 @@ __device__ inline void far_flush(const uint32_t* __restrict__ fl, int nfl,
     }
 }
 
-template <int ORDER, int CRIT, bool TPM, bool REC, bool FAR>
+// W waves walk one group together (W > 1: small walks, see walk_waves). They
+// pop up to 64 W nodes per step, share the lists in LDS, take every W-th
+// entry of them each and add their shares of a target's force in wave order at
+// the end, so results do not depend on timing. The nodes accepted and opened
+// are those of the one-wave walk. Bound: latency (a step is one round trip for
+// its nodes, one for the particles of opened leaves and 4 barriers, about 3.5 us
+// for 256 nodes with 4 waves; about 10 steps per group at 4,096 particles).
+// Issuing a step's node loads before the evaluation of the step before it
+// changed nothing with 4 waves and cost 10 % with 2.
+template <int ORDER, int CRIT, bool TPM, bool REC, bool FAR, int W>
 #ifndef BH_WALK_MIN_WAVES
 #define BH_WALK_MIN_WAVES 5
 #endif
 // Walks without the far field are held to 96 VGPRs (5 waves per SIMD): the
 // traversal is latency-bound and needs the resident waves.
-__global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
+__global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) void walk_kernel(
     WalkParams P, const WalkNode* __restrict__ nodes, const float4* __restrict__ spart,
     const uint32_t* __restrict__ sleaf, const RootGeom* __restrict__ geom,
     const uint4* __restrict__ groups, const int* __restrict__ info,
@@ -449,17 +465,29 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
     uint32_t* __restrict__ rec_n, int rec_cap, int rec_groups, float rec_band2,
     uint32_t rec_min_count)
 {
+    static_assert(W == 1 || !FAR, "the group far field walks with one wave");
+    constexpr int kCellCap = WalkCaps<W>::kCell;
+    constexpr int kPartCap = WalkCaps<W>::kPart;
+    constexpr int kLdsStack = WalkCaps<W>::kLdsStack;
+    constexpr int kThreads = 64 * W;
     __shared__ float4 cA[kCellCap];
     __shared__ float4 cB[kCellCap];
     __shared__ float2 cC[kCellCap];
     __shared__ float4 pl[kPartCap];
-    __shared__ int lfFirst[64];
-    __shared__ uint32_t lfPre[64];
-    __shared__ float lfSx[64], lfSy[64], lfSz[64];
+    __shared__ int lfFirst[kThreads];
+    __shared__ uint32_t lfPre[kThreads];
+    __shared__ float lfSx[kThreads], lfSy[kThreads], lfSz[kThreads];
+    __shared__ int lstk[W > 1 ? kLdsStack : 1];
+    __shared__ uint32_t wtot[W > 1 ? W : 1][6];  // per wave: totals of one step
+    __shared__ int sticket;
     __shared__ uint32_t fl[FAR ? kFarCap : 1];
     __shared__ float fsum[FAR ? kFarTerms : 1];
 
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wv =
+        W == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    // W waves share W stack regions
+    stack_cap *= W;
     int* stk = stack_all + static_cast<size_t>(blockIdx.x) * static_cast<size_t>(stack_cap);
     const float ux = geom->unit_f[0], uy = geom->unit_f[1], uz = geom->unit_f[2];
     const float wfx = geom->width_f[0], wfy = geom->width_f[1], wfz = geom->width_f[2];
@@ -486,7 +514,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
     int drained = 0;
     for (;;) {
         int t = ngroups;
-        if (lane == 0) {
+        if (threadIdx.x == 0) {
             for (;;) {
                 t = ticket_position(atomicAdd(&work[queue * kTicketStride], 1u), queue, nq);
                 if (t < ngroups || drained == nq - 1)
@@ -495,6 +523,13 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                 queue = (queue + 1) % nq;
             }
             t = t < ngroups ? t : ngroups;
+        }
+        if (W > 1) {
+            __syncthreads();  // every wave has read the ticket before
+            if (threadIdx.x == 0)
+                sticket = t;
+            __syncthreads();
+            t = sticket;
         }
         // the whole wave is active here, so the first lane is lane 0
         const int ticket = __builtin_amdgcn_readfirstlane(t);
@@ -525,7 +560,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
             const unsigned long long dm = __ballot(due);
             if (dm == 0ull)
                 continue;
-            if (due)
+            if (due && wv == 0)
                 lfFirst[__popcll(dm & lt)] = lane;
             nact = static_cast<int>(__popcll(dm));
             __syncthreads();
@@ -535,7 +570,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
         const int dj = nact <= 16 ? 4 : (nact <= 32 ? 2 : 1);
         const int tw = 64 / dj;  // lanes per list share
         const int tl = lane & (tw - 1);
-        const int j0 = lane / tw;
+        const int j0 = lane / tw + dj * wv;
         const bool active = tl < nact;
         const int s = static_cast<int>(gr.x) + (P.alevel ? (active ? lfFirst[tl] : 0) : tl);
         const bool target = active;
@@ -576,8 +611,12 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
         int ncell = 0, npart = 0;
         int nrec = 0;
         int sp = 1;
-        if (lane == 0)
-            stk[0] = 0;  // root
+        if (threadIdx.x == 0) {
+            if (W > 1)
+                lstk[0] = 0;
+            else
+                stk[0] = 0;  // root
+        }
         __syncthreads();
 
         // Every iteration pops at least one node and a node is pushed at most
@@ -586,13 +625,17 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
         int iters = 0;
         while (sp > 0) {
             if (++iters > node_cap) {
-                if (lane == 0)
+                if (threadIdx.x == 0)
                     atomicOr(err, kErrStackOverflow);
                 break;
             }
-            const int take = sp < 64 ? sp : 64;
+            const int take = sp < kThreads ? sp : kThreads;
             sp -= take;
-            int node = lane < take ? stk[sp + lane] : -1;
+            int node = -1;
+            if (static_cast<int>(threadIdx.x) < take) {
+                const int at = sp + static_cast<int>(threadIdx.x);
+                node = W > 1 && at < kLdsStack ? lstk[W > 1 ? at : 0] : stk[at];
+            }
             if (node >= node_cap) {
                 atomicOr(err, kErrStackOverflow);
                 node = -1;
@@ -694,8 +737,21 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
             if (REC) {
                 near = near && accept;
                 const unsigned long long rm = __ballot(near);
+                int nnear = static_cast<int>(__popcll(rm));
+                int before = 0;  // near nodes of the waves before this one
+                if (W > 1) {
+                    if (lane == 0)
+                        wtot[wv][5] = static_cast<uint32_t>(nnear);
+                    __syncthreads();
+                    nnear = 0;
+#pragma unroll
+                    for (int k = 0; k < W; ++k) {
+                        before += k < wv ? static_cast<int>(wtot[k][5]) : 0;
+                        nnear += static_cast<int>(wtot[k][5]);
+                    }
+                }
                 if (near) {
-                    const int slot = nrec + static_cast<int>(__popcll(rm & lt));
+                    const int slot = nrec + before + static_cast<int>(__popcll(rm & lt));
                     if (slot < rec_cap) {
                         rec_lists[static_cast<size_t>(g) * rec_cap + slot] =
                             static_cast<uint32_t>(node);
@@ -709,7 +765,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                         open = nch != 0;
                     }
                 }
-                nrec += static_cast<int>(__popcll(rm));
+                nrec += nnear;
             }
 
             if (FAR) {
@@ -733,62 +789,98 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                 nfar += __popcll(fm);
             }
 
-            // 1) accepted nodes -> LDS cell list (point masses -> particle list)
+            // What this step adds: counts per wave, then (W > 1) the offsets of
+            // the waves before.
             if (CRIT == 3) {
                 mono = mono && accept;
                 accept = accept && !mono;
-                const unsigned long long mm = __ballot(mono);
-                const int nm = static_cast<int>(__popcll(mm));
-                if (nm > 0) {
-                    if (npart + nm >= kPartCap) {  // uniform; keeps npart < kPartCap
-                        eval_parts<TPM>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
-                        npp += static_cast<unsigned long long>(npart);
-                        npart = 0;
-                        __syncthreads();
-                    }
-                    if (mono)
-                        pl[npart + static_cast<int>(__popcll(mm & lt))] =
-                            make_float4(px, py, pz, w.mass);
-                    npart += nm;
-                    nmono += static_cast<unsigned long long>(nm);
+            }
+            const unsigned long long mm = CRIT == 3 ? __ballot(mono) : 0ull;
+            const unsigned long long am = __ballot(accept);
+            const unsigned long long dm = __ballot(direct);
+            const uint32_t nc = open ? meta_nchild(w.meta) : 0u;
+            const uint32_t lc = direct ? meta_count(w.meta) : 0u;
+            const uint32_t cinc = winclusive(nc);
+            const uint32_t linc = winclusive(lc);
+            int nm = static_cast<int>(__popcll(mm)), na = static_cast<int>(__popcll(am));
+            int nd = static_cast<int>(__popcll(dm));
+            int ctot = static_cast<int>(wlast(cinc));
+            uint32_t ltot = wlast(linc);
+            int om = 0, oa = 0, od = 0, oc = 0;
+            uint32_t ol = 0;
+            if (W > 1) {
+                if (lane == 0) {
+                    wtot[wv][0] = static_cast<uint32_t>(nm);
+                    wtot[wv][1] = static_cast<uint32_t>(na);
+                    wtot[wv][2] = static_cast<uint32_t>(nd);
+                    wtot[wv][3] = static_cast<uint32_t>(ctot);
+                    wtot[wv][4] = ltot;
+                }
+                __syncthreads();
+                nm = na = nd = ctot = 0;
+                ltot = 0;
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    const bool prior = k < wv;
+                    om += prior ? static_cast<int>(wtot[k][0]) : 0;
+                    oa += prior ? static_cast<int>(wtot[k][1]) : 0;
+                    od += prior ? static_cast<int>(wtot[k][2]) : 0;
+                    oc += prior ? static_cast<int>(wtot[k][3]) : 0;
+                    ol += prior ? wtot[k][4] : 0u;
+                    nm += static_cast<int>(wtot[k][0]);
+                    na += static_cast<int>(wtot[k][1]);
+                    nd += static_cast<int>(wtot[k][2]);
+                    ctot += static_cast<int>(wtot[k][3]);
+                    ltot += wtot[k][4];
                 }
             }
-            const unsigned long long am = __ballot(accept);
+
+            // 1) accepted nodes -> LDS cell list (point masses -> particle list)
+            if (CRIT == 3 && nm > 0) {
+                if (npart + nm >= kPartCap) {  // uniform; keeps npart < kPartCap
+                    eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+                    npp += static_cast<unsigned long long>(npart);
+                    npart = 0;
+                    __syncthreads();
+                }
+                if (mono)
+                    pl[npart + om + static_cast<int>(__popcll(mm & lt))] =
+                        make_float4(px, py, pz, w.mass);
+                npart += nm;
+                nmono += static_cast<unsigned long long>(nm);
+            }
             if (accept) {
-                const int slot = ncell + static_cast<int>(__popcll(am & lt));
+                const int slot = ncell + oa + static_cast<int>(__popcll(am & lt));
                 cA[slot] = make_float4(px, py, pz, w.mass);
                 cB[slot] = make_float4(w.qxx, w.qxy, w.qxz, w.qyy);
                 // the open walk's expansion needs eps^2 trs, the TreePM one trs
                 cC[slot] = make_float2(w.qyz, TPM ? w.trs : P.eps2 * w.trs);
             }
-            ncell += static_cast<int>(__popcll(am));
+            ncell += na;
 
             // 2) children of opened nodes -> traversal stack
-            const uint32_t nc = open ? meta_nchild(w.meta) : 0u;
-            const uint32_t cinc = winclusive(nc);
-            const int ctot = static_cast<int>(wlast(cinc));
             if (sp + ctot > stack_cap) {
-                if (lane == 0)
+                if (threadIdx.x == 0)
                     atomicOr(err, kErrStackOverflow);
             } else {
                 if (open) {
-                    const int base = sp + static_cast<int>(cinc - nc);
-                    for (uint32_t j = 0; j < nc; ++j)
-                        stk[base + static_cast<int>(j)] = w.first + static_cast<int>(j);
+                    const int base = sp + oc + static_cast<int>(cinc - nc);
+                    for (uint32_t j = 0; j < nc; ++j) {
+                        const int at = base + static_cast<int>(j);
+                        if (W > 1 && at < kLdsStack)
+                            lstk[W > 1 ? at : 0] = w.first + static_cast<int>(j);
+                        else
+                            stk[at] = w.first + static_cast<int>(j);
+                    }
                 }
                 sp += ctot;
             }
 
             // 3) opened leaves -> descriptors, then their particles -> LDS
-            const unsigned long long dm = __ballot(direct);
-            const int nd = static_cast<int>(__popcll(dm));
-            const uint32_t lc = direct ? meta_count(w.meta) : 0u;
-            const uint32_t linc = winclusive(lc);
-            const uint32_t ltot = wlast(linc);
             if (direct) {
-                const int slot = static_cast<int>(__popcll(dm & lt));
+                const int slot = od + static_cast<int>(__popcll(dm & lt));
                 lfFirst[slot] = w.first;
-                lfPre[slot] = linc - lc;
+                lfPre[slot] = ol + linc - lc;
                 lfSx[slot] = sx;
                 lfSy[slot] = sy;
                 lfSz[slot] = sz;
@@ -800,8 +892,8 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                 nfl = 0;
             }
 
-            if (ncell > kCellCap - 64) {
-                eval_cells<ORDER, TPM>(cA, cB, cC, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
+            if (ncell > kCellCap - kThreads) {
+                eval_cells<ORDER, TPM, W>(cA, cB, cC, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
                 npc += static_cast<unsigned long long>(ncell);
                 ncell = 0;
                 __syncthreads();
@@ -811,7 +903,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
             while (done < ltot) {
                 const uint32_t room = static_cast<uint32_t>(kPartCap - npart);
                 const uint32_t chunk = ltot - done < room ? ltot - done : room;
-                for (uint32_t f = static_cast<uint32_t>(lane); f < chunk; f += 64u) {
+                for (uint32_t f = threadIdx.x; f < chunk; f += static_cast<uint32_t>(kThreads)) {
                     const uint32_t gi = done + f;
                     int lo = 0, hi = nd - 1;
                     while (lo < hi) {
@@ -829,21 +921,37 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                 npart += static_cast<int>(chunk);
                 done += chunk;
                 if (npart == kPartCap) {
-                    eval_parts<TPM>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+                    eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
                     npp += static_cast<unsigned long long>(npart);
                     npart = 0;
                     __syncthreads();
                 }
             }
         }
-        eval_cells<ORDER, TPM>(cA, cB, cC, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
-        eval_parts<TPM>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+        eval_cells<ORDER, TPM, W>(cA, cB, cC, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
+        eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
         npc += static_cast<unsigned long long>(ncell);
         npp += static_cast<unsigned long long>(npart);
         for (int o = 32; o >= tw; o >>= 1) {  // the list shares of one target
             ax += __shfl_xor(ax, o, 64);
             ay += __shfl_xor(ay, o, 64);
             az += __shfl_xor(az, o, 64);
+        }
+        if (W > 1) {
+            // the waves' shares, in wave order (the lists are free now)
+            __syncthreads();
+            if (wv > 0)
+                cA[(wv - 1) * 64 + lane] = make_float4(ax, ay, az, 0.0f);
+            __syncthreads();
+            if (wv == 0) {
+#pragma unroll
+                for (int k = 0; k < W - 1; ++k) {
+                    const float4 v = cA[k * 64 + lane];
+                    ax += v.x;
+                    ay += v.y;
+                    az += v.z;
+                }
+            }
         }
         if (FAR) {
             // the rest of the queue, then the group's expansion at each target
@@ -869,7 +977,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
         }
         npp = 0;
         npc = 0;
-        if (REC && lane == 0 && g < rec_groups)
+        if (REC && threadIdx.x == 0 && g < rec_groups)
             rec_n[g] = static_cast<uint32_t>(nrec < rec_cap ? nrec : rec_cap);
         __syncthreads();
 
@@ -889,7 +997,7 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
                 P.amag[s] = sqrtf(ax * ax + ay * ay + az * az);
         }
     }
-    if (stats && lane == 0) {
+    if (stats && threadIdx.x == 0) {
         atomicAdd(&stats[0], tot_pp);
         atomicAdd(&stats[1], tot_pc);
         if (CRIT == 3 && tot_mono)
@@ -901,17 +1009,78 @@ __global__ __launch_bounds__(64, FAR ? 1 : BH_WALK_MIN_WAVES) void walk_kernel(
     }
 }
 
-template <int ORDER, int CRIT, bool TPM, bool REC = false, bool FAR = false>
-void launch_walk_t(Device& d, const WalkParams& p, unsigned grid, unsigned long long* stats,
-                   const LffState* L = nullptr, float band = 0.0f, int min_count = 0)
+// Waves per group. A walk keeps about `slots` waves resident (walk_slots, 24
+// per CU). With fewer groups than that its time is the latency of its heaviest
+// group, which W waves cut: they test 64 W nodes per step and split the lists.
+// Past that point the chip is full and the steps' barriers only cost (2 waves
+// per group: 5-20 % on the COM walk of 80,000 particles and more). Walk times
+// in us with 1 / 2 / 4 / 8 waves (Plummer, theta 0.5; slots = 6,144):
+//   COM, cap 16       4,099: 167 / 97 / 72 / 85     32,768: 394 / 278 / 262 / 398
+//                    65,536: 600 / 561 / 588 / 906 100,003: 656 / 689 / 767 / -
+//   bounds, cap 64   20,000: 979 / 513 / 378 / 221 100,000: 1284 / 941 / 759 / 906
+//                   300,001: 2844 / 2550 / 2530 / 3154
+//   relative        100,000: 374 / 286 / 296 / 616 260,000: 557 / 502 / 668 / -
+//                   500,000: 578 / 587 / 756 / -
+//   periodic TreePM  64^3:   492 / 450 / 541 / 881  128^3: 2250 / 2274 / 2505 / -
+// The relative and TreePM walks, whose lists take longer per entry or flush
+// more often, gain from 2 waves up to 3.5 groups per slot. COM runs keep one
+// wave from 0.47 groups per slot on and under block time steps: adding a
+// target's terms in another order moves its FP32 force by 2e-7 (4,096
+// particles) to 5e-7 (65,536), which an FP64 state integrated over tens of steps
+// shows (1.6e-9 of the velocities after 20 steps at 65,536), for 7 % of the walk
+// there. The count depends on n, the criterion and the GPU only; the recording
+// walk takes the plain one's, so that an idle correction changes no bit.
+int walk_waves(const Device& d, const WalkParams& p)
 {
-    walk_kernel<ORDER, CRIT, TPM, REC, FAR><<<grid, 64, 0, d.stream>>>(
+    const float slots = static_cast<float>(d.walk_slots);
+    const float G = static_cast<float>(walk_groups_usual(d.n, d.group_cap));
+    if (p.alevel)
+        return 1;
+    if (p.criterion == 1 || p.criterion == 2)
+        return 8.0f * G <= slots ? 8 : G <= 1.1f * slots ? 4 : 1;
+    if (G <= kWalkFourWaves * slots)
+        return 4;
+    return (p.criterion == 3 || p.rs > 0.0f) && G <= 3.5f * slots ? 2 : 1;
+}
+
+template <int W, int ORDER, int CRIT, bool TPM, bool REC, bool FAR>
+void launch_walk_w(Device& d, const WalkParams& p, unsigned long long* stats, const LffState* L,
+                   float band, int min_count)
+{
+    // W waves per workgroup, each with a stack region; no more workgroups than
+    // the groups n particles usually make (idle ones only draw tickets)
+    const unsigned grid = static_cast<unsigned>(
+        std::max<size_t>(std::min(d.stack_waves / W, walk_groups_usual(d.n, d.group_cap)), 1));
+    walk_kernel<ORDER, CRIT, TPM, REC, FAR, W><<<grid, 64 * W, 0, d.stream>>>(
         p, d.wnode, d.spart, d.sleaf, d.geom, d.groups, d.level_info,
         static_cast<int>(d.node_cap), d.work_counter,
         d.stack, static_cast<int>(d.stack_cap), d.acc[0], d.acc[1], d.acc[2], d.err, stats,
         L ? L->lists : nullptr, L ? L->list_n : nullptr, L ? L->list_cap : 0,
         L ? static_cast<int>(L->list_groups) : 0, band * band,
         static_cast<uint32_t>(min_count > 0 ? min_count : 0));
+}
+
+template <int ORDER, int CRIT, bool TPM, bool REC = false, bool FAR = false>
+void launch_walk_t(Device& d, const WalkParams& p, unsigned long long* stats,
+                   const LffState* L = nullptr, float band = 0.0f, int min_count = 0)
+{
+    if constexpr (!FAR) {
+        switch (walk_waves(d, p)) {
+        case 8:
+            if constexpr (CRIT == 1 || CRIT == 2)
+                return launch_walk_w<8, ORDER, CRIT, TPM, REC, FAR>(d, p, stats, L, band, min_count);
+            break;
+        case 4:
+            return launch_walk_w<4, ORDER, CRIT, TPM, REC, FAR>(d, p, stats, L, band, min_count);
+        case 2:
+            if constexpr (CRIT == 0 || CRIT == 3)
+                return launch_walk_w<2, ORDER, CRIT, TPM, REC, FAR>(d, p, stats, L, band, min_count);
+            break;
+        default:
+            break;
+        }
+    }
+    launch_walk_w<1, ORDER, CRIT, TPM, REC, FAR>(d, p, stats, L, band, min_count);
 }
 
 }  // namespace
@@ -922,13 +1091,12 @@ void launch_walk_record(Device& d, const WalkParams& p, unsigned long long* stat
     if (d.n == 0)
         return;
     launch_fill_u32(d.work_counter, 0u, kTicketWords, d.stream);
-    const unsigned grid = static_cast<unsigned>(d.stack_waves);
     if (p.criterion == 1)
-        launch_walk_t<2, 1, false, true>(d, p, grid, stats, &L, band, min_count);
+        launch_walk_t<2, 1, false, true>(d, p, stats, &L, band, min_count);
     else if (p.criterion == 2)
-        launch_walk_t<2, 2, false, true>(d, p, grid, stats, &L, band, min_count);
+        launch_walk_t<2, 2, false, true>(d, p, stats, &L, band, min_count);
     else
-        launch_walk_t<2, 0, false, true>(d, p, grid, stats, &L, band, min_count);
+        launch_walk_t<2, 0, false, true>(d, p, stats, &L, band, min_count);
 }
 
 void launch_walk(Device& d, const WalkParams& p, unsigned long long* stats)
@@ -936,48 +1104,47 @@ void launch_walk(Device& d, const WalkParams& p, unsigned long long* stats)
     if (d.n == 0)
         return;
     launch_fill_u32(d.work_counter, 0u, kTicketWords, d.stream);
-    const unsigned grid = static_cast<unsigned>(d.stack_waves);
     const bool tpm = p.rs > 0.0f;
     if (p.far2 > 0.0f && !tpm && p.order >= 2) {
         // quadrupole walk with the group far-field expansion
         if (p.criterion == 1)
-            launch_walk_t<2, 1, false, false, true>(d, p, grid, stats);
+            launch_walk_t<2, 1, false, false, true>(d, p, stats);
         else if (p.criterion == 2)
-            launch_walk_t<2, 2, false, false, true>(d, p, grid, stats);
+            launch_walk_t<2, 2, false, false, true>(d, p, stats);
         else if (p.criterion == 3)
-            launch_walk_t<2, 3, false, false, true>(d, p, grid, stats);
+            launch_walk_t<2, 3, false, false, true>(d, p, stats);
         else
-            launch_walk_t<2, 0, false, false, true>(d, p, grid, stats);
+            launch_walk_t<2, 0, false, false, true>(d, p, stats);
         return;
     }
     if (p.criterion == 3) {
         if (p.order >= 2)
-            tpm ? launch_walk_t<2, 3, true>(d, p, grid, stats)
-                : launch_walk_t<2, 3, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<2, 3, true>(d, p, stats)
+                : launch_walk_t<2, 3, false>(d, p, stats);
         else
-            tpm ? launch_walk_t<1, 3, true>(d, p, grid, stats)
-                : launch_walk_t<1, 3, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<1, 3, true>(d, p, stats)
+                : launch_walk_t<1, 3, false>(d, p, stats);
     } else if (p.criterion == 2) {
         if (p.order >= 2)
-            tpm ? launch_walk_t<2, 2, true>(d, p, grid, stats)
-                : launch_walk_t<2, 2, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<2, 2, true>(d, p, stats)
+                : launch_walk_t<2, 2, false>(d, p, stats);
         else
-            tpm ? launch_walk_t<1, 2, true>(d, p, grid, stats)
-                : launch_walk_t<1, 2, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<1, 2, true>(d, p, stats)
+                : launch_walk_t<1, 2, false>(d, p, stats);
     } else if (p.order >= 2) {
         if (p.criterion == 1)
-            tpm ? launch_walk_t<2, 1, true>(d, p, grid, stats)
-                : launch_walk_t<2, 1, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<2, 1, true>(d, p, stats)
+                : launch_walk_t<2, 1, false>(d, p, stats);
         else
-            tpm ? launch_walk_t<2, 0, true>(d, p, grid, stats)
-                : launch_walk_t<2, 0, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<2, 0, true>(d, p, stats)
+                : launch_walk_t<2, 0, false>(d, p, stats);
     } else {
         if (p.criterion == 1)
-            tpm ? launch_walk_t<1, 1, true>(d, p, grid, stats)
-                : launch_walk_t<1, 1, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<1, 1, true>(d, p, stats)
+                : launch_walk_t<1, 1, false>(d, p, stats);
         else
-            tpm ? launch_walk_t<1, 0, true>(d, p, grid, stats)
-                : launch_walk_t<1, 0, false>(d, p, grid, stats);
+            tpm ? launch_walk_t<1, 0, true>(d, p, stats)
+                : launch_walk_t<1, 0, false>(d, p, stats);
     }
 }
 
