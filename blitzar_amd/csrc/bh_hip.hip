@@ -1460,20 +1460,28 @@ bh_hip_result_t bh_hip_direct_forces_fp64(bh_hip_handle_t* h, const uint32_t* ta
             h->last_error = "direct_forces_fp64: target index out of range";
             return BH_HIP_INVALID_ARGUMENT;
         }
-    uint32_t* dt = nullptr;
-    double* dout = nullptr;
-    bool ok = dalloc(h, &dt, nt, "targets") && dalloc(h, &dout, 3 * static_cast<size_t>(nt), "out");
-    ok = ok && check(h, hipMemcpy(dt, targets, nt * 4, hipMemcpyHostToDevice), "targets");
+    // workspace and targets in the staging buffer when they fit
+    bh::Device& d = h->d;
+    const size_t words = bh::direct_fp64_words(d.n, nt);
+    const size_t need = words + (static_cast<size_t>(nt) + 1) / 2;
+    double* ws = d.stage;
+    const bool own = need > 3 * d.n;
+    bool ok = !own || dalloc(h, &ws, need, "direct sum");
     if (ok) {
+        uint32_t* dt = reinterpret_cast<uint32_t*>(ws + words);
         ensure_rank(h);
-        bh::launch_direct_fp64(h->d, dt, nt, h->p.softening, h->p.min_distance2, dout);
-        ok = check(h, hipGetLastError(), "direct launch") &&
-             check(h, hipStreamSynchronize(h->d.stream), "direct") &&
-             check(h, hipMemcpy(acc3, dout, 3 * static_cast<size_t>(nt) * 8, hipMemcpyDeviceToHost),
-                   "direct out");
+        ok = check(h, hipMemcpyAsync(dt, targets, nt * sizeof(uint32_t), hipMemcpyHostToDevice,
+                                     d.stream),
+                   "targets");
+        if (ok) {
+            bh::launch_direct_fp64(d, dt, nt, h->p.softening, h->p.min_distance2, ws);
+            ok = check(h, hipGetLastError(), "direct launch") &&
+                 copy_out(h, acc3, ws, 3 * static_cast<size_t>(nt) * sizeof(double), "direct out");
+        }
+        (void)hipStreamSynchronize(d.stream);
     }
-    dfree(h, dt);
-    dfree(h, dout);
+    if (own)
+        dfree(h, ws);
     return ok ? BH_HIP_OK : BH_HIP_INTERNAL_ERROR;
 }
 

@@ -372,8 +372,11 @@ void launch_from_caller(Device& d, int which);
 // store -> caller-ordered stage (0 = pos, 1 = vel: FP64 triples; 2 = acc: FP32 triples)
 void launch_to_caller(Device& d, int which);
 void launch_init_ids(Device& d);
+// FP64 direct sum; ws_dev holds direct_fp64_words(n, nt) doubles, the result
+// (3 per target) first.
+size_t direct_fp64_words(size_t n, uint32_t nt);
 void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, double eps,
-                        double min_d2, double* out_dev);
+                        double min_d2, double* ws_dev);
 void launch_energy(Device& d, double* out_dev);
 void launch_potential(Device& d, const uint32_t* slots_dev, uint32_t ns, double eps,
                       double min_d2, double* out_dev);

@@ -1,0 +1,38 @@
+"""The FP64 direct sum over target tiles and source ranges against the oracle's."""
+import numpy as np
+import pytest
+
+import blitzar_amd as B
+
+pytestmark = pytest.mark.gpu
+
+
+# tiles of 8 targets (one, one short, one over, many, more than n), source
+# ranges of at least 1,024 (one range, ragged ones, 8 and more), a workspace
+# that fits the staging buffer and one that does not; with softening, and
+# without it, where coincident pairs and pairs below min_distance2 are skipped
+@pytest.mark.parametrize("eps", [0.01, 0.0])
+@pytest.mark.parametrize("n, nt", [(1, 1), (2, 2), (9, 30), (1023, 7), (2049, 8), (8192, 9),
+                                   (9001, 3000), (70001, 257)])
+def test_direct_sum_matches_oracle(oracle, n, nt, eps):
+    rng = np.random.default_rng(n + nt)
+    pos = rng.standard_normal((n, 3))
+    pos[n // 2] = pos[0]  # a coincident pair (n > 1)
+    if n > 4:
+        pos[3] = pos[1] + 1e-7  # below min_distance2 when unsoftened
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    t = np.concatenate([[0, n - 1], rng.integers(0, n, nt)])[:nt].astype(np.uint32)
+    e = float(np.float32(eps))
+    with B.OctreeHip(n, softening=eps, min_softening=0.0, min_distance2=1e-12) as s:
+        s.upload(pos, None, m)
+        if n > 8:
+            s.build_tree()  # a permuted store
+        a = s.direct_forces_fp64(t)
+    ref = oracle.direct_fp64(pos, m.astype(np.float64), t.astype(np.int32), e, float(np.float32(1e-12)))
+    for k, i in enumerate(t):
+        d = pos - pos[i]
+        r2 = (d * d).sum(1) + e * e
+        w = np.where(r2 > 1e-12, m * np.maximum(r2, 1e-100) ** -1.5, 0.0)
+        S = (w * np.linalg.norm(d, axis=1)).sum()
+        # a few FP64 roundings a term and at most n / 256 additions in a row
+        assert np.abs(a[k] - ref[k]).max() <= 1e-13 * S, (k, i)
