@@ -105,6 +105,8 @@ struct bh_hip_handle {
     float* lff_train_params = nullptr;  // normalised-output copy used while training
     uint32_t* lff_order = nullptr;
     size_t lff_order_cap = 0;
+    float* lff_rows = nullptr;  // X and Y of lff_gradient / lff_forward, kept for the next call
+    size_t lff_rows_cap = 0;    // (rows)
 };
 
 namespace {
@@ -1617,14 +1619,15 @@ bool lff_alloc_core(bh_hip_handle* h)
     if (!dalloc(h, &L.params, bh::kLffParams, "lff params") ||
         !dalloc(h, &L.adam_m, bh::kLffParams, "lff adam m") ||
         !dalloc(h, &L.adam_v, bh::kLffParams, "lff adam v") ||
-        !dalloc(h, &L.grad, bh::kLffParams, "lff grad") ||
+        !dalloc(h, &L.grad, bh::kLffParams + 4, "lff grad") ||
         !dalloc(h, &h->lff_train_params, bh::kLffParams, "lff train params") ||
         !dalloc(h, &L.partial, static_cast<size_t>(L.partial_blocks) * bh::kLffParams,
                 "lff partial") ||
         !dalloc(h, &L.loss_partial, L.partial_blocks, "lff loss partial") ||
-        !dalloc(h, &L.loss_acc, 4, "lff loss") || !dalloc(h, &L.bias, 144, "lff bias") ||
+        !dalloc(h, &L.bias, 144, "lff bias") ||
         !dalloc(h, &L.tuple_counter, 2, "lff counter"))
         return false;
+    L.loss_acc = L.grad + bh::kLffParams;  // read with the gradient in one copy
     short* frag = nullptr;
     if (!dalloc(h, &frag, 14 * 64 * 8, "lff fragments"))  // 14 x 64 lanes x 8 BF16
         return false;
@@ -1671,6 +1674,31 @@ bool lff_alloc_lists(bh_hip_handle* h)
     L.list_groups = groups;
     return dalloc(h, &L.lists, groups * static_cast<size_t>(cap), "lff lists") &&
            dalloc(h, &L.list_n, groups, "lff list counts");
+}
+
+// Feature rows (and targets, unless Y is null) of one call in the handle's row
+// buffer, which grows to the largest call: X first, Y after lff_rows_cap rows.
+// (Allocating and freeing both per call cost about 0.1 ms.)
+bool lff_stage_rows(bh_hip_handle* h, const float* X, const float* Y, uint32_t n)
+{
+    constexpr size_t kRow = bh::kLffInputs + bh::kLffOutputs;
+    if (h->lff_rows_cap < n) {
+        dfree(h, h->lff_rows);
+        h->lff_rows = nullptr;
+        h->lff_rows_cap = 0;
+        const size_t cap = (static_cast<size_t>(n) + 3) & ~static_cast<size_t>(3);
+        if (!dalloc(h, &h->lff_rows, cap * kRow, "rows"))
+            return false;
+        h->lff_rows_cap = cap;
+    }
+    const size_t rows = n;
+    return check(h, hipMemcpyAsync(h->lff_rows, X, rows * bh::kLffInputs * sizeof(float),
+                                   hipMemcpyHostToDevice, h->d.stream),
+                 "rows X") &&
+           (!Y || check(h, hipMemcpyAsync(h->lff_rows + h->lff_rows_cap * bh::kLffInputs, Y,
+                                          rows * bh::kLffOutputs * sizeof(float),
+                                          hipMemcpyHostToDevice, h->d.stream),
+                        "rows Y"));
 }
 
 }  // namespace
@@ -1893,36 +1921,30 @@ bh_hip_result_t bh_hip_lff_gradient(bh_hip_handle_t* h, const float* X, const fl
     if (!lff_alloc_core(h))
         return BH_HIP_INTERNAL_ERROR;
     bh::LffState& L = h->lff;
-    float *dX = nullptr, *dY = nullptr, *dP = nullptr;
-    uint32_t* dO = nullptr;
-    std::vector<uint32_t> ord(n);
-    std::iota(ord.begin(), ord.end(), 0u);
     const int nblocks = std::min<int>(L.partial_blocks, static_cast<int>((n + 63) / 64));
-    bool ok = dalloc(h, &dX, static_cast<size_t>(n) * bh::kLffInputs, "grad X") &&
-              dalloc(h, &dY, static_cast<size_t>(n) * bh::kLffOutputs, "grad Y") &&
-              dalloc(h, &dP, bh::kLffParams, "grad P") && dalloc(h, &dO, n, "grad order");
-    ok = ok && check(h, hipMemcpy(dX, X, static_cast<size_t>(n) * bh::kLffInputs * 4,
-                                  hipMemcpyHostToDevice), "grad X") &&
-         check(h, hipMemcpy(dY, Y, static_cast<size_t>(n) * bh::kLffOutputs * 4,
-                            hipMemcpyHostToDevice), "grad Y") &&
-         check(h, hipMemcpy(dP, params, bh::kLffParams * 4, hipMemcpyHostToDevice), "grad P") &&
-         check(h, hipMemcpy(dO, ord.data(), n * 4, hipMemcpyHostToDevice), "grad order") &&
-         check(h, hipMemset(L.loss_acc, 0, 4), "grad loss");
-    if (ok) {
-        bh::launch_lff_grad(h->d, L, dX, dY, dO, 0, n, 1.0f, dP, nblocks);
-        bh::launch_lff_adam(h->d, L, nblocks, dP, L.grad, 0.0f, 1);
-        float lsum = 0.0f;
-        ok = check(h, hipGetLastError(), "grad") && check(h, hipStreamSynchronize(h->d.stream), "grad") &&
-             check(h, hipMemcpy(grad, L.grad, bh::kLffParams * 4, hipMemcpyDeviceToHost), "grad") &&
-             check(h, hipMemcpy(&lsum, L.loss_acc, 4, hipMemcpyDeviceToHost), "grad loss");
-        if (loss)
-            *loss = lsum / static_cast<float>(n);
+    if (!lff_stage_rows(h, X, Y, n) ||
+        !check(h, hipMemcpyAsync(h->lff_train_params, params, bh::kLffParams * 4,
+                                 hipMemcpyHostToDevice, h->d.stream),
+               "grad P")) {
+        (void)hipStreamSynchronize(h->d.stream);
+        return BH_HIP_INTERNAL_ERROR;
     }
-    dfree(h, dX);
-    dfree(h, dY);
-    dfree(h, dP);
-    dfree(h, dO);
-    return ok ? BH_HIP_OK : BH_HIP_INTERNAL_ERROR;
+    const float* dX = h->lff_rows;
+    const float* dY = dX + static_cast<size_t>(h->lff_rows_cap) * bh::kLffInputs;
+    bh::launch_fill_u32(reinterpret_cast<uint32_t*>(L.loss_acc), 0u, 1, h->d.stream);
+    bh::launch_lff_grad(h->d, L, dX, dY, nullptr, 0, n, 1.0f, h->lff_train_params, nblocks);
+    bh::launch_lff_adam(h->d, L, nblocks, h->lff_train_params, L.grad, 0.0f, 1);
+    float out[bh::kLffParams + 1];
+    const bool ok = check(h, hipGetLastError(), "grad") &&
+                    copy_out(h, out, L.grad, sizeof(out), "grad");
+    if (!ok) {
+        (void)hipStreamSynchronize(h->d.stream);  // the caller's rows are free again
+        return BH_HIP_INTERNAL_ERROR;
+    }
+    std::memcpy(grad, out, bh::kLffParams * sizeof(float));
+    if (loss)
+        *loss = out[bh::kLffParams] / static_cast<float>(n);
+    return BH_HIP_OK;
 }
 
 bh_hip_result_t bh_hip_lff_forward(bh_hip_handle_t* h, const float* X, uint32_t n, float* Y)
@@ -1931,19 +1953,17 @@ bh_hip_result_t bh_hip_lff_forward(bh_hip_handle_t* h, const float* X, uint32_t 
         return BH_HIP_INVALID_ARGUMENT;
     if (!lff_alloc_core(h))
         return BH_HIP_INTERNAL_ERROR;
-    float *dX = nullptr, *dY = nullptr;
-    bool ok = dalloc(h, &dX, static_cast<size_t>(n) * bh::kLffInputs, "fwd X") &&
-              dalloc(h, &dY, static_cast<size_t>(n) * bh::kLffOutputs, "fwd Y");
-    ok = ok && check(h, hipMemcpy(dX, X, static_cast<size_t>(n) * bh::kLffInputs * 4,
-                                  hipMemcpyHostToDevice), "fwd X");
-    if (ok) {
-        bh::launch_lff_forward(h->d, h->lff, dX, n, dY);
-        ok = check(h, hipGetLastError(), "fwd") && check(h, hipStreamSynchronize(h->d.stream), "fwd") &&
-             check(h, hipMemcpy(Y, dY, static_cast<size_t>(n) * bh::kLffOutputs * 4,
-                                hipMemcpyDeviceToHost), "fwd Y");
+    if (!lff_stage_rows(h, X, nullptr, n)) {
+        (void)hipStreamSynchronize(h->d.stream);
+        return BH_HIP_INTERNAL_ERROR;
     }
-    dfree(h, dX);
-    dfree(h, dY);
+    float* dY = h->lff_rows + static_cast<size_t>(h->lff_rows_cap) * bh::kLffInputs;
+    bh::launch_lff_forward(h->d, h->lff, h->lff_rows, n, dY);
+    const bool ok =
+        check(h, hipGetLastError(), "fwd") &&
+        copy_out(h, Y, dY, static_cast<size_t>(n) * bh::kLffOutputs * sizeof(float), "fwd Y");
+    if (!ok)
+        (void)hipStreamSynchronize(h->d.stream);
     return ok ? BH_HIP_OK : BH_HIP_INTERNAL_ERROR;
 }
 

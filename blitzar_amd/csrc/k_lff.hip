@@ -35,7 +35,7 @@
 //   lff_tuple_kernel   : per recorded (group, node) and target: features and
 //                        the exact residual (direct sum over the node's
 //                        particles, FP32) -> training tuples
-//   lff_grad_kernel    : FP32 forward + backward of the MSE loss over a
+//   lff_grad_kernel    : FP32 MFMA forward + backward of the MSE loss over a
 //                        minibatch; per-workgroup partial gradients
 //   lff_adam_kernel    : reduces partial gradients, Adam update
 //   lff_pack_kernel    : weights -> BF16 MFMA A-operand fragments
@@ -105,12 +105,6 @@ __device__ inline bf16x4 pack4(float a, float b, float c, float d)
 
 // Training arithmetic (FP32, correctly rounded division).
 __device__ inline float sigmoidf(float z) { return 1.0f / (1.0f + __expf(-z)); }
-__device__ inline float siluf(float z) { return z * sigmoidf(z); }
-__device__ inline float dsiluf(float z)
-{
-    const float s = sigmoidf(z);
-    return s * (1.0f + z * (1.0f - s));
-}
 // Inference activation on log2(e)-scaled pre-activations (see above): one
 // v_exp_f32 and one v_rcp_f32.
 __device__ inline float silu2(float z)
@@ -361,138 +355,323 @@ __global__ __launch_bounds__(64) void lff_tuple_kernel(
 }
 
 // ---- training: FP32 forward/backward -----------------------------------------
-// One workgroup = one wave; lane i handles sample i of a 64-sample chunk.
-// Gradients of the mean squared error over `nbatch` samples; each workgroup
-// writes its partial gradient (and partial loss) for the samples it handled.
-__global__ __launch_bounds__(64) void lff_grad_kernel(
+// Gradients of the mean squared error over `nbatch` samples, on the FP32 matrix
+// cores (v_mfma_f32_16x16x4_f32; FP32 products and sums, as the vector form).
+// A workgroup of 4 waves takes chunks of 64 samples and writes its partial
+// gradient and loss.
+//   * Forward and backward, wave w on samples 16w..16w+15: layers transposed as
+//     in the inference kernel, weights the A operand (read from LDS in fragment
+//     order, 4 k-steps per float4), samples the B columns. Step (t, j) of a
+//     product over 64 units covers the units 16t + 4q + j (q = lane / 16), so a
+//     lane's result register [t][j] of one layer is its B operand of the next:
+//     nothing moves between lanes.
+//   * Weight gradients contract over samples: activations and deltas go through
+//     LDS as [unit][sample] rows, and wave w sums its 16 rows (of W2 and W3) or
+//     columns (of W1) over the chunk's 64 samples, so the workgroup holds one
+//     copy of the gradient in registers (28 per lane).
+// Bound: FP32 matrix issue, 292 MFMA of 32 cycles per 16 samples (15 us for
+// 65,536 samples on the card), one wave per SIMD by LDS (127 KB). The
+// lane-per-sample vector form took 503 us for 65,536 samples, this one 46 us.
+constexpr int kGradChunk = 64;
+constexpr int kGradRow = kGradChunk + 4;  // float4-aligned rows, banks spread
+
+__device__ inline f32x4 mfma4(float a, float b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+struct GradLds {
+    f32x4 w1[4 * 2 * 64];   // [mt][cc][lane][i]: W1[4 (4 cc + i) + q][16 mt + r]
+    f32x4 w2f[4 * 4 * 64];  // [mh][t][lane][j]:  W2[16 t + 4 q + j][16 mh + r]
+    f32x4 w2b[4 * 4 * 64];  // [ma][t][lane][j]:  W2[16 ma + r][16 t + 4 q + j]
+    f32x4 w3f[4 * 64];      // [t][lane][j]:      W3[16 t + 4 q + j][r], rows r >= 3 zero
+    float w3b[4 * 64];      // [mt][lane]:        W3[16 mt + r][q], q = 3 zero
+    float b1[NH], b2[NH], b3[4];
+    float loss[4];
+    float x[NF * kGradRow];
+    float h1[NH * kGradRow], h2[NH * kGradRow], d1[NH * kGradRow], d2[NH * kGradRow];
+    float dy[4 * kGradRow];
+};
+
+// order: sample indices (null: the identity)
+__global__ __launch_bounds__(256) void lff_grad_kernel(
     const float* __restrict__ X, const float* __restrict__ Y, const uint32_t* __restrict__ order,
     size_t first, uint32_t nbatch, float yscale, const float* __restrict__ P,
     float* __restrict__ partial, float* __restrict__ loss_partial)
 {
-    __shared__ float sP[NP];
-    __shared__ float sX[64][NF + 1];
-    __shared__ float sZ1[64][NH + 1];
-    __shared__ float sH1[64][NH + 1];
-    __shared__ float sZ2[64][NH + 1];
-    __shared__ float sD1[64][NH + 1];
-    __shared__ float sD2[64][NH + 1];
-    __shared__ float sDY[64][NO];
-    const int t = threadIdx.x;
-    for (int k = t; k < NP; k += 64)
-        sP[k] = P[k];
-    float gW1[NF], gW2[NH], gW3[NO], gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, loss = 0.0f;
-    for (int k = 0; k < NF; ++k)
-        gW1[k] = 0.0f;
-    for (int k = 0; k < NH; ++k)
-        gW2[k] = 0.0f;
-    for (int k = 0; k < NO; ++k)
-        gW3[k] = 0.0f;
+    __shared__ GradLds S;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    for (int k = tid; k < 4 * 2 * 64; k += 256) {
+        const int l = k & 63, cc = (k >> 6) & 1, mt = k >> 7;
+        for (int i = 0; i < 4; ++i)
+            S.w1[k][i] = P[OFF_W1 + (4 * (4 * cc + i) + (l >> 4)) * NH + 16 * mt + (l & 15)];
+    }
+    for (int k = tid; k < 4 * 4 * 64; k += 256) {
+        const int l = k & 63, t = (k >> 6) & 3, m = k >> 8;
+        for (int j = 0; j < 4; ++j) {
+            const int u = 16 * t + 4 * (l >> 4) + j, v = 16 * m + (l & 15);
+            S.w2f[k][j] = P[OFF_W2 + u * NH + v];
+            S.w2b[k][j] = P[OFF_W2 + v * NH + u];
+        }
+    }
+    {
+        const int l = tid & 63, t = tid >> 6;
+        for (int j = 0; j < 4; ++j)
+            S.w3f[tid][j] = (l & 15) < NO
+                                ? P[OFF_W3 + (16 * t + 4 * (l >> 4) + j) * NO + (l & 15)]
+                                : 0.0f;
+        S.w3b[tid] =
+            (l >> 4) < NO ? P[OFF_W3 + (16 * t + (l & 15)) * NO + (l >> 4)] : 0.0f;
+    }
+    if (tid < NH) {
+        S.b1[tid] = P[OFF_B1 + tid];
+        S.b2[tid] = P[OFF_B2 + tid];
+    }
+    if (tid < 4)
+        S.b3[tid] = tid < NO ? P[OFF_B3 + tid] : 0.0f;
+
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 gW2[4] = {zero, zero, zero, zero};  // rows 16w.. of W2, by column tile
+    f32x4 gW1[2] = {zero, zero};              // columns 16w.. of W1, by row tile
+    f32x4 gW3 = zero;                         // rows 16w.. of W3
+    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, loss = 0.0f;
     const float inv_b = 1.0f / static_cast<float>(nbatch);
-    __syncthreads();
-    const uint32_t nchunks = (nbatch + 63) / 64;
+    const uint32_t nchunks = (nbatch + kGradChunk - 1) / kGradChunk;
     for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-        const uint32_t bi = ch * 64 + t;
+        {  // 4 threads a sample, 8 features each
+            const int sl = tid >> 2, part = tid & 3;
+            const uint32_t bi = ch * kGradChunk + sl;
+            f32x4 v[2] = {zero, zero};
+            if (bi < nbatch) {
+                const size_t src = order ? static_cast<size_t>(order[first + bi]) : first + bi;
+                const f32x4* row = reinterpret_cast<const f32x4*>(X + src * NF) + 2 * part;
+                v[0] = row[0];
+                v[1] = row[1];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                S.x[(8 * part + k) * kGradRow + sl] = v[k >> 2][k & 3];
+        }
+        const int col = 16 * w + r;  // this lane's sample in the chunk
+        const uint32_t bi = ch * kGradChunk + col;
         const bool valid = bi < nbatch;
-        const size_t src = valid ? static_cast<size_t>(order[first + bi]) : 0;
-        float x[NF], y[NO];
-        for (int k = 0; k < NF; ++k) {
-            x[k] = valid ? X[src * NF + k] : 0.0f;
-            sX[t][k] = x[k];
-        }
-        for (int k = 0; k < NO; ++k)
-            y[k] = valid ? Y[src * NO + k] * yscale : 0.0f;
-        // forward (activations of this lane's sample live in its LDS rows)
-        for (int a = 0; a < NH; ++a) {
-            float z = sP[OFF_B1 + a];
-            for (int k = 0; k < NF; ++k)
-                z += x[k] * sP[OFF_W1 + k * NH + a];
-            sZ1[t][a] = z;
-            sH1[t][a] = siluf(z);
-        }
-        float out[NO];
-        for (int k = 0; k < NO; ++k)
-            out[k] = sP[OFF_B3 + k];
-        for (int h = 0; h < NH; ++h) {
-            float z = sP[OFF_B2 + h];
-            for (int a = 0; a < NH; ++a)
-                z += sH1[t][a] * sP[OFF_W2 + a * NH + h];
-            sZ2[t][h] = z;
-            const float h2 = siluf(z);
+        float y[NO] = {0.0f, 0.0f, 0.0f};
+        if (valid && q == 0) {
+            const size_t src = order ? static_cast<size_t>(order[first + bi]) : first + bi;
             for (int k = 0; k < NO; ++k)
-                out[k] += h2 * sP[OFF_W3 + h * NO + k];
-        }
-        // backward
-        float dy[NO];
-        for (int k = 0; k < NO; ++k) {
-            const float e = out[k] - y[k];
-            dy[k] = valid ? 2.0f * e * inv_b : 0.0f;
-            loss += valid ? e * e : 0.0f;
-            sDY[t][k] = dy[k];
-        }
-        for (int h = 0; h < NH; ++h) {
-            float g = 0.0f;
-            for (int k = 0; k < NO; ++k)
-                g += dy[k] * sP[OFF_W3 + h * NO + k];
-            sD2[t][h] = g * dsiluf(sZ2[t][h]);
-        }
-        for (int a = 0; a < NH; ++a) {
-            float g = 0.0f;
-            for (int h = 0; h < NH; ++h)
-                g += sD2[t][h] * sP[OFF_W2 + a * NH + h];
-            sD1[t][a] = g * dsiluf(sZ1[t][a]);
+                y[k] = Y[src * NO + k] * yscale;
         }
         __syncthreads();
-        // weight gradients: lane t owns output column t of W1 and W2, row t of W3
-        for (int i = 0; i < 64; ++i) {
-            const float d1 = sD1[i][t];
-            const float d2 = sD2[i][t];
-            gb1 += d1;
-            gb2 += d2;
-            for (int k = 0; k < NF; ++k)
-                gW1[k] += sX[i][k] * d1;
-            for (int a = 0; a < NH; ++a)
-                gW2[a] += sH1[i][a] * d2;
-            const float h2 = siluf(sZ2[i][t]);
-            for (int k = 0; k < NO; ++k)
-                gW3[k] += h2 * sDY[i][k];
-            if (t < NO)
-                gb3 += sDY[i][t];
+        // layer 1
+        f32x4 h1[4], s1[4];  // activation and its derivative
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+            h1[mt] = *reinterpret_cast<const f32x4*>(&S.b1[16 * mt + 4 * q]);
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+            float b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                b[i] = S.x[(4 * (4 * cc + i) + q) * kGradRow + col];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt)
+                    h1[mt] = mfma4(S.w1[(mt * 2 + cc) * 64 + lane][i], b[i], h1[mt]);
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float z = h1[mt][j], s = sigmoidf(z);
+                s1[mt][j] = s * (1.0f + z * (1.0f - s));
+                h1[mt][j] = z * s;
+                S.h1[(16 * mt + 4 * q + j) * kGradRow + col] = h1[mt][j];
+            }
+        // layer 2
+        f32x4 h2[4], s2[4];
+#pragma unroll
+        for (int mh = 0; mh < 4; ++mh)
+            h2[mh] = *reinterpret_cast<const f32x4*>(&S.b2[16 * mh + 4 * q]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int mh = 0; mh < 4; ++mh)
+                    h2[mh] = mfma4(S.w2f[(mh * 4 + t) * 64 + lane][j], h1[t][j], h2[mh]);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float z = h2[mt][j], s = sigmoidf(z);
+                s2[mt][j] = s * (1.0f + z * (1.0f - s));
+                h2[mt][j] = z * s;
+                S.h2[(16 * mt + 4 * q + j) * kGradRow + col] = h2[mt][j];
+            }
+        // output (rows 0..2, held by the lanes of q = 0) and its error; two
+        // chains, so that the steps overlap
+        f32x4 o0 = zero, o1 = zero;
+        if (q == 0)
+            o0 = *reinterpret_cast<const f32x4*>(S.b3);
+#pragma unroll
+        for (int t = 0; t < 4; t += 2)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                o0 = mfma4(S.w3f[t * 64 + lane][j], h2[t][j], o0);
+                o1 = mfma4(S.w3f[(t + 1) * 64 + lane][j], h2[t + 1][j], o1);
+            }
+        float dq = 0.0f;  // dLoss/dy_q of sample r
+#pragma unroll
+        for (int k = 0; k < NO; ++k) {
+            const float e = (o0[k] + o1[k]) - y[k];
+            float dk = 0.0f;
+            if (valid && q == 0) {
+                dk = 2.0f * e * inv_b;
+                loss += e * e;
+            }
+            dk = __shfl(dk, r, 64);
+            dq = q == k ? dk : dq;
+        }
+        S.dy[q * kGradRow + col] = dq;  // row 3 stays zero
+        // deltas of layer 2, then of layer 1
+        f32x4 d2[4], d1[4] = {zero, zero, zero, zero};
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+            d2[mt] = mfma4(S.w3b[mt * 64 + lane], dq, zero) * s2[mt];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                S.d2[(16 * t + 4 * q + j) * kGradRow + col] = d2[t][j];
+#pragma unroll
+                for (int ma = 0; ma < 4; ++ma)
+                    d1[ma] = mfma4(S.w2b[(ma * 4 + t) * 64 + lane][j], d2[t][j], d1[ma]);
+            }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            d1[mt] *= s1[mt];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                S.d1[(16 * mt + 4 * q + j) * kGradRow + col] = d1[mt][j];
+        }
+        __syncthreads();
+        // weight gradients: step i of float4 c covers samples 16c + 4q + i
+        const int row = (16 * w + r) * kGradRow;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int off = 16 * c + 4 * q;
+            const auto at = [&](const float* v, int m) {
+                return *reinterpret_cast<const f32x4*>(v + m + off);
+            };
+            const f32x4 ah1 = at(S.h1, row), ah2 = at(S.h2, row), bd1 = at(S.d1, row);
+            const f32x4 bd2 = at(S.d2, row);
+            gb1 += (bd1[0] + bd1[1]) + (bd1[2] + bd1[3]);
+            gb2 += (bd2[0] + bd2[1]) + (bd2[2] + bd2[3]);
+            const f32x4 bdy = r < NO ? at(S.dy, r * kGradRow) : zero;
+            gb3 += (bdy[0] + bdy[1]) + (bdy[2] + bdy[3]);
+            f32x4 b2[4], ax[2];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                b2[m] = at(S.d2, (16 * m + r) * kGradRow);
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                ax[m] = at(S.x, (16 * m + r) * kGradRow);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    gW2[m] = mfma4(ah1[i], b2[m][i], gW2[m]);
+                gW3 = mfma4(ah2[i], bdy[i], gW3);
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    gW1[m] = mfma4(ax[m][i], bd1[i], gW1[m]);
+            }
         }
         __syncthreads();
     }
     float* out = partial + static_cast<size_t>(blockIdx.x) * NP;
-    for (int k = 0; k < NF; ++k)
-        out[OFF_W1 + k * NH + t] = gW1[k];
-    out[OFF_B1 + t] = gb1;
-    for (int a = 0; a < NH; ++a)
-        out[OFF_W2 + a * NH + t] = gW2[a];
-    out[OFF_B2 + t] = gb2;
-    for (int k = 0; k < NO; ++k)
-        out[OFF_W3 + t * NO + k] = gW3[k];
-    if (t < NO)
-        out[OFF_B3 + t] = gb3;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            out[OFF_W2 + (16 * w + 4 * q + j) * NH + 16 * m + r] = gW2[m][j];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            out[OFF_W1 + (16 * m + 4 * q + j) * NH + 16 * w + r] = gW1[m][j];
+        if (r < NO)
+            out[OFF_W3 + (16 * w + 4 * q + j) * NO + r] = gW3[j];
+    }
+    for (int o = 32; o >= 16; o >>= 1) {  // the quarters' samples
+        gb1 += __shfl_xor(gb1, o, 64);
+        gb2 += __shfl_xor(gb2, o, 64);
+        gb3 += __shfl_xor(gb3, o, 64);
+    }
+    if (q == 0) {
+        out[OFF_B1 + 16 * w + r] = gb1;
+        out[OFF_B2 + 16 * w + r] = gb2;
+        if (w == 0 && r < NO)
+            out[OFF_B3 + r] = gb3;
+    }
     // partial loss (sum of squared errors of this workgroup)
     for (int o = 32; o > 0; o >>= 1)
         loss += __shfl_xor(loss, o, 64);
-    if (t == 0)
-        loss_partial[blockIdx.x] = loss;
+    if (lane == 0)
+        S.loss[w] = loss;
+    __syncthreads();
+    if (tid == 0)
+        loss_partial[blockIdx.x] = (S.loss[0] + S.loss[1]) + (S.loss[2] + S.loss[3]);
 }
 
 // Sums the partial gradients into grad (when non-null) and applies Adam when
-// lr > 0. step is 1-based.
+// lr > 0 (step is 1-based); the block past the parameters adds the partial
+// losses to *loss. 32 parameters a block, 8 threads each: with one thread per
+// parameter the chain of nb loads took 60 us for 256 partials, and the losses
+// another 13 us on a thread of their own; this takes 4 us.
+constexpr int kAdamParams = 32;
+
 __global__ __launch_bounds__(256) void lff_adam_kernel(const float* __restrict__ partial, int nb,
                                                        float* __restrict__ P,
                                                        float* __restrict__ m,
                                                        float* __restrict__ v,
                                                        float* __restrict__ grad, float lr,
-                                                       float b1, float b2, int step)
+                                                       float b1, float b2, int step,
+                                                       const float* __restrict__ loss_partial,
+                                                       float* __restrict__ loss)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float red[8][kAdamParams];
+    const int c = threadIdx.x % kAdamParams, sl = threadIdx.x / kAdamParams;
+    const bool losses = blockIdx.x * kAdamParams >= NP;  // the last block
+    const int k = losses ? 0 : blockIdx.x * kAdamParams + c;
+    float g = 0.0f;
+    if (losses) {
+        for (int b = threadIdx.x; b < nb; b += 256)
+            g += loss_partial[b];
+    } else if (k < NP) {
+#pragma unroll 8
+        for (int b = sl; b < nb; b += 8)
+            g += partial[static_cast<size_t>(b) * NP + k];
+    }
+    red[sl][c] = g;
+    __syncthreads();
+    if (sl != 0)
+        return;
+    g = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        g += red[i][c];
+    if (losses) {
+        for (int o = 16; o > 0; o >>= 1)
+            g += __shfl_xor(g, o, 32);
+        if (threadIdx.x == 0)
+            *loss += g;
+        return;
+    }
     if (k >= NP)
         return;
-    float g = 0.0f;
-    for (int b = 0; b < nb; ++b)
-        g += partial[static_cast<size_t>(b) * NP + k];
     if (grad)
         grad[k] = g;
     if (lr > 0.0f) {
@@ -504,16 +683,6 @@ __global__ __launch_bounds__(256) void lff_adam_kernel(const float* __restrict__
         const float vh = vk / (1.0f - powf(b2, static_cast<float>(step)));
         P[k] -= lr * mh / (sqrtf(vh) + 1e-8f);
     }
-}
-
-__global__ void lff_loss_sum_kernel(const float* __restrict__ lp, int nb, float* __restrict__ out)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0)
-        return;
-    float s = 0.0f;
-    for (int b = 0; b < nb; ++b)
-        s += lp[b];
-    *out += s;
 }
 
 // ---- inference: BF16 MFMA -----------------------------------------------------
@@ -865,16 +1034,16 @@ void launch_lff_grad(Device& d, const LffState& L, const float* X, const float* 
                      const uint32_t* order, size_t first, uint32_t nbatch, float yscale,
                      const float* P, int nblocks)
 {
-    lff_grad_kernel<<<nblocks, 64, 0, d.stream>>>(X, Y, order, first, nbatch, yscale, P,
+    lff_grad_kernel<<<nblocks, 256, 0, d.stream>>>(X, Y, order, first, nbatch, yscale, P,
                                                   L.partial, L.loss_partial);
 }
 
 void launch_lff_adam(Device& d, const LffState& L, int nblocks, float* P, float* grad, float lr,
                      int step)
 {
-    lff_adam_kernel<<<(NP + 255) / 256, 256, 0, d.stream>>>(L.partial, nblocks, P, L.adam_m,
-                                                           L.adam_v, grad, lr, 0.9f, 0.999f, step);
-    lff_loss_sum_kernel<<<1, 64, 0, d.stream>>>(L.loss_partial, nblocks, L.loss_acc);
+    lff_adam_kernel<<<(NP + kAdamParams - 1) / kAdamParams + 1, 256, 0, d.stream>>>(
+        L.partial, nblocks, P, L.adam_m, L.adam_v, grad, lr, 0.9f, 0.999f, step, L.loss_partial,
+        L.loss_acc);
 }
 
 void launch_lff_pack(Device& d, const LffState& L)
