@@ -295,7 +295,7 @@ bool alloc_all(bh_hip_handle* h, uint64_t n)
     if (!dalloc_zero(h, &d.sort_hist, d.sort_hist_cap, "sort hist", d.stream))
         return false;
     if (!dalloc(h, &d.level_info, 2 * bh::kLevels + 8, "level info") ||
-        !dalloc(h, &d.geom, 1, "geometry") || !dalloc(h, &d.aabb_bits, 8, "aabb") ||
+        !dalloc(h, &d.geom, 1, "geometry") ||
         !dalloc(h, &d.err, 4, "error flags") || !dalloc(h, &d.work_counter, bh::kTicketWords, "work counter") ||
         !dalloc(h, &h->stats, 8, "walk stats"))
         return false;
@@ -597,9 +597,14 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
     bh::Device& d = h->d;
     rec(ev ? ev->b0 : nullptr, d.stream);
     bh::launch_aabb(d);
-    bh::launch_keys(d, h->p.key_mode);
-    rec(ev ? ev->s0 : nullptr, d.stream);
-    bh::launch_radix_sort(d, d.n, h->p.key_mode == 1 ? 30 : 63);
+    if (bh::use_keys_sort(d.n, h->p.key_mode)) {
+        rec(ev ? ev->s0 : nullptr, d.stream);
+        bh::launch_keys_sort(d, h->p.key_mode);
+    } else {
+        bh::launch_keys(d, h->p.key_mode);
+        rec(ev ? ev->s0 : nullptr, d.stream);
+        bh::launch_radix_sort(d, d.n, h->p.key_mode == 1 ? 30 : 63);
+    }
     rec(ev ? ev->s1 : nullptr, d.stream);
     bh::launch_tie_fix(d);
     // The topology needs only the sorted keys: it runs on the side stream

@@ -228,7 +228,6 @@ struct Device {
     int* level_info = nullptr;  // [0..22) base, [22..44) count, [44] total, [45] max level, [46] groups
 
     RootGeom* geom = nullptr;
-    unsigned long long* aabb_bits = nullptr;  // 6 ordered-encoded doubles
     int* err = nullptr;
     unsigned int* work_counter = nullptr;
     int* stack = nullptr;  // per-resident-wave traversal stacks
@@ -292,15 +291,20 @@ struct PmState {
 // k_keys.hip
 void launch_aabb(Device& d);
 void launch_keys(Device& d, int key_mode);
-// k_sort.hip: stable LSD radix sort of (keys, vals) pairs, 8-bit digits over
-// bits [0, key_bits). Result lands back in d.keys / d.vals.
+// k_sort.hip: stable sort of (keys, vals) pairs by bits [0, key_bits). Result
+// lands back in d.keys / d.vals.
 void launch_radix_sort(Device& d, size_t n, int key_bits);
+// Keys of the current positions and their sort in one go (the sort's first pass
+// makes the keys), where use_keys_sort; else launch_keys, then launch_radix_sort.
+bool use_keys_sort(size_t n, int key_mode);
+void launch_keys_sort(Device& d, int key_mode);
 size_t radix_hist_words(size_t n);
 // The same sort on explicit buffers: (keys, vals) in, (keys_alt, vals_alt) the
 // second buffer pair, hist_ws radix_hist_words(n) words whose scan part
 // starts zeroed once. Returns true when the result ends in the alternate
 // buffers (an odd number of passes). Nothing is allocated.
-int radix_sort_passes(int key_bits);
+int radix_sort_passes(size_t n, int key_bits);
+bool sort_uses_scan(size_t n, int key_bits);  // only then *err and hist_ws are used
 bool radix_sort_buffers(uint64_t* keys, uint64_t* keys_alt, uint32_t* vals, uint32_t* vals_alt,
                         uint32_t* hist_ws, size_t n, int key_bits, int* err, hipStream_t stream);
 // The same sort reading (keys_in, vals_in), which it never writes: pass 0

@@ -12,28 +12,17 @@
 // with the 10-bit masks and therefore keeps only the low 10 bits per axis.
 //
 // HBM traffic: AABB reads 24 B/particle (FP64 SoA); keys read 24 B and write
-// 12 B per particle. The AABB combines per-block partial extrema in a second
-// one-block kernel (uses Device::diag, 6 doubles per block, 1024 blocks).
+// 12 B per particle (on builds of up to about 4M particles the sort's first pass
+// makes the keys as it loads the positions, see k_sort.hip). The AABB combines
+// per-block partial extrema in a second one-block kernel (uses Device::diag, 6
+// doubles per block, 1024 blocks).
 #include "bh_internal.h"
+#include "morton.h"
 
 #include <cfloat>
 
 namespace bh {
 namespace {
-
-constexpr unsigned long long kSign = 0x8000000000000000ull;
-
-__device__ inline unsigned long long order_bits(double x)
-{
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
-    return (b & kSign) ? ~b : (b | kSign);
-}
-
-__device__ inline double from_order_bits(unsigned long long e)
-{
-    const unsigned long long b = (e & kSign) ? (e & ~kSign) : ~e;
-    return __longlong_as_double(static_cast<long long>(b));
-}
 
 __device__ inline double wave_min(double v)
 {
@@ -90,9 +79,10 @@ __global__ __launch_bounds__(256) void aabb_kernel(const double* __restrict__ px
     }
 }
 
-// Combine the per-block extrema (one block).
-__global__ __launch_bounds__(256) void aabb_final_kernel(const double* __restrict__ partial,
-                                                         int nb, unsigned long long* bits)
+// Combine the per-block extrema and derive the root geometry (one block; the
+// two took a launch each, about 4 us of a small build).
+__global__ __launch_bounds__(256) void geometry_kernel(const double* __restrict__ partial, int nb,
+                                                       RootGeom* __restrict__ g)
 {
     __shared__ double red[6][4];
     double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
@@ -112,62 +102,26 @@ __global__ __launch_bounds__(256) void aabb_final_kernel(const double* __restric
         }
     }
     __syncthreads();
-    if (threadIdx.x < 6) {
+    if (threadIdx.x < 3) {
         const int a = threadIdx.x;
-        double v = red[a][0];
-        for (int k = 1; k < 4; ++k)
-            v = a < 3 ? fmin(v, red[a][k]) : fmax(v, red[a][k]);
-        bits[a] = order_bits(v);
-    }
-}
-
-// Root geometry from the FP64 AABB (one thread).
-__global__ void geometry_kernel(const unsigned long long* bits, RootGeom* g)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0)
-        return;
-    for (int a = 0; a < 3; ++a) {
-        const float lo = static_cast<float>(from_order_bits(bits[a]));
-        const float hi = static_cast<float>(from_order_bits(bits[3 + a]));
-        const float inv = __fdiv_rn(1.0f, fmaxf(hi - lo, 1.0e-12f));
-        g->lo[a] = lo;
+        double l = red[a][0], h = red[3 + a][0];
+        for (int k = 1; k < 4; ++k) {
+            l = fmin(l, red[a][k]);
+            h = fmax(h, red[3 + a][k]);
+        }
+        const float flo = static_cast<float>(l);
+        const float fhi = static_cast<float>(h);
+        const float inv = __fdiv_rn(1.0f, fmaxf(fhi - flo, 1.0e-12f));
+        g->lo[a] = flo;
         g->inv[a] = inv;
         // The lattice unit is half of one quantisation step of the FP32 frame:
         // step = 1 / (inv * (2^21 - 1)).
         const double step = 1.0 / (static_cast<double>(inv) * static_cast<double>(kQMax));
-        g->lo_d[a] = static_cast<double>(lo);
+        g->lo_d[a] = static_cast<double>(flo);
         g->unit_d[a] = 0.5 * step;
         g->unit_f[a] = static_cast<float>(0.5 * step);
         g->width_f[a] = static_cast<float>(step);
     }
-}
-
-__device__ inline unsigned long long spread21(unsigned int v)
-{
-    unsigned long long x = v & 0x1fffffu;
-    x = (x | (x << 32)) & 0x001f00000000ffffull;
-    x = (x | (x << 16)) & 0x001f0000ff0000ffull;
-    x = (x | (x << 8)) & 0x100f00f00f00f00full;
-    x = (x | (x << 4)) & 0x10c30c30c30c30c3ull;
-    x = (x | (x << 2)) & 0x1249249249249249ull;
-    return x;
-}
-
-// The reference interleave as it executes: 32-bit lanes, 10-bit masks.
-__device__ inline unsigned long long spread_ref32(unsigned int v)
-{
-    v = (v | (v << 16)) & 0x030000FFu;
-    v = (v | (v << 8)) & 0x0300F00Fu;
-    v = (v | (v << 4)) & 0x030C30C3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return static_cast<unsigned long long>(v);
-}
-
-__device__ inline unsigned int quantise(float p, float lo, float inv)
-{
-    const float t = fminf(fmaxf((p - lo) * inv, 0.0f), 1.0f);
-    const unsigned int q = static_cast<unsigned int>(__fmaf_rn(t, 2097151.0f, 0.5f));
-    return min(kQMax, q);
 }
 
 template <int MODE>
@@ -181,15 +135,7 @@ __global__ __launch_bounds__(256) void keys_kernel(const double* __restrict__ px
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
-    const unsigned int qx = quantise(static_cast<float>(px[i]), g->lo[0], g->inv[0]);
-    const unsigned int qy = quantise(static_cast<float>(py[i]), g->lo[1], g->inv[1]);
-    const unsigned int qz = quantise(static_cast<float>(pz[i]), g->lo[2], g->inv[2]);
-    unsigned long long k;
-    if (MODE == 1)
-        k = (spread_ref32(qx) << 2) | (spread_ref32(qy) << 1) | spread_ref32(qz);
-    else
-        k = (spread21(qx) << 2) | (spread21(qy) << 1) | spread21(qz);
-    keys[i] = k;
+    keys[i] = morton_key<MODE>(px[i], py[i], pz[i], g);
     vals[i] = static_cast<uint32_t>(i);
 }
 
@@ -204,8 +150,7 @@ void launch_aabb(Device& d)
         nb = static_cast<int>(std::max<size_t>(blocks, 1));
         aabb_kernel<<<nb, 256, 0, d.stream>>>(d.pos[0], d.pos[1], d.pos[2], d.n, d.diag);
     }
-    aabb_final_kernel<<<1, 256, 0, d.stream>>>(d.diag, nb, d.aabb_bits);
-    geometry_kernel<<<1, 64, 0, d.stream>>>(d.aabb_bits, d.geom);
+    geometry_kernel<<<1, 256, 0, d.stream>>>(d.diag, nb, d.geom);
 }
 
 void launch_keys(Device& d, int key_mode)

@@ -1,5 +1,5 @@
-// Stable LSD radix sort of (64-bit key, 32-bit value) pairs, device-wide
-// exclusive scan, equal-key tie ordering and the particle-store permutation.
+// Stable sorts of (64-bit key, 32-bit value) pairs (tile sort and merge; LSD radix
+// for large inputs), device-wide exclusive scan, equal-key tie ordering and the particle-store permutation.
 //
 // Contract followed: thrust::sort_by_key(keys, identity indices) at
 // engine/physics/octree/cuda/linear/OctBuild.inl:96 -- ascending keys, equal
@@ -8,11 +8,12 @@
 // tie_fix_kernel then reorders every run of equal keys by particle id, which
 // restores the reference contract exactly.
 //
-// One pass (8-bit digit) = histogram kernel (reads 8 B/key), one single-pass
+// One radix pass (8-bit digit) = histogram kernel (reads 8 B/key), one single-pass
 // scan of the digit-major tile counts, and a scatter kernel that ranks keys inside a tile
 // of 4096 with wave ballots, reorders the tile in LDS and writes digit runs
 // contiguously (reads 12 B/key, writes 12 B/key).
 #include "bh_internal.h"
+#include "morton.h"
 #include "scan_lookback.h"
 
 namespace bh {
@@ -166,6 +167,259 @@ __global__ __launch_bounds__(kScanBlock) void scan_lookback_kernel(
     }
 }
 
+// ---- tile sort and merge ----------------------------------------------------
+// Tiles are sorted in LDS by merging (8 pairs per thread in registers, then
+// runs two by two), and the tiles' runs are merged two by two in memory (merge
+// path). Everything is stable. FULL: keys compare whole; else under kmask.
+// Bound: latency up to a few hundred thousand pairs (a tile of 4,096: 9 rounds of
+// a binary search and 8 dependent LDS reads, 26 us; a merge pass 8-10 us, half of
+// it the split search), then the merge's issue rate (2,097,152 pairs: 17 us a pass,
+// 2.9 TB/s). Sorting the tiles with the radix sort's ballot ranking took 39 us.
+constexpr int kMergePer = 8;  // pairs per thread
+
+// LDS place of pair i: one unused place after every 8, so that threads 8 pairs
+// apart meet different banks.
+__host__ __device__ constexpr uint32_t lds_at(uint32_t i) { return i + (i >> 3); }
+
+template <bool FULL>
+__device__ inline bool key_gt(unsigned long long a, unsigned long long b, unsigned long long kmask)
+{
+    return FULL ? a > b : (a & kmask) > (b & kmask);
+}
+
+// First kMergePer outputs from output dd on of the merge of A = sk[a, a + na) and
+// B = sk[b, b + nb) (equal keys: A first), in registers; dd <= na + nb, outputs past
+// na + nb are not defined.
+template <bool FULL>
+__device__ inline void lds_merge(const unsigned long long* sk, const uint32_t* sv, uint32_t a,
+                                 uint32_t na, uint32_t b, uint32_t nb, uint32_t dd,
+                                 unsigned long long kmask, unsigned long long* key, uint32_t* val)
+{
+    uint32_t lo = dd > nb ? dd - nb : 0u, hi = dd < na ? dd : na;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (key_gt<FULL>(sk[lds_at(a + mid)], sk[lds_at(b + dd - 1u - mid)], kmask))
+            hi = mid;
+        else
+            lo = mid + 1u;
+    }
+    uint32_t ia = a + lo, ib = b + dd - lo;
+    const uint32_t ea = a + na, eb = b + nb;
+    unsigned long long ka = ia < ea ? sk[lds_at(ia)] : 0ull,
+                       kb = ib < eb ? sk[lds_at(ib)] : 0ull;
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const bool ta = ia < ea && (ib >= eb || !key_gt<FULL>(ka, kb, kmask));
+        key[k] = ta ? ka : kb;
+        const uint32_t at = ta ? ia : ib;
+        val[k] = at < eb ? sv[lds_at(at)] : 0u;
+        ia += ta ? 1u : 0u;
+        ib += ta ? 0u : 1u;
+        const uint32_t nx = ta ? ia : ib;
+        const unsigned long long kn = nx < (ta ? ea : eb) ? sk[lds_at(nx)] : 0ull;
+        ka = ta ? kn : ka;
+        kb = ta ? kb : kn;
+    }
+}
+
+// Sorts THREADS * kMergePer pairs in sk / sv (places past the valid pairs hold
+// keys of all ones, which stay behind every valid pair). Every thread calls it
+// after a barrier; it ends with one.
+template <int THREADS, bool FULL>
+__device__ inline void tile_sort(unsigned long long* sk, uint32_t* sv, unsigned long long kmask)
+{
+    const uint32_t o = threadIdx.x * kMergePer;
+    unsigned long long key[kMergePer];
+    uint32_t val[kMergePer];
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        key[k] = sk[lds_at(o + k)];
+        val[k] = sv[lds_at(o + k)];
+    }
+    // odd-even transposition: neighbours swap only when out of order
+#pragma unroll
+    for (int r = 0; r < kMergePer; ++r)
+#pragma unroll
+        for (int k = r & 1; k + 1 < kMergePer; k += 2) {
+            const bool sw = key_gt<FULL>(key[k], key[k + 1], kmask);
+            const unsigned long long x = key[k], y = key[k + 1];
+            const uint32_t u = val[k], v = val[k + 1];
+            key[k] = sw ? y : x;
+            key[k + 1] = sw ? x : y;
+            val[k] = sw ? v : u;
+            val[k + 1] = sw ? u : v;
+        }
+#pragma unroll 1
+    for (uint32_t run = kMergePer;; run *= 2) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kMergePer; ++k) {
+            sk[lds_at(o + k)] = key[k];
+            sv[lds_at(o + k)] = val[k];
+        }
+        __syncthreads();
+        if (run >= THREADS * kMergePer)
+            return;
+        const uint32_t p = o & ~(2u * run - 1u);
+        lds_merge<FULL>(sk, sv, p, run, p + run, run, o - p, kmask, key, val);
+    }
+}
+
+// Where a tile's pairs come from: arrays, or the particles' positions (MODE 0 or
+// 1: the key mode; the value is the store slot).
+struct PairsIn {
+    const unsigned long long* __restrict__ keys;
+    const uint32_t* __restrict__ vals;
+    __device__ void load(size_t i, unsigned long long& k, uint32_t& v) const
+    {
+        k = keys[i];
+        v = vals[i];
+    }
+};
+template <int MODE>
+struct PositionsIn {
+    const double* __restrict__ px;
+    const double* __restrict__ py;
+    const double* __restrict__ pz;
+    const RootGeom* __restrict__ g;
+    __device__ void load(size_t i, unsigned long long& k, uint32_t& v) const
+    {
+        k = morton_key<MODE>(px[i], py[i], pz[i], g);
+        v = static_cast<uint32_t>(i);
+    }
+};
+
+template <int THREADS, bool FULL, class In>
+__global__ __launch_bounds__(THREADS) void tile_sort_kernel(
+    In in, unsigned long long* __restrict__ keys_out, uint32_t* __restrict__ vals_out, size_t n,
+    unsigned long long kmask)
+{
+    constexpr uint32_t T = THREADS * kMergePer;
+    __shared__ unsigned long long sk[lds_at(T)];
+    __shared__ uint32_t sv[lds_at(T)];
+    const size_t t0 = static_cast<size_t>(blockIdx.x) * T;
+    const uint32_t tn = static_cast<uint32_t>(n - t0 < T ? n - t0 : T);
+    unsigned long long key[kMergePer];
+    uint32_t val[kMergePer];
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const uint32_t i = threadIdx.x + k * THREADS;
+        key[k] = ~0ull;
+        val[k] = 0u;
+        if (i < tn)
+            in.load(t0 + i, key[k], val[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const uint32_t i = threadIdx.x + k * THREADS;
+        sk[lds_at(i)] = key[k];
+        sv[lds_at(i)] = val[k];
+    }
+    __syncthreads();
+    tile_sort<THREADS, FULL>(sk, sv, kmask);
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const uint32_t i = threadIdx.x + k * THREADS;
+        if (i < tn) {
+            keys_out[t0 + i] = sk[lds_at(i)];
+            vals_out[t0 + i] = sv[lds_at(i)];
+        }
+    }
+}
+
+// Elements of A among the first d of the merge of A[0, la) and B[0, lb) (equal
+// keys: A first), by a whole wavefront: 64 probes per step, each step one round
+// trip for a 64th of the range.
+template <bool FULL>
+__device__ inline uint32_t wave_merge_split(const unsigned long long* __restrict__ A, uint32_t la,
+                                            const unsigned long long* __restrict__ B, uint32_t lb,
+                                            uint32_t d, unsigned long long kmask)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t lo = d > lb ? d - lb : 0u, hi = d < la ? d : la;
+    while (lo < hi) {  // the first i in [lo, hi) with A[i] > B[d - 1 - i], else hi
+        const uint32_t step = (hi - lo + 63u) / 64u;
+        const uint32_t i = lo + lane * step;
+        const bool past = i >= hi || key_gt<FULL>(A[i], B[d - 1u - i], kmask);
+        const unsigned long long m = __ballot(past);
+        const uint32_t f = m ? static_cast<uint32_t>(__builtin_ctzll(m)) : 64u;
+        if (f == 0u)
+            break;  // already past at lo
+        const uint32_t at = lo + f * step;
+        lo += (f - 1u) * step + 1u;
+        hi = at < hi ? at : hi;
+    }
+    return lo;
+}
+
+// One merge pass: runs of `run` pairs (a multiple of kMergeOut / 2, the last
+// one ragged) two by two into runs of 2 run; a block writes kMergeOut
+// consecutive pairs of one merged run.
+constexpr int kMergeBlock = 256;
+constexpr int kMergeOut = kMergeBlock * kMergePer;
+
+template <bool FULL>
+__global__ __launch_bounds__(kMergeBlock) void merge_kernel(
+    const unsigned long long* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
+    unsigned long long* __restrict__ keys_out, uint32_t* __restrict__ vals_out, size_t n,
+    size_t run, unsigned long long kmask)
+{
+    __shared__ unsigned long long sk[lds_at(kMergeOut)];
+    __shared__ uint32_t sv[lds_at(kMergeOut)];
+    __shared__ uint32_t split[2];
+    const int t = threadIdx.x;
+    const size_t o0 = static_cast<size_t>(blockIdx.x) * kMergeOut;
+    const size_t p0 = o0 / (2 * run) * (2 * run);
+    const uint32_t la = static_cast<uint32_t>(n - p0 < run ? n - p0 : run);
+    const uint32_t lb =
+        static_cast<uint32_t>(n - p0 - la < run ? n - p0 - la : run);
+    const unsigned long long* A = keys_in + p0;
+    const unsigned long long* B = A + la;
+    const uint32_t d0 = static_cast<uint32_t>(o0 - p0);
+    const uint32_t d1 = d0 + kMergeOut < la + lb ? d0 + kMergeOut : la + lb;
+    const uint32_t cnt = d1 - d0;
+    if (t < 128) {
+        const uint32_t v = wave_merge_split<FULL>(A, la, B, lb, t < 64 ? d0 : d1, kmask);
+        if ((t & 63) == 0)
+            split[t >> 6] = v;
+    }
+    __syncthreads();
+    const uint32_t a0 = split[0], a1 = split[1];
+    const uint32_t na = a1 - a0, nb = cnt - na;
+    // outputs d0.. take A[a0, a1) and B[d0 - a0, ...): i < na from A, else from B
+    const size_t ga = p0 + a0, gb = p0 + la + (d0 - a0) - na;
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const uint32_t i = static_cast<uint32_t>(t + k * kMergeBlock);
+        if (i < cnt) {
+            const size_t g = (i < na ? ga : gb) + i;
+            sk[lds_at(i)] = keys_in[g];
+            sv[lds_at(i)] = vals_in[g];
+        }
+    }
+    __syncthreads();
+    const uint32_t o = static_cast<uint32_t>(t * kMergePer);
+    unsigned long long key[kMergePer];
+    uint32_t val[kMergePer];
+    lds_merge<FULL>(sk, sv, 0u, na, na, nb, o < cnt ? o : cnt, kmask, key, val);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k)
+        if (o + k < cnt) {
+            sk[lds_at(o + k)] = key[k];
+            sv[lds_at(o + k)] = val[k];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMergePer; ++k) {
+        const uint32_t i = static_cast<uint32_t>(t + k * kMergeBlock);
+        if (i < cnt) {
+            keys_out[o0 + i] = sk[lds_at(i)];
+            vals_out[o0 + i] = sv[lds_at(i)];
+        }
+    }
+}
+
 // Runs of equal keys: order the run by particle id (insertion sort; runs are
 // short unless particles coincide).
 __global__ __launch_bounds__(256) void tie_fix_kernel(const unsigned long long* __restrict__ keys,
@@ -287,15 +541,80 @@ size_t radix_hist_words(size_t n)
     return 256 * tiles + scan_block_sums_words(256 * tiles);
 }
 
-int radix_sort_passes(int key_bits) { return (key_bits + 7) / 8; }
+namespace {
+
+// Tile sort and merge, or LSD radix? The radix sort's time is its passes' (20 us
+// each up to 65,536 pairs: three launches that leave the chip idle; 84 us at
+// 8,388,608), whatever their order; the merge sort adds a pass per doubling of
+// n past the tile. Sorts inside a build, us, merge / radix: 4,099 pairs 38 / 140,
+// 65,536 64 / 182, 1,048,576 128 / 212, 4,194,304 370 / 416, 8,388,608
+// 750 / 672. With 4 passes (30-bit keys) they meet near 131,072 pairs (110 / 114).
+bool use_merge(size_t n, int key_bits)
+{
+    const int passes = (key_bits + 7) / 8;
+    return passes > 1 && n <= (static_cast<size_t>(4096) << (5 * passes / 4));
+}
+
+// Threads of a tile's workgroup (8 pairs each). A tile is one workgroup's latency,
+// 2.5 us per doubling with 512 threads, 4 with 1,024: the larger tile pays once
+// it saves a pass over many pairs (2,097,152: 187 / 179 us).
+int tile_threads(size_t n) { return n <= 2048 ? 256 : n <= 1200000 ? 512 : 1024; }
+
+// Returns true when the result is in the first output pair. Reads `in` only in the
+// first pass.
+template <bool FULL, class In>
+bool merge_sort(const In& in, unsigned long long* kout, uint32_t* vout, unsigned long long* knext,
+                uint32_t* vnext, size_t n, unsigned long long kmask, hipStream_t stream)
+{
+    const int threads = tile_threads(n);
+    const size_t tile = static_cast<size_t>(threads) * kMergePer;
+    const unsigned nt = static_cast<unsigned>((n + tile - 1) / tile);
+    if (threads == 256)
+        tile_sort_kernel<256, FULL><<<nt, 256, 0, stream>>>(in, kout, vout, n, kmask);
+    else if (threads == 512)
+        tile_sort_kernel<512, FULL><<<nt, 512, 0, stream>>>(in, kout, vout, n, kmask);
+    else
+        tile_sort_kernel<1024, FULL><<<nt, 1024, 0, stream>>>(in, kout, vout, n, kmask);
+    const unsigned nb = static_cast<unsigned>((n + kMergeOut - 1) / kMergeOut);
+    bool first = true;
+    for (size_t run = tile; run < n; run *= 2) {
+        merge_kernel<FULL><<<nb, kMergeBlock, 0, stream>>>(kout, vout, knext, vnext, n, run, kmask);
+        std::swap(kout, knext);
+        std::swap(vout, vnext);
+        first = !first;
+    }
+    return first;
+}
+
+}  // namespace
+
+int radix_sort_passes(size_t n, int key_bits)
+{
+    if (!use_merge(n, key_bits))
+        return (key_bits + 7) / 8;
+    int passes = 1;  // the tiles
+    for (size_t run = static_cast<size_t>(tile_threads(n)) * kMergePer; run < n; run *= 2)
+        ++passes;
+    return passes;
+}
+
+bool sort_uses_scan(size_t n, int key_bits) { return !use_merge(n, key_bits); }
 
 bool radix_sort_from(const uint64_t* keys_in, const uint32_t* vals_in, uint64_t* keys_a,
                      uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b, uint32_t* hist_ws,
                      size_t n, int key_bits, int* err, hipStream_t stream)
 {
-    const int passes = radix_sort_passes(key_bits);
+    const int passes = radix_sort_passes(n, key_bits);
     if (n <= 1)
         return false;
+    if (use_merge(n, key_bits)) {
+        const PairsIn in{reinterpret_cast<const unsigned long long*>(keys_in), vals_in};
+        unsigned long long* ka = reinterpret_cast<unsigned long long*>(keys_a);
+        unsigned long long* kb = reinterpret_cast<unsigned long long*>(keys_b);
+        return key_bits < 64 ? merge_sort<false>(in, ka, vals_a, kb, vals_b, n,
+                                                 (1ull << key_bits) - 1ull, stream)
+                             : merge_sort<true>(in, ka, vals_a, kb, vals_b, n, ~0ull, stream);
+    }
     const uint32_t ntiles = static_cast<uint32_t>((n + kTile - 1) / kTile);
     const size_t hn = static_cast<size_t>(ntiles) * 256;
     uint32_t* hist = hist_ws;
@@ -339,6 +658,26 @@ void launch_radix_sort(Device& d, size_t n, int key_bits)
     if (radix_sort_buffers(d.keys, d.keys_b, d.vals, d.vals_b, d.sort_hist, n, key_bits, d.err,
                            d.stream)) {
         // Result is in the alternate buffers: swap the roles so d.keys/d.vals hold it.
+        std::swap(d.keys, d.keys_b);
+        std::swap(d.vals, d.vals_b);
+    }
+}
+
+bool use_keys_sort(size_t n, int key_mode) { return n > 1 && use_merge(n, key_mode == 1 ? 30 : 63); }
+
+void launch_keys_sort(Device& d, int key_mode)
+{
+    // keys end in d.keys_b / d.vals_b when the first output pair holds them
+    unsigned long long* ka = reinterpret_cast<unsigned long long*>(d.keys_b);
+    unsigned long long* kb = reinterpret_cast<unsigned long long*>(d.keys);
+    // (63- and 30-bit keys hold nothing above those bits: they compare whole)
+    const bool first =
+        key_mode == 1
+            ? merge_sort<true>(PositionsIn<1>{d.pos[0], d.pos[1], d.pos[2], d.geom}, ka, d.vals_b,
+                               kb, d.vals, d.n, ~0ull, d.stream)
+            : merge_sort<true>(PositionsIn<0>{d.pos[0], d.pos[1], d.pos[2], d.geom}, ka, d.vals_b,
+                               kb, d.vals, d.n, ~0ull, d.stream);
+    if (first) {
         std::swap(d.keys, d.keys_b);
         std::swap(d.vals, d.vals_b);
     }

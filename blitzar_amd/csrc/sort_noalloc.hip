@@ -14,7 +14,7 @@
 // made on it; host code only ever passes that looked-up address to kernels.
 // Every call on one GPU shares the array: calls that overlap on one GPU (two
 // streams, two threads) race and give wrong results. The error word is
-// cleared by a fill kernel at the start of each call; the scan status words
+// cleared by a fill kernel at the start of each call that scans; the scan status words
 // carry an epoch (scan_lookback.h), so they need clearing only once, at
 // set-up; the histograms are fully rewritten by every pass.
 #include "../../include/bh_hip.h"
@@ -150,14 +150,16 @@ bh_hip_result_t bh_hip_sort_pairs_noalloc(const uint64_t* keys, const uint32_t* 
         }
         return BH_HIP_OK;
     }
-    bh::launch_fill_u32(reinterpret_cast<uint32_t*>(flags), 0u, 1, s);
+    const bool scans = bh::sort_uses_scan(n, key_bits);  // else nothing raises a flag
+    if (scans)
+        bh::launch_fill_u32(reinterpret_cast<uint32_t*>(flags), 0u, 1, s);
     // The passes alternate between two buffer pairs and must end in the
     // output. Disjoint input and output: the output is the pair the last pass
     // writes, the scratch pair the other. Sorting in place (either output
     // array is its input): pass 0 must not write the input, so it writes the
     // scratch pair; an odd pass count then ends there and is copied out.
     const bool in_place = keys_out == keys || vals_out == vals;
-    const bool odd = (bh::radix_sort_passes(key_bits) & 1) != 0;
+    const bool odd = (bh::radix_sort_passes(n, key_bits) & 1) != 0;
     bool copy_out = false;
     if (!in_place) {
         if (odd)
@@ -178,7 +180,7 @@ bh_hip_result_t bh_hip_sort_pairs_noalloc(const uint64_t* keys, const uint32_t* 
             e = hipMemcpyAsync(vals_out, svals, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
     }
     int host_flags = 0;
-    if (e == hipSuccess)
+    if (e == hipSuccess && scans)
         e = hipMemcpyAsync(&host_flags, flags, sizeof(int), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess)
         e = hipStreamSynchronize(s);

@@ -150,7 +150,8 @@ typedef struct bh_hip_timings {
     uint64_t mono_interactions; /* relative_mono: accepted nodes evaluated as point masses
                                    (per target; also counted in pp_interactions) */
     /* parts of build_ms */
-    double keys_ms;     /* AABB + Morton keys */
+    double keys_ms;     /* AABB, and the Morton keys unless the sort makes them
+                           (builds of up to 4,194,304 particles) */
     double permute_ms;  /* equal-key tie order + store permutation */
     double tree_ms;     /* topology, from the end of the sort (it runs beside the
                            permutation, on a second stream) */
