@@ -292,7 +292,8 @@ bool alloc_all(bh_hip_handle* h, uint64_t n)
         !dalloc(h, &d.groups, n, "groups"))
         return false;
     d.sort_hist_cap = bh::radix_hist_words(n);
-    if (!dalloc_zero(h, &d.sort_hist, d.sort_hist_cap, "sort hist", d.stream))
+    if (!dalloc_zero(h, &d.sort_hist, d.sort_hist_cap, "sort hist", d.stream) ||
+        !dalloc(h, &d.cross, bh::cross_words(n), "straddling nodes"))
         return false;
     if (!dalloc(h, &d.level_info, 2 * bh::kLevels + 8, "level info") ||
         !dalloc(h, &d.geom, 1, "geometry") ||

@@ -126,10 +126,17 @@ enum DeviceError : int {
 // One-pass tree topology (k_tree.hip): tiles of kTopoTile sorted keys; it
 // handles buckets of up to kTopoHalo particles (wider ones build level by
 // level). Its per-tile, per-level node counts need topo_count_words(n) words.
-constexpr int kTopoTile = 4096;
+constexpr int kTopoTile = 1024;
 constexpr int kTopoHalo = 64;
 inline uint32_t topo_tiles(size_t n) { return static_cast<uint32_t>((n + kTopoTile - 1) / kTopoTile); }
 inline size_t topo_count_words(size_t n) { return static_cast<size_t>(kLevels) * (topo_tiles(n) + 1); }
+// Nodes left over by the moments' passes over tiles (kLevels words per unit of
+// each pass, see cross_moments_kernel; the passes' units shrink 512-fold).
+inline size_t cross_words(size_t n)
+{
+    const size_t t = topo_tiles(n);
+    return static_cast<size_t>(kLevels) * (t + t / 512 + t / 262144 + 4);
+}
 
 // Parameters the walk needs (by value into the kernel).
 struct WalkParams {
@@ -224,6 +231,8 @@ struct Device {
     uint32_t* bnd_tmp = nullptr;   // per-level child bounds (8 per node) from count to emit
     uint32_t* big_list = nullptr;  // per-level indices of nodes searched by a whole wavefront
     uint32_t* topo_cnt = nullptr;  // one-pass topology: node counts per tile and level
+    bool topo_tiled = false;       // the last topology came from the one-pass build
+    uint32_t* cross = nullptr;     // moments: nodes that straddle tiles (cross_words)
     uint32_t* scan_blocks = nullptr;
     int* level_info = nullptr;  // [0..22) base, [22..44) count, [44] total, [45] max level, [46] groups
 

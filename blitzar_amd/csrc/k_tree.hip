@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256) void tree_emit_kernel(
 // the one at hi_s a leaf and each other the parent of the next. Level L's
 // nodes in breadth-first order are the particles with lo_s <= L <= hi_s in
 // increasing order, so a node's index is its level's base plus its rank
-// among them. Passes: per 4,096-particle tile, each particle's [lo, hi] (one
+// among them. Passes: per 1,024-particle tile, each particle's [lo, hi] (one
 // word) and the tile's node count per level; a scan of the counts per level;
 // per tile, the nodes in place; then, per node, what a tile cannot see
 // (parents of later siblings, child counts, counts of internal nodes and of
@@ -523,8 +523,8 @@ __global__ __launch_bounds__(kTopoThreads) void topo_count_kernel(
     }
 }
 
-// Exclusive scan of each level's tile counts (one block per level, in place);
-// the level totals go to tilecnt[kLevels * ntiles + L].
+// Exclusive scan of each level's tile counts (one block per level, 4 tiles per
+// thread, in place); the level totals go to tilecnt[kLevels * ntiles + L].
 __global__ __launch_bounds__(kScanBlock) void topo_scan_kernel(uint32_t* __restrict__ tilecnt,
                                                                uint32_t ntiles)
 {
@@ -532,13 +532,20 @@ __global__ __launch_bounds__(kScanBlock) void topo_scan_kernel(uint32_t* __restr
     const int L = blockIdx.x;
     uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
     uint32_t carry = 0;
-    for (uint32_t b = 0; b < ntiles; b += kScanBlock) {
-        const uint32_t t = b + threadIdx.x;
-        const uint32_t v = t < ntiles ? col[t] : 0u;
+    for (uint32_t b = 0; b < ntiles; b += 4 * kScanBlock) {
+        const uint32_t t = b + 4 * threadIdx.x;
+        uint32_t v[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            v[k] = t + k < ntiles ? col[t + k] : 0u;
         uint32_t total = 0;
-        const uint32_t ex = block_exclusive256(v, tmp, &total);
-        if (t < ntiles)
-            col[t] = carry + ex;
+        uint32_t ex = carry + block_exclusive256((v[0] + v[1]) + (v[2] + v[3]), tmp, &total);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            if (t + k < ntiles)
+                col[t + k] = ex;
+            ex += v[k];
+        }
         carry += total;
     }
     if (threadIdx.x == 0)
@@ -912,6 +919,23 @@ __device__ inline NodeMeta node_meta(int node, const uint64_t* __restrict__ npre
     return NodeMeta{nprefix[node], nchild[node], nfirst[node], ncount[node]};
 }
 
+// Refit (moments of the current positions on an earlier topology):
+// particles may have left their cells. The moments and bmax are
+// exact for the current positions, and a target inside a node's
+// bounding sphere opens it whatever its size. The level the walk
+// derives the cell size from is lowered only once the particles
+// reach beyond 1.5 times the cell's half-width. (The bound e of a
+// parent exceeds its half-width by half its child's excess: lowering
+// at any excess doubled the size of every ancestor of one escaped
+// particle, up to the root, and the 8M block-step walk took 1.3-4x
+// longer than after a rebuild.) A fresh build keeps the true level.
+__device__ inline int refit_level(int level, float e)
+{
+    while (level > 0 && 1.5f * ldexpf(1.0f, kMaxLevel - level) < e)
+        --level;
+    return level;
+}
+
 template <bool OCT, bool LEAF, class Part>
 __device__ inline void node_moments(int node, int level, const NodeMeta& meta,
                                     const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn,
@@ -1035,21 +1059,7 @@ __device__ inline void node_moments(int node, int level, const NodeMeta& meta,
             for (int k = 0; k < 10; ++k)
                 o[k] = oc.t[k];
         }
-        // Refit (moments of the current positions on an earlier topology):
-        // particles may have left their cells. The moments and bmax are
-        // exact for the current positions, and a target inside a node's
-        // bounding sphere opens it whatever its size. The level the walk
-        // derives the cell size from is lowered only once the particles
-        // reach beyond 1.5 times the cell's half-width. (The bound e of a
-        // parent exceeds its half-width by half its child's excess: lowering
-        // at any excess doubled the size of every ancestor of one escaped
-        // particle, up to the root, and the 8M block-step walk took 1.3-4x
-        // longer than after a rebuild.) A fresh build keeps the true level.
-        int wlevel = level;
-        if (refit) {
-            while (wlevel > 0 && 1.5f * ldexpf(1.0f, kMaxLevel - wlevel) < e)
-                --wlevel;
-        }
+        const int wlevel = refit ? refit_level(level, e) : level;
         WalkNode w;
         w.comx = cx;
         w.comy = cy;
@@ -1161,6 +1171,321 @@ __global__ __launch_bounds__(kLeafThreads) void leaf_moments_kernel(
     }
 }
 
+constexpr uint32_t kNoNode = 0xffffffffu;
+
+// An internal node summed by 8 lanes, one child each: node_moments' loop over the
+// children is one wavefront's chain of about 700 dependent instructions (2.5 us)
+// whatever the number of nodes; here the children's terms are formed side by
+// side and only the additions stay in sequence, one quantity per lane, through
+// LDS. The same operations in the same order: the same bits. Lanes 8 g .. 8 g + 7 of
+// the wavefront take node g (kNoNode: none); every lane calls it.
+template <bool OCT>
+struct CoopLds {
+    float a[8][8][4];                          // child: mass, position
+    float b[8][8][8];                          // child: second-order terms, trs, bmax, extent
+    float o[OCT ? 8 : 1][OCT ? 8 : 1][10];     // child: third-order terms
+    float out[8][16];                          // the node record
+};
+
+__device__ inline void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool OCT>
+__device__ inline void node_moments_coop(CoopLds<OCT>& S, uint32_t node, int level,
+                                         const NodeMeta& meta, const RootGeom* __restrict__ geom,
+                                         WalkNode* __restrict__ wn, float* __restrict__ ext,
+                                         float* __restrict__ noct, int refit)
+{
+    const int g = (threadIdx.x & 63) >> 3, j = threadIdx.x & 7;
+    const bool on = node != kNoNode;
+    const uint32_t nc = on ? meta.nchild : 1u;
+    const bool live = static_cast<uint32_t>(j) < nc;
+    const uint32_t child = on ? meta.first + (live ? static_cast<uint32_t>(j) : nc - 1u) : 0u;
+    const WalkNode ch = wn[child];  // (no node: the root's slot, read and dropped)
+    const float ux = geom->unit_f[0], uy = geom->unit_f[1], uz = geom->unit_f[2];
+    // the node's lattice centre from a child's: one level up
+    const int sh = kMaxLevel - level;
+    int c[3] = {ch.cx, ch.cy, ch.cz};
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        c[a] = static_cast<int>(
+            ((2u * (static_cast<uint32_t>(c[a] + 1) >> (sh + 1)) + 1u) << sh) - 1u);
+    const float rx = __fmaf_rn(static_cast<float>(ch.cx - c[0]), ux, ch.comx);
+    const float ry = __fmaf_rn(static_cast<float>(ch.cy - c[1]), uy, ch.comy);
+    const float rz = __fmaf_rn(static_cast<float>(ch.cz - c[2]), uz, ch.comz);
+    *reinterpret_cast<float4*>(S.a[g][j]) = make_float4(live ? ch.mass : 0.0f, rx, ry, rz);
+    wave_lds_fence();
+    float acc = 0.0f;  // lanes 0 and 4: mass; the others: one axis each
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        acc = __fmaf_rn(S.a[g][k][0], (j & 3) == 0 ? 1.0f : S.a[g][k][j & 3], acc);
+    wave_lds_fence();
+    if (j < 4)
+        S.a[g][0][j] = acc;
+    wave_lds_fence();
+    const float4 sum = *reinterpret_cast<const float4*>(S.a[g][0]);
+    const float M = sum.x;
+    float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+    if (M > 0.0f) {
+        cx = sum.y / M;
+        cy = sum.z / M;
+        cz = sum.w / M;
+    }
+    const float dx = __fsub_rn(rx, cx), dy = __fsub_rn(ry, cy), dz = __fsub_rn(rz, cz);
+    const float r2 = norm2_rn(dx, dy, dz);
+    const float tx = __fmul_rn(3.0f, dx), ty = __fmul_rn(3.0f, dy);
+    const float m = ch.mass;
+    float e = 0.0f;
+    if (refit && live && on) {
+        const int off = max(abs(ch.cx - c[0]), max(abs(ch.cy - c[1]), abs(ch.cz - c[2])));
+        e = ext[child] + static_cast<float>(off);
+    }
+    float* t = S.b[g][j];
+    t[0] = live ? __fmaf_rn(m, __fmaf_rn(tx, dx, -r2), ch.qxx) : 0.0f;
+    t[1] = live ? __fmaf_rn(m, __fmul_rn(tx, dy), ch.qxy) : 0.0f;
+    t[2] = live ? __fmaf_rn(m, __fmul_rn(tx, dz), ch.qxz) : 0.0f;
+    t[3] = live ? __fmaf_rn(m, __fmaf_rn(ty, dy, -r2), ch.qyy) : 0.0f;
+    t[4] = live ? __fmaf_rn(m, __fmul_rn(ty, dz), ch.qyz) : 0.0f;
+    t[5] = live ? __fmaf_rn(m, r2, ch.trs) : 0.0f;
+    t[6] = live && m > 0.0f ? __fadd_rn(sqrtf(r2), ch.bmax) : 0.0f;
+    t[7] = e;
+    if (OCT) {
+        Oct oc;
+        oct_zero(oc);
+        if (live && on)
+            oct_add_child(oc, noct + static_cast<size_t>(child) * 10, ch, dx, dy, dz);
+#pragma unroll
+        for (int k = 0; k < 10; ++k)
+            S.o[OCT ? g : 0][OCT ? j : 0][k] = oc.t[k];
+    }
+    wave_lds_fence();
+    acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float v = S.b[g][k][j];
+        acc = j < 6 ? __fadd_rn(acc, v) : fmaxf(acc, v);
+    }
+    float* w = S.out[g];
+    if (j < 5)
+        w[4 + j] = acc;
+    else if (j == 5)
+        w[10] = acc;
+    else if (j == 6)
+        w[9] = acc;
+    else {
+        if (refit && on)
+            ext[node] = acc;
+        int* wi = reinterpret_cast<int*>(w);
+        w[0] = cx;
+        w[1] = cy;
+        w[2] = cz;
+        w[3] = M;
+        wi[11] = static_cast<int>(meta.first);
+        wi[12] = c[0];
+        wi[13] = c[1];
+        wi[14] = c[2];
+        wi[15] = static_cast<int>(make_meta(
+            nc, static_cast<uint32_t>(refit ? refit_level(level, acc) : level),
+            min(meta.count, kMaxLeafCount)));
+    }
+    wave_lds_fence();
+    if (on) {
+        reinterpret_cast<float2*>(wn + node)[j] = *reinterpret_cast<const float2*>(&w[2 * j]);
+        if (OCT) {
+            for (int k = j; k < 10; k += 8) {
+                float v = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    v += S.o[OCT ? g : 0][OCT ? q : 0][k];
+                noct[static_cast<size_t>(node) * 10 + k] = v;
+            }
+        }
+    }
+    wave_lds_fence();  // the next call writes S
+}
+
+// The nodes that the lanes of one wavefront hold (has; node, meta each) on one
+// level: a few by 8 lanes each, many by a lane each.
+constexpr int kCoopMax = 16;
+
+template <bool OCT>
+__device__ inline void wave_nodes(CoopLds<OCT>& S, bool has, uint32_t node, int level,
+                                  const NodeMeta& meta, const RootGeom* __restrict__ geom,
+                                  WalkNode* __restrict__ wn, float* __restrict__ ext,
+                                  float* __restrict__ noct, int refit, int* err)
+{
+    unsigned long long m = __ballot(has);
+    if (__popcll(m) > kCoopMax) {
+        if (has)
+            node_moments<OCT, false>(static_cast<int>(node), level, meta, geom, wn, ext, noct,
+                                     refit, err, [](uint32_t, const double*) { return float4{}; });
+        return;
+    }
+    while (m) {
+        // group g of lanes takes the g-th holder's node
+        const int g = (threadIdx.x & 63) >> 3;
+        unsigned long long k = m;
+        for (int i = 0; i < g; ++i)
+            k &= k - 1ull;
+        const int src = k ? __builtin_ctzll(k) : 0;
+        NodeMeta t;
+        t.nchild = __shfl(meta.nchild, src, 64);
+        t.first = __shfl(meta.first, src, 64);
+        t.count = __shfl(meta.count, src, 64);
+        const uint32_t at = __shfl(node, src, 64);
+        node_moments_coop<OCT>(S, k ? at : kNoNode, level, t, geom, wn, ext, noct, refit);
+        for (int i = 0; i < 8 && m; ++i)
+            m &= m - 1ull;
+    }
+}
+
+// Internal nodes, after the leaves, of a tree from the one-pass topology, whose
+// scanned counts say which nodes of each level start in a tile. One wavefront per
+// tile sums, level by level, the internal nodes that lie whole inside the tile,
+// and leaves in cross[L][tile] the one node of each level (if any) that starts in
+// it and ends past it; cross_moments_kernel takes those. Bound: latency (about
+// 1.5 us a level; 4-6 levels of a tile hold internal nodes). One launch per level
+// for all internal nodes, 21 launches, took 62 us at 4,099 particles, 88 at
+// 65,536 and 254 at 8,388,608; the tiles and what they leave take 41, 61 and 210.
+template <bool OCT>
+__global__ __launch_bounds__(64, 3) void tile_moments_kernel(
+    const uint64_t* __restrict__ nprefix, const uint32_t* __restrict__ nstart,
+    const uint32_t* __restrict__ ncount, const uint32_t* __restrict__ nchild,
+    const uint32_t* __restrict__ nfirst, const int* __restrict__ info,
+    const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn, float* __restrict__ ext,
+    float* __restrict__ noct, int refit, int* err, const uint32_t* __restrict__ tilecnt,
+    uint32_t ntiles, uint32_t* __restrict__ cross)
+{
+    __shared__ CoopLds<OCT> S;
+    __shared__ uint32_t lvFirst[kLevels], lvEnd[kLevels];  // the tile's nodes per level
+    const uint32_t tile = blockIdx.x;
+    const uint32_t lim = (tile + 1u) * kTopoTile;
+    bool any = false;
+    if (threadIdx.x < kLevels) {
+        const int L = threadIdx.x;
+        const uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
+        const uint32_t c0 = col[tile];
+        const uint32_t c1 =
+            tile + 1 < ntiles ? col[tile + 1] : tilecnt[static_cast<size_t>(kLevels) * ntiles + L];
+        const bool kept = info[kLevels + L] > 0;  // levels past the node capacity were dropped
+        any = kept && c1 > c0 && L < kMaxLevel;
+        lvFirst[L] = static_cast<uint32_t>(info[L]) + c0;
+        lvEnd[L] = static_cast<uint32_t>(info[L]) + (kept ? c1 : c0);
+        cross[static_cast<size_t>(L) * ntiles + tile] = kNoNode;
+    }
+    uint32_t levels = static_cast<uint32_t>(__ballot(any));  // those with nodes
+    __syncthreads();
+    NodeMeta meta, next = {};
+    uint32_t start = 0u, nextStart = 0u;
+    const auto fetch = [&](uint32_t node, uint32_t end, NodeMeta& m, uint32_t& s) {
+        m = NodeMeta{};
+        if (node < end) {
+            m = node_meta(static_cast<int>(node), nprefix, ncount, nchild, nfirst);
+            s = nstart[node];
+        }
+    };
+    const auto sum = [&](uint32_t node, int L) {
+        const bool in = meta.nchild != 0u;  // (else a leaf, or no node)
+        const bool past = in && start + meta.count > lim;
+        if (past)  // at most one node of a level
+            cross[static_cast<size_t>(L) * ntiles + tile] = node;
+        wave_nodes<OCT>(S, in && !past, node, L, meta, geom, wn, ext, noct, refit, err);
+    };
+    int L = levels ? 31 - __builtin_clz(levels) : -1;
+    if (L >= 0)
+        fetch(lvFirst[L] + threadIdx.x, lvEnd[L], next, nextStart);
+    while (L >= 0) {
+        const uint32_t e = lvEnd[L];
+        uint32_t node = lvFirst[L] + threadIdx.x;
+        levels ^= 1u << L;
+        const int above = levels ? 31 - __builtin_clz(levels) : -1;
+        meta = next;
+        start = nextStart;
+        if (above >= 0)  // the next level's fields while this one is summed
+            fetch(lvFirst[above] + threadIdx.x, lvEnd[above], next, nextStart);
+        sum(node, L);
+        for (uint32_t at = lvFirst[L] + 64u; at < e; at += 64u) {  // the whole wavefront
+            node += 64u;
+            fetch(node, e, meta, start);
+            sum(node, L);
+        }
+        __syncthreads();  // the next level reads these nodes
+        L = above;
+    }
+}
+
+// The nodes the tiles left: unit u of this pass is kCrossUnits consecutive units of
+// the pass before (of tiles, in the first), held by one workgroup. cross_in[L * nin
+// + i] is the node of level L that starts in input unit i and ends past it;
+// the workgroup computes those inside its own unit and passes on the one per
+// level that ends past it. The last pass has one unit, which holds everything.
+constexpr int kCrossUnits = 512;
+
+template <bool OCT>
+__global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
+    const uint64_t* __restrict__ nprefix, const uint32_t* __restrict__ nstart,
+    const uint32_t* __restrict__ ncount, const uint32_t* __restrict__ nchild,
+    const uint32_t* __restrict__ nfirst, const RootGeom* __restrict__ geom,
+    WalkNode* __restrict__ wn, float* __restrict__ ext, float* __restrict__ noct, int refit,
+    int* err, const uint32_t* __restrict__ cross_in, uint32_t nin, uint64_t unit,
+    uint32_t* __restrict__ cross_out, uint32_t nout)
+{
+    __shared__ CoopLds<OCT> S[kCrossUnits / 64];
+    __shared__ uint32_t sNode[kMaxLevel][kCrossUnits];
+    __shared__ uint32_t sLevels;  // bit L: this unit holds input nodes of level L
+    const uint32_t i = blockIdx.x * kCrossUnits + threadIdx.x;
+    const uint64_t lim = (static_cast<uint64_t>(blockIdx.x) + 1) * unit;
+    if (threadIdx.x == 0)
+        sLevels = 0u;
+    uint32_t has = 0u;
+#pragma unroll
+    for (int L = 0; L < kMaxLevel; ++L) {
+        const uint32_t v = i < nin ? cross_in[static_cast<size_t>(L) * nin + i] : kNoNode;
+        sNode[L][threadIdx.x] = v;
+        has |= v != kNoNode ? 1u << L : 0u;
+    }
+    if (nout > 1 && threadIdx.x < kMaxLevel)
+        cross_out[static_cast<size_t>(threadIdx.x) * nout + blockIdx.x] = kNoNode;
+    __syncthreads();
+    if (has)
+        atomicOr(&sLevels, has);
+    __syncthreads();
+    uint32_t levels = sLevels;
+    NodeMeta meta, next = {};
+    uint32_t node = kNoNode, start = 0u, nextNode = kNoNode, nextStart = 0u;
+    const auto fetch = [&](int L) {
+        nextNode = sNode[L][threadIdx.x];
+        if (nextNode != kNoNode) {
+            next = node_meta(static_cast<int>(nextNode), nprefix, ncount, nchild, nfirst);
+            nextStart = nstart[nextNode];
+        }
+    };
+    int L = levels ? 31 - __builtin_clz(levels) : -1;
+    if (L >= 0)
+        fetch(L);
+    while (L >= 0) {
+        levels ^= 1u << L;
+        const int above = levels ? 31 - __builtin_clz(levels) : -1;
+        node = nextNode;
+        meta = next;
+        start = nextStart;
+        if (above >= 0)  // the next level's fields while this one is summed
+            fetch(above);
+        const bool past = node != kNoNode && nout > 1 &&
+                          static_cast<uint64_t>(start) + meta.count > lim;
+        if (past)
+            cross_out[static_cast<size_t>(L) * nout + blockIdx.x] = node;
+        wave_nodes<OCT>(S[threadIdx.x >> 6], node != kNoNode && !past, node, L, meta, geom, wn,
+                        ext, noct, refit, err);
+        __syncthreads();
+        L = above;
+    }
+}
+
 // sleaf[s] = the leaf holding particle s (topology built level by level).
 __global__ __launch_bounds__(256) void leaf_fill_kernel(const uint32_t* __restrict__ nstart,
                                                         const uint32_t* __restrict__ ncount,
@@ -1178,8 +1503,8 @@ __global__ __launch_bounds__(256) void leaf_fill_kernel(const uint32_t* __restri
     }
 }
 
-// Internal nodes of one level (deepest level first, after the leaves), one
-// thread per node of the level. (Listing the internal ones first so that
+// Internal nodes of one level (deepest level first, after the leaves) of a tree
+// built level by level, one thread per node of the level. (Listing the internal ones first so that
 // whole wavefronts sum them was slower: the level is latency-bound, and the
 // mostly idle wavefronts of this form keep more loads in flight.)
 template <bool OCT>
@@ -1336,7 +1661,8 @@ void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s)
 {
     const uint32_t n = static_cast<uint32_t>(d.n);
     const unsigned long long* sorted = reinterpret_cast<const unsigned long long*>(d.keys);
-    if (n > 0 && bucket <= kTopoHalo && d.topo_cnt) {
+    d.topo_tiled = n > 0 && bucket <= kTopoHalo && d.topo_cnt;
+    if (d.topo_tiled) {
         const uint32_t ntiles = topo_tiles(d.n);
         uint32_t* pinfo = d.bnd_tmp;  // n words (the level-by-level build's child bounds)
         if (bucket == 16)  // the default
@@ -1393,36 +1719,54 @@ void launch_groups(Device& d, uint32_t gmax, hipStream_t s)
                                                d.nparent, d.gscan, d.level_info, d.groups, gmax);
 }
 
-void launch_tree_moments(Device& d, bool refit)
+namespace {
+
+template <bool OCT>
+void launch_moments_t(Device& d, int rf)
 {
-    const int rf = refit ? 1 : 0;
     const uint32_t n = static_cast<uint32_t>(d.n);
-    const unsigned gl = static_cast<unsigned>((d.n + kLeafChunk - 1) / kLeafChunk);
-    if (gl > 0) {
-        if (d.noct)
-            leaf_moments_kernel<true><<<gl, kLeafThreads, 0, d.stream>>>(
-                d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.sleaf, n,
-                d.level_info, d.pos[0], d.pos[1], d.pos[2], d.mass, d.geom, d.wnode, d.spart,
-                d.next, d.noct, rf, d.err);
-        else
-            leaf_moments_kernel<false><<<gl, kLeafThreads, 0, d.stream>>>(
-                d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.sleaf, n,
-                d.level_info, d.pos[0], d.pos[1], d.pos[2], d.mass, d.geom, d.wnode, d.spart,
-                d.next, nullptr, rf, d.err);
+    float* noct = OCT ? d.noct : nullptr;
+    leaf_moments_kernel<OCT>
+        <<<(n + kLeafChunk - 1) / kLeafChunk, kLeafThreads, 0, d.stream>>>(
+            d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.sleaf, n, d.level_info,
+            d.pos[0], d.pos[1], d.pos[2], d.mass, d.geom, d.wnode, d.spart, d.next, noct, rf,
+            d.err);
+    if (d.topo_tiled) {
+        uint32_t* in = d.cross;
+        uint32_t nin = topo_tiles(d.n);
+        uint64_t unit = kTopoTile;
+        tile_moments_kernel<OCT><<<nin, 64, 0, d.stream>>>(
+            d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.level_info, d.geom, d.wnode,
+            d.next, noct, rf, d.err, d.topo_cnt, nin, in);
+        while (nin > 1) {
+            uint32_t* out = in + static_cast<size_t>(kLevels) * nin;
+            const uint32_t nout = (nin + kCrossUnits - 1) / kCrossUnits;
+            unit *= kCrossUnits;
+            cross_moments_kernel<OCT><<<nout, kCrossUnits, 0, d.stream>>>(
+                d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.geom, d.wnode, d.next, noct,
+                rf, d.err, in, nin, unit, out, nout);
+            in = out;
+            nin = nout;
+        }
+        return;
     }
     // level kMaxLevel holds leaves only
-    for (int L = kMaxLevel - 1; L >= 0; --L) {
-        const size_t bound = level_bound(L, d.n, d.node_cap);
-        const unsigned g = level_grid(bound);
-        if (d.noct)
-            tree_moments_kernel<true><<<g, 256, 0, d.stream>>>(
-                d.nprefix, d.ncount, d.nchild, d.nfirst, d.level_info, L, d.geom, d.wnode, d.next,
-                d.noct, rf, d.err);
-        else
-            tree_moments_kernel<false><<<g, 256, 0, d.stream>>>(
-                d.nprefix, d.ncount, d.nchild, d.nfirst, d.level_info, L, d.geom, d.wnode, d.next,
-                nullptr, rf, d.err);
-    }
+    for (int L = kMaxLevel - 1; L >= 0; --L)
+        tree_moments_kernel<OCT><<<level_grid(level_bound(L, d.n, d.node_cap)), 256, 0, d.stream>>>(
+            d.nprefix, d.ncount, d.nchild, d.nfirst, d.level_info, L, d.geom, d.wnode, d.next,
+            noct, rf, d.err);
+}
+
+}  // namespace
+
+void launch_tree_moments(Device& d, bool refit)
+{
+    if (d.n == 0)
+        return;
+    if (d.noct)
+        launch_moments_t<true>(d, refit ? 1 : 0);
+    else
+        launch_moments_t<false>(d, refit ? 1 : 0);
 }
 
 }  // namespace bh
