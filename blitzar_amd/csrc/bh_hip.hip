@@ -71,10 +71,10 @@ struct bh_hip_handle {
     // A failed device allocation after creation leaves the handle unusable:
     // every later call returns an error with this message.
     std::string broken;
-    // Error word of the device copied (pinned) after each build, and the event
-    // that marks the copy; read while the walk queued behind the build runs.
-    int* err_host = nullptr;
+    // Marks the end of a build, whose last kernel writes the error word to
+    // d.report; read while the walk queued behind the build runs.
     hipEvent_t built = nullptr;
+    bool reported = false;  // d.report holds the end of the current call
     // The topology and the walk groups of a build run on a second stream
     // (default priority), beside the store permutation and the moments:
     // sorted -> topology (side), topo -> moments (main), groups -> walk (main).
@@ -326,6 +326,24 @@ bool zero_err(bh_hip_handle* h)
     return check(h, hipGetLastError(), "error flag reset");
 }
 
+bool ensure_ring(bh_hip_handle* h, size_t bytes)
+{
+    if (h->pinned_bytes >= bytes)
+        return true;
+    if (h->pinned)
+        (void)hipHostFree(h->pinned);
+    h->pinned = nullptr;
+    h->pinned_bytes = 0;
+    if (!check(h, hipHostMalloc(reinterpret_cast<void**>(&h->pinned), bytes,
+                                hipHostMallocDefault),
+               "pinned copy buffer")) {
+        (void)hipGetLastError();
+        return false;
+    }
+    h->pinned_bytes = bytes;
+    return true;
+}
+
 // Device memory to pageable caller memory. The runtime's own copy of pageable
 // memory drains its staging buffer with one host thread, 10 GB/s into memory
 // the caller has not touched yet (the thread takes the page faults). Here the
@@ -344,20 +362,8 @@ bool copy_out(bh_hip_handle* h, void* dst, const void* src, size_t bytes, const 
         std::clamp((bytes / kRingSlots + 4095) & ~static_cast<size_t>(4095), kRingChunkMin,
                    kRingChunk);
     const size_t nchunks = (bytes + chunk - 1) / chunk;
-    const size_t ring = std::min(nchunks, kRingSlots) * chunk;
-    if (h->pinned_bytes < ring) {
-        if (h->pinned)
-            (void)hipHostFree(h->pinned);
-        h->pinned = nullptr;
-        h->pinned_bytes = 0;
-        if (!check(h, hipHostMalloc(reinterpret_cast<void**>(&h->pinned), ring,
-                                    hipHostMallocDefault),
-                   "pinned copy buffer")) {
-            (void)hipGetLastError();
-            return false;
-        }
-        h->pinned_bytes = ring;
-    }
+    if (!ensure_ring(h, std::min(nchunks, kRingSlots) * chunk))
+        return false;
     for (hipEvent_t& e : h->ring_ev)
         if (!e && !check(h, hipEventCreateWithFlags(&e, hipEventDisableTiming), "event"))
             return false;
@@ -443,17 +449,16 @@ constexpr int kFatalBits =
 // Synchronise and turn device error bits into a message.
 bh_hip_result_t finish(bh_hip_handle* h, const char* what)
 {
+    bh::launch_report(h->d, h->stats);
     if (!check(h, hipGetLastError(), what) || !check(h, hipStreamSynchronize(h->d.stream), what))
         return BH_HIP_INTERNAL_ERROR;
+    h->reported = true;
     if (h->pm_failed) {
         h->pm_failed = false;
         h->last_error = std::string("[octree_hip] ") + what + ": rocFFT execution failed";
         return BH_HIP_INTERNAL_ERROR;
     }
-    int flags = 0;
-    if (!check(h, hipMemcpy(&flags, h->d.err, sizeof(int), hipMemcpyDeviceToHost), "error read"))
-        return BH_HIP_INTERNAL_ERROR;
-    flags |= h->err_carry;
+    const int flags = h->d.report->err | h->err_carry;
     h->err_carry = 0;
     if (flags != 0) {
         std::string m = std::string("[octree_hip] ") + what + ":";
@@ -513,7 +518,7 @@ Built check_build(bh_hip_handle* h)
 {
     if (!check(h, hipEventSynchronize(h->built), "build"))
         return Built::kFatal;
-    const int bits = *h->err_host;
+    const int bits = h->d.report->err_build;
     if (!(bits & bh::kErrNodeOverflow))
         return Built::kOk;
     if (!check(h, hipStreamSynchronize(h->d.stream), "build"))
@@ -527,7 +532,7 @@ Built check_build(bh_hip_handle* h)
 }
 
 // Bits of the device error word at the last build (and before it).
-int bits_at_build(const bh_hip_handle* h) { return *h->err_host | h->err_carry; }
+int bits_at_build(const bh_hip_handle* h) { return h->d.report->err_build | h->err_carry; }
 
 StepEvents* next_events(bh_hip_handle* h)
 {
@@ -632,7 +637,7 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
         bh::launch_tree_moments(d);
     (void)hipStreamWaitEvent(d.stream, h->ev_groups, 0);
     rec(ev ? ev->b1 : nullptr, d.stream);
-    (void)hipMemcpyAsync(h->err_host, d.err, sizeof(int), hipMemcpyDeviceToHost, d.stream);
+    bh::launch_end_build(d);
     (void)hipEventRecord(h->built, d.stream);
     h->have_tree = true;
 }
@@ -647,7 +652,7 @@ void queue_refit(bh_hip_handle* h, StepEvents* ev)
         rec(e, d.stream);
     bh::launch_tree_moments(d, true);
     rec(ev ? ev->b1 : nullptr, d.stream);
-    (void)hipMemcpyAsync(h->err_host, d.err, sizeof(int), hipMemcpyDeviceToHost, d.stream);
+    bh::launch_end_build(d);
     (void)hipEventRecord(h->built, d.stream);
 }
 
@@ -793,13 +798,19 @@ void begin_call(bh_hip_handle* h)
 {
     h->events_used = 0;
     h->int_used = 0;
-    bh::launch_fill_u32(reinterpret_cast<uint32_t*>(h->stats), 0u, 16, h->d.stream);
+    h->err_carry = 0;
+    h->reported = false;
+    bh::launch_begin_call(h->d, h->stats);
 }
 
-// After a synchronised call: fold event times and counters into h->t.
+// After a call: fold event times and counters into h->t.
 void end_call(bh_hip_handle* h)
 {
     bh_hip_timings_t t{};
+    if (!h->reported) {  // a call that failed before finish
+        bh::launch_report(h->d, h->stats);
+        h->reported = hipStreamSynchronize(h->d.stream) == hipSuccess;
+    }
     if (h->timing) {
         for (size_t k = 0; k < h->events_used; ++k) {
             const StepEvents& e = h->events[k];
@@ -824,8 +835,9 @@ void end_call(bh_hip_handle* h)
                 t.integrate_ms += a;
         }
     }
-    unsigned long long st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (hipMemcpy(st, h->stats, sizeof(st), hipMemcpyDeviceToHost) == hipSuccess) {
+    if (h->reported) {
+        const unsigned long long* st = h->d.report->stats;
+        const int* info = h->d.report->info;
         t.pp_interactions = st[0];
         t.pc_interactions = st[1];
         t.particle_steps = st[2];
@@ -834,9 +846,6 @@ void end_call(bh_hip_handle* h)
         t.mono_interactions = st[5];
         t.lff_pairs = st[6];
         t.lff_tiles = st[7];
-    }
-    int info[2 * bh::kLevels + 4];
-    if (hipMemcpy(info, h->d.level_info, sizeof(info), hipMemcpyDeviceToHost) == hipSuccess) {
         t.node_count = static_cast<uint64_t>(info[bh::kInfoTotal]);
         t.max_level = info[bh::kInfoMaxLevel];
         t.groups = info[bh::kInfoGroups];
@@ -952,7 +961,8 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
     // due is found on the device; the slices in between have no force
     // evaluation, so one predictor spans them (constant acceleration makes k
     // single-slice predictors one predictor over k q).
-    uint32_t* due = reinterpret_cast<uint32_t*>(d.diag);
+    uint32_t* due = reinterpret_cast<uint32_t*>(d.err + 1);
+    bool due_known = false;  // the last correction found the next due tick
     const uint64_t slices = 1ull << a.levels;
     // The tree is built at the first force evaluation of each global step
     // and refitted (moments of the predicted positions on the same topology)
@@ -966,15 +976,12 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
         const uint64_t end = h->ad_tick + slices;
         bool first_slice = true;
         while (h->ad_tick < end) {
-            const uint32_t t0 = static_cast<uint32_t>(h->ad_tick);
-            bh::launch_adaptive_next_due(d, a, t0, due);
-            uint32_t next = 0;
-            if (!check(h, hipMemcpyAsync(&next, due, sizeof(next), hipMemcpyDeviceToHost,
-                                         d.stream),
-                       "adaptive schedule") ||
-                !check(h, hipStreamSynchronize(d.stream), "adaptive schedule"))
+            if (!due_known)
+                bh::launch_adaptive_next_due(d, a, static_cast<uint32_t>(h->ad_tick), due);
+            bh::launch_due_report(d, due);
+            if (!check(h, hipStreamSynchronize(d.stream), "adaptive schedule"))
                 return fail();
-            const uint64_t t = std::min<uint64_t>(end, h->ad_tick + (next - t0));
+            const uint64_t t = std::min<uint64_t>(end, h->ad_tick + d.report->due);
             bh::launch_adaptive_drift(d, a, static_cast<double>(t - h->ad_tick) * a.quantum);
             h->ad_tick = t;
             const uint32_t tt = static_cast<uint32_t>(t);
@@ -985,7 +992,8 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
             if (!build_and_walk(h, next_events(h), wp, !first_slice && !rebuild_each))
                 return fail();
             first_slice = false;
-            bh::launch_adaptive_correct(d, a, tt, h->stats + 2);
+            bh::launch_adaptive_correct(d, a, tt, h->stats + 2, due);
+            due_known = true;
             if (bits_at_build(h) & kFatalBits) {
                 stop = true;
                 break;
@@ -1097,11 +1105,11 @@ bh_hip_result_t bh_hip_create(const bh_hip_params_t* params, uint64_t n, bh_hip_
         ok = ok && check(h, hipEventCreateWithFlags(x, hipEventDisableTiming), "event");
     ok = ok && alloc_all(h, n);
     ok = ok && check(h, hipEventCreateWithFlags(&h->built, hipEventDisableTiming), "event") &&
-         check(h, hipHostMalloc(reinterpret_cast<void**>(&h->err_host), sizeof(int),
+         check(h, hipHostMalloc(reinterpret_cast<void**>(&h->d.report), sizeof(bh::HostReport),
                                 hipHostMallocDefault),
-               "pinned error word");
+               "pinned report");
     if (ok)
-        *h->err_host = 0;
+        std::memset(h->d.report, 0, sizeof(bh::HostReport));
     if (ok && h->p.pm_mesh > 0 && !bh::pm_setup(h->pm, h->p.pm_mesh, h->d.stream)) {
         h->last_error = "bh_hip_create: particle-mesh setup (rocFFT plans, meshes) failed";
         ok = false;
@@ -1145,8 +1153,8 @@ void bh_hip_destroy(bh_hip_handle_t* h)
     for (hipEvent_t x : {h->ev_sorted, h->ev_topo, h->ev_groups})
         if (x)
             (void)hipEventDestroy(x);
-    if (h->err_host)
-        (void)hipHostFree(h->err_host);
+    if (h->d.report)
+        (void)hipHostFree(h->d.report);
     for (hipEvent_t x : h->ring_ev)
         if (x)
             (void)hipEventDestroy(x);
@@ -1243,6 +1251,21 @@ bh_hip_result_t bh_hip_download(bh_hip_handle_t* h, double* pos3, double* vel3)
     if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     bh::Device& d = h->d;
+    const size_t bytes = 3 * d.n * sizeof(double);
+    if (bytes <= kRingChunkMin && ensure_ring(h, 2 * bytes)) {
+        // small: both straight to pinned memory, one wait
+        for (int which = 0; which < 2; ++which)
+            if (which == 0 ? pos3 : vel3)
+                bh::launch_to_caller(d, which, h->pinned + which * bytes);
+        if (!check(h, hipGetLastError(), "download") ||
+            !check(h, hipStreamSynchronize(d.stream), "download"))
+            return BH_HIP_INTERNAL_ERROR;
+        if (pos3)
+            std::memcpy(pos3, h->pinned, bytes);
+        if (vel3)
+            std::memcpy(vel3, h->pinned + bytes, bytes);
+        return BH_HIP_OK;
+    }
     for (int which = 0; which < 2; ++which) {
         double* dst = which == 0 ? pos3 : vel3;
         if (!dst)
@@ -1258,7 +1281,7 @@ bh_hip_result_t bh_hip_build_tree(bh_hip_handle_t* h)
 {
     if (!h)
         return BH_HIP_INVALID_ARGUMENT;
-    if (!usable(h) || !zero_err(h))
+    if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     begin_call(h);
     if (!build_checked(h, next_events(h))) {
@@ -1279,7 +1302,7 @@ bh_hip_result_t bh_hip_compute_accelerations(bh_hip_handle_t* h, float* acc3)
         h->last_error = "compute_accelerations: key_mode REFERENCE30 builds topology only";
         return BH_HIP_INVALID_ARGUMENT;
     }
-    if (!usable(h) || !zero_err(h))
+    if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     begin_call(h);
     if (!queue_force(h)) {
@@ -1288,12 +1311,18 @@ bh_hip_result_t bh_hip_compute_accelerations(bh_hip_handle_t* h, float* acc3)
         end_call(h);
         return BH_HIP_INTERNAL_ERROR;
     }
+    // the result on its way before the wait: small ones straight to pinned memory
+    const size_t bytes = 3 * h->d.n * sizeof(float);
+    const bool direct = acc3 && bytes <= kRingChunkMin && ensure_ring(h, bytes);
+    if (acc3)
+        bh::launch_to_caller(h->d, 2, direct ? h->pinned : nullptr);
     bh_hip_result_t r = finish(h, "compute_accelerations");
     end_call(h);
     if (r != BH_HIP_OK || !acc3)
         return r;
-    bh::launch_to_caller(h->d, 2);
-    if (!copy_out(h, acc3, h->d.stage, 3 * h->d.n * sizeof(float), "acc download"))
+    if (direct)
+        std::memcpy(acc3, h->pinned, bytes);
+    else if (!copy_out(h, acc3, h->d.stage, 3 * h->d.n * sizeof(float), "acc download"))
         return BH_HIP_INTERNAL_ERROR;
     return BH_HIP_OK;
 }
@@ -1306,7 +1335,7 @@ bh_hip_result_t bh_hip_step(bh_hip_handle_t* h, double dt, int32_t nsteps)
         h->last_error = "step: key_mode REFERENCE30 builds topology only";
         return BH_HIP_INVALID_ARGUMENT;
     }
-    if (!usable(h) || !zero_err(h))
+    if (!usable(h))
         return BH_HIP_INTERNAL_ERROR;
     if (h->p.adaptive_max_level > 0)
         return step_adaptive(h, dt, nsteps);

@@ -175,6 +175,17 @@ struct AdaptiveParams {
     double box;       // periodic cube side (0 = open): positions wrapped after updates
 };
 
+// What the host reads back of a call, in pinned memory that kernels write: one
+// wait for the stream, no copies. (Each small copy of device memory took the
+// host about 27 us, three of them at the end of a call.)
+struct HostReport {
+    int err_build;  // error word after the last build
+    int err;        // and at the end of the call
+    uint32_t due;   // block time steps: ticks to the next force evaluation
+    unsigned long long stats[8];
+    int info[2 * kLevels + 4];
+};
+
 // Device buffers of one solver instance. The particle store is kept in the
 // order of the last sort (Morton order); `id` maps a store slot to the
 // caller's particle index and `rank` maps back.
@@ -239,6 +250,8 @@ struct Device {
     RootGeom* geom = nullptr;
     int* err = nullptr;
     unsigned int* work_counter = nullptr;
+    bool tickets_zero = false;  // a build's last kernel has cleared work_counter
+    HostReport* report = nullptr;  // pinned
     int* stack = nullptr;  // per-resident-wave traversal stacks
     size_t stack_waves = 0;
     size_t stack_cap = 0;
@@ -383,7 +396,8 @@ void launch_wrap(Device& d, double box);
 // caller-ordered stage -> store (0 = pos, 1 = vel: FP64 triples; 2 = mass: FP32)
 void launch_from_caller(Device& d, int which);
 // store -> caller-ordered stage (0 = pos, 1 = vel: FP64 triples; 2 = acc: FP32 triples)
-void launch_to_caller(Device& d, int which);
+// (to: another buffer, pinned host memory included)
+void launch_to_caller(Device& d, int which, void* to = nullptr);
 void launch_init_ids(Device& d);
 // FP64 direct sum; ws_dev holds direct_fp64_words(n, nt) doubles, the result
 // (3 per target) first.
@@ -394,6 +408,12 @@ void launch_energy(Device& d, double* out_dev);
 void launch_potential(Device& d, const uint32_t* slots_dev, uint32_t ns, double eps,
                       double min_d2, double* out_dev);
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
+// start of a call: error word and counters cleared
+void launch_begin_call(Device& d, unsigned long long* stats);
+// end of a build: error word to the report, walk tickets cleared
+void launch_end_build(Device& d);
+// end of a call: error word, counters and level table to the report
+void launch_report(Device& d, const unsigned long long* stats);
 // k_pm.hip: plans and meshes for an N^3 mesh (host allocation); the force
 // pass adds the long-range acceleration to acc and applies the clamp.
 bool pm_setup(PmState& pm, int N, hipStream_t stream);
@@ -408,7 +428,8 @@ void launch_adaptive_drift(Device& d, const AdaptiveParams& a, double span);
 void launch_adaptive_next_due(Device& d, const AdaptiveParams& a, uint32_t t, uint32_t* out);
 // count (optional, device): += number of particles corrected
 void launch_adaptive_correct(Device& d, const AdaptiveParams& a, uint32_t tick,
-                             unsigned long long* count);
+                             unsigned long long* count, uint32_t* due);
+void launch_due_report(Device& d, uint32_t* due);
 void launch_gather_u32(Device& d, const uint32_t* src_by_slot, uint32_t* out_by_caller);
 
 }  // namespace bh

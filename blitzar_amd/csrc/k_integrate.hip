@@ -446,18 +446,20 @@ void launch_from_caller(Device& d, int which)
                                                                dst[2], d.n);
 }
 
-void launch_to_caller(Device& d, int which)
+void launch_to_caller(Device& d, int which, void* to)
 {
     if (d.n == 0)
         return;
+    if (!to)
+        to = d.stage;
     if (which == 2) {
         to_caller3_kernel<float><<<blocks_for(d.n), 256, 0, d.stream>>>(
-            reinterpret_cast<float*>(d.stage), d.id, d.acc[0], d.acc[1], d.acc[2], d.n);
+            static_cast<float*>(to), d.id, d.acc[0], d.acc[1], d.acc[2], d.n);
         return;
     }
     double** src = which == 0 ? d.pos : d.vel;
-    to_caller3_kernel<double><<<blocks_for(d.n), 256, 0, d.stream>>>(d.stage, d.id, src[0],
-                                                                     src[1], src[2], d.n);
+    to_caller3_kernel<double><<<blocks_for(d.n), 256, 0, d.stream>>>(
+        static_cast<double*>(to), d.id, src[0], src[1], src[2], d.n);
 }
 
 namespace {
@@ -608,6 +610,23 @@ __device__ inline void correct_one(
     level[i] = adaptive_level(nx[i], ny[i], nz[i], x, y, z, a);
 }
 
+// Ticks from t to the next multiple of the cadence 2^(L - level) (ticks count
+// from a multiple of 2^L).
+__device__ inline uint32_t ticks_to_due(uint32_t level, int L, uint32_t t)
+{
+    const uint32_t c = 1u << (static_cast<uint32_t>(L) - level);
+    return (t / c + 1u) * c - t;
+}
+
+// The next due tick to the report, and the word cleared for the next minimum.
+__global__ void due_report_kernel(uint32_t* due, HostReport* rep)
+{
+    if (threadIdx.x == 0) {
+        rep->due = *due;
+        *due = 0xffffffffu;
+    }
+}
+
 // Corrector for the particles active at `tick` (their new force is in acc).
 __global__ __launch_bounds__(256) void adaptive_correct_kernel(
     double* __restrict__ px, double* __restrict__ py, double* __restrict__ pz,
@@ -615,39 +634,49 @@ __global__ __launch_bounds__(256) void adaptive_correct_kernel(
     const float* __restrict__ nx, const float* __restrict__ ny, const float* __restrict__ nz,
     float* __restrict__ bx, float* __restrict__ by, float* __restrict__ bz,
     uint32_t* __restrict__ level, uint32_t* __restrict__ last, size_t n, AdaptiveParams a,
-    uint32_t tick, unsigned long long* __restrict__ count)
+    uint32_t tick, unsigned long long* __restrict__ count, uint32_t* __restrict__ due_out)
 {
     // Grid-stride over the particles; the count of corrected particles is
     // summed per block and added with one atomic per block (a single counter
-    // every wave updates would serialise them).
+    // every wave updates would serialise them). The pass also finds the next due
+    // tick from the levels it reads and sets (as adaptive_next_due_kernel does).
     __shared__ unsigned long long block_count[4];
+    __shared__ uint32_t block_due[4];
     unsigned long long ndue = 0;
+    uint32_t next = 0xffffffffu;
     for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
          i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const uint32_t lv = min(level[i], static_cast<uint32_t>(a.levels));
+        uint32_t lv = min(level[i], static_cast<uint32_t>(a.levels));
         const uint32_t cadence = 1u << (static_cast<uint32_t>(a.levels) - lv);
-        if ((tick & (cadence - 1u)) != 0u)
-            continue;
-        ++ndue;
-        correct_one(px, py, pz, vx, vy, vz, nx, ny, nz, bx, by, bz, level, last, i, a, tick);
-    }
-    if (count) {
-        for (int o = 32; o > 0; o >>= 1)
-            ndue += __shfl_xor(ndue, o, 64);
-        if ((threadIdx.x & 63) == 0)
-            block_count[threadIdx.x >> 6] = ndue;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const unsigned long long t =
-                block_count[0] + block_count[1] + block_count[2] + block_count[3];
-            if (t)
-                atomicAdd(count, t);
+        if ((tick & (cadence - 1u)) == 0u) {
+            ++ndue;
+            correct_one(px, py, pz, vx, vy, vz, nx, ny, nz, bx, by, bz, level, last, i, a, tick);
+            lv = min(level[i], static_cast<uint32_t>(a.levels));
         }
+        next = min(next, ticks_to_due(lv, a.levels, tick));
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        ndue += __shfl_xor(ndue, o, 64);
+        next = min(next, static_cast<uint32_t>(__shfl_xor(static_cast<int>(next), o, 64)));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        block_count[threadIdx.x >> 6] = ndue;
+        block_due[threadIdx.x >> 6] = next;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned long long t =
+            block_count[0] + block_count[1] + block_count[2] + block_count[3];
+        if (count && t)
+            atomicAdd(count, t);
+        next = min(min(block_due[0], block_due[1]), min(block_due[2], block_due[3]));
+        if (next != 0xffffffffu)
+            atomicMin(due_out, next);
     }
 }
 
-// Smallest tick after t at which some particle is due: min over particles of
-// (t / cadence + 1) * cadence (ticks count from a multiple of 2^L).
+// Ticks from t to the next tick at which some particle is due, the minimum over
+// the particles (first slice of a call; later slices get it from the correction).
 __global__ __launch_bounds__(256) void adaptive_next_due_kernel(const uint32_t* __restrict__ level,
                                                                 size_t n, int L, uint32_t t,
                                                                 uint32_t* __restrict__ out)
@@ -657,9 +686,7 @@ __global__ __launch_bounds__(256) void adaptive_next_due_kernel(const uint32_t* 
     uint32_t due = 0xffffffffu;
     for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
          i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const uint32_t lv = min(level[i], static_cast<uint32_t>(L));
-        const uint32_t c = 1u << (static_cast<uint32_t>(L) - lv);
-        due = min(due, (t / c + 1u) * c);
+        due = min(due, ticks_to_due(min(level[i], static_cast<uint32_t>(L)), L, t));
     }
     for (int o = 32; o > 0; o >>= 1)
         due = min(due, static_cast<uint32_t>(__shfl_xor(static_cast<int>(due), o, 64)));
@@ -715,14 +742,19 @@ void launch_adaptive_next_due(Device& d, const AdaptiveParams& a, uint32_t t, ui
 }
 
 void launch_adaptive_correct(Device& d, const AdaptiveParams& a, uint32_t tick,
-                             unsigned long long* count)
+                             unsigned long long* count, uint32_t* due)
 {
     d.aabb_parts = 0;
     if (d.n == 0)
         return;
     adaptive_correct_kernel<<<reduce_blocks(d.n), 256, 0, d.stream>>>(
         d.pos[0], d.pos[1], d.pos[2], d.vel[0], d.vel[1], d.vel[2], d.acc[0], d.acc[1], d.acc[2],
-        d.aacc[0], d.aacc[1], d.aacc[2], d.alevel, d.atick, d.n, a, tick, count);
+        d.aacc[0], d.aacc[1], d.aacc[2], d.alevel, d.atick, d.n, a, tick, count, due);
+}
+
+void launch_due_report(Device& d, uint32_t* due)
+{
+    due_report_kernel<<<1, 64, 0, d.stream>>>(due, d.report);
 }
 
 void launch_gather_u32(Device& d, const uint32_t* src_by_slot, uint32_t* out_by_caller)

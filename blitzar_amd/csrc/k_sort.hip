@@ -521,6 +521,34 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t v, size_t n)
         p[i] = v;
 }
 
+__global__ void begin_call_kernel(int* err, unsigned long long* stats)
+{
+    if (threadIdx.x == 0)
+        *err = 0;
+    if (threadIdx.x < 8)
+        stats[threadIdx.x] = 0ull;
+}
+
+__global__ __launch_bounds__(256) void end_build_kernel(const int* err, unsigned int* tickets,
+                                                        HostReport* rep)
+{
+    for (int i = threadIdx.x; i < kTicketWords; i += blockDim.x)
+        tickets[i] = 0u;
+    if (threadIdx.x == 0)
+        rep->err_build = *err;
+}
+
+__global__ void report_kernel(const int* err, const unsigned long long* stats, const int* info,
+                              HostReport* rep)
+{
+    if (threadIdx.x == 0)
+        rep->err = *err;
+    if (threadIdx.x < 8)
+        rep->stats[threadIdx.x] = stats[threadIdx.x];
+    if (threadIdx.x < 2 * kLevels + 4)
+        rep->info[threadIdx.x] = info[threadIdx.x];
+}
+
 }  // namespace
 
 size_t scan_block_sums_words(size_t max_n) { return scan_workspace_words(max_n); }
@@ -734,6 +762,22 @@ void launch_rank(Device& d)
     if (d.n == 0)
         return;
     rank_kernel<<<static_cast<unsigned>((d.n + 255) / 256), 256, 0, d.stream>>>(d.id, d.n, d.rank);
+}
+
+void launch_begin_call(Device& d, unsigned long long* stats)
+{
+    begin_call_kernel<<<1, 64, 0, d.stream>>>(d.err, stats);
+}
+
+void launch_end_build(Device& d)
+{
+    end_build_kernel<<<1, 256, 0, d.stream>>>(d.err, d.work_counter, d.report);
+    d.tickets_zero = true;
+}
+
+void launch_report(Device& d, const unsigned long long* stats)
+{
+    report_kernel<<<1, 64, 0, d.stream>>>(d.err, stats, d.level_info, d.report);
 }
 
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s)

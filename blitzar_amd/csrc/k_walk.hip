@@ -1089,12 +1089,21 @@ void launch_walk_t(Device& d, const WalkParams& p, unsigned long long* stats,
 
 }  // namespace
 
+namespace {
+void clear_tickets(Device& d)
+{
+    if (!d.tickets_zero)
+        launch_fill_u32(d.work_counter, 0u, kTicketWords, d.stream);
+    d.tickets_zero = false;  // the walk draws from them
+}
+}  // namespace
+
 void launch_walk_record(Device& d, const WalkParams& p, unsigned long long* stats,
                         const LffState& L, float band, int min_count)
 {
     if (d.n == 0)
         return;
-    launch_fill_u32(d.work_counter, 0u, kTicketWords, d.stream);
+    clear_tickets(d);
     if (p.criterion == 1)
         launch_walk_t<2, 1, false, true>(d, p, stats, &L, band, min_count);
     else if (p.criterion == 2)
@@ -1107,7 +1116,7 @@ void launch_walk(Device& d, const WalkParams& p, unsigned long long* stats)
 {
     if (d.n == 0)
         return;
-    launch_fill_u32(d.work_counter, 0u, kTicketWords, d.stream);
+    clear_tickets(d);
     const bool tpm = p.rs > 0.0f;
     if (p.far2 > 0.0f && !tpm && p.order >= 2) {
         // quadrupole walk with the group far-field expansion
