@@ -597,6 +597,21 @@ uint32_t group_max(const bh_hip_handle* h)
     return g;
 }
 
+void end_build(bh_hip_handle* h, StepEvents* ev)
+{
+    rec(ev ? ev->b1 : nullptr, h->d.stream);
+    bh::launch_end_build(h->d);
+    (void)hipEventRecord(h->built, h->d.stream);
+    h->rank_valid = false;
+    h->have_tree = true;
+}
+
+// Builds of up to this many particles stay on one stream: there the kernels are
+// too short to overlap, and each event between the streams costs about 4 us (a
+// step of 4,099 particles 205 on two streams, 191 us on one; of 131,072 721 / 706;
+// 262,144 1,108 / 1,097; 524,288 1,701 / 1,726; 1,048,576 3,258 / 3,309).
+constexpr size_t kOneStreamMax = 200000;
+
 // Queue one tree build for the current positions.
 void queue_build(bh_hip_handle* h, StepEvents* ev)
 {
@@ -613,6 +628,20 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
     }
     rec(ev ? ev->s1 : nullptr, d.stream);
     bh::launch_tie_fix(d);
+    if (d.n <= kOneStreamMax) {
+        bh::launch_tree_build(d, h->leaf_depth, h->p.bucket_capacity, d.stream);
+        rec(ev ? ev->t1 : nullptr, d.stream);
+        bh::launch_permute_all(d, d.stream);
+        rec(ev ? ev->p1 : nullptr, d.stream);
+        rec(ev ? ev->j1 : nullptr, d.stream);
+        if (h->p.key_mode == 0) {
+            d.group_cap = group_max(h);
+            bh::launch_groups(d, d.group_cap, d.stream);
+            bh::launch_tree_moments(d);
+        }
+        end_build(h, ev);
+        return;
+    }
     // The topology needs only the sorted keys: it runs on the side stream
     // while the main stream permutes the positions and masses. The rest of
     // the store (velocities, ids, |a|) and the walk groups follow the
@@ -630,16 +659,12 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
     (void)hipEventRecord(h->ev_groups, h->side);
     bh::launch_permute_store(d, d.stream);
     rec(ev ? ev->p1 : nullptr, d.stream);
-    h->rank_valid = false;
     (void)hipStreamWaitEvent(d.stream, h->ev_topo, 0);
     rec(ev ? ev->j1 : nullptr, d.stream);
     if (h->p.key_mode == 0)
         bh::launch_tree_moments(d);
     (void)hipStreamWaitEvent(d.stream, h->ev_groups, 0);
-    rec(ev ? ev->b1 : nullptr, d.stream);
-    bh::launch_end_build(d);
-    (void)hipEventRecord(h->built, d.stream);
-    h->have_tree = true;
+    end_build(h, ev);
 }
 
 // Moments of the current positions on the topology of the last build (block

@@ -349,6 +349,7 @@ void launch_tie_fix(Device& d);
 // then velocities, ids, |a| and the block time-step arrays, each on its stream
 void launch_permute_store(Device& d, hipStream_t s);
 void launch_permute_rest(Device& d, hipStream_t s);
+void launch_permute_all(Device& d, hipStream_t s);  // both in one launch
 void launch_rank(Device& d);  // rebuild rank from id
 // k_tree.hip
 void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s);

@@ -486,6 +486,32 @@ __global__ __launch_bounds__(256) void permute_rest_kernel(
         oam[s] = am[j];
 }
 
+// Both parts in one launch, where they run one after the other anyway.
+__global__ __launch_bounds__(256) void permute_all_kernel(
+    const uint32_t* __restrict__ src, size_t n, const double* __restrict__ px,
+    const double* __restrict__ py, const double* __restrict__ pz, const float* __restrict__ m,
+    const double* __restrict__ vx, const double* __restrict__ vy, const double* __restrict__ vz,
+    const uint32_t* __restrict__ id, const float* __restrict__ am, double* __restrict__ opx,
+    double* __restrict__ opy, double* __restrict__ opz, float* __restrict__ om,
+    double* __restrict__ ovx, double* __restrict__ ovy, double* __restrict__ ovz,
+    uint32_t* __restrict__ oid, float* __restrict__ oam)
+{
+    const size_t s = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (s >= n)
+        return;
+    const uint32_t j = src[s];
+    opx[s] = px[j];
+    opy[s] = py[j];
+    opz[s] = pz[j];
+    om[s] = m[j];
+    ovx[s] = vx[j];
+    ovy[s] = vy[j];
+    ovz[s] = vz[j];
+    oid[s] = id[j];
+    if (am)
+        oam[s] = am[j];
+}
+
 // The block time-step arrays follow the store through the same permutation.
 __global__ __launch_bounds__(256) void permute_adaptive_kernel(
     const uint32_t* __restrict__ src, size_t n, const float* __restrict__ ax,
@@ -720,6 +746,39 @@ void launch_tie_fix(Device& d)
                                                 d.vals, d.id, d.n);
 }
 
+namespace {
+
+void swap_positions(Device& d)
+{
+    for (int a = 0; a < 3; ++a)
+        std::swap(d.pos[a], d.pos_b[a]);
+    std::swap(d.mass, d.mass_b);
+}
+
+void swap_rest(Device& d)
+{
+    for (int a = 0; a < 3; ++a)
+        std::swap(d.vel[a], d.vel_b[a]);
+    std::swap(d.id, d.id_b);
+    if (d.amag_live)
+        std::swap(d.amag, d.amag_b);
+}
+
+void permute_adaptive(Device& d, unsigned blocks, hipStream_t st)
+{
+    if (!d.alevel)
+        return;
+    permute_adaptive_kernel<<<blocks, 256, 0, st>>>(
+        d.vals, d.n, d.aacc[0], d.aacc[1], d.aacc[2], d.alevel, d.atick, d.aacc_b[0], d.aacc_b[1],
+        d.aacc_b[2], d.alevel_b, d.atick_b);
+    for (int a = 0; a < 3; ++a)
+        std::swap(d.aacc[a], d.aacc_b[a]);
+    std::swap(d.alevel, d.alevel_b);
+    std::swap(d.atick, d.atick_b);
+}
+
+}  // namespace
+
 void launch_permute_store(Device& d, hipStream_t st)
 {
     if (d.n == 0)
@@ -728,9 +787,7 @@ void launch_permute_store(Device& d, hipStream_t st)
     permute_store_kernel<<<blocks, 256, 0, st>>>(d.vals, d.n, d.pos[0], d.pos[1], d.pos[2],
                                                  d.mass, d.pos_b[0], d.pos_b[1], d.pos_b[2],
                                                  d.mass_b);
-    for (int a = 0; a < 3; ++a)
-        std::swap(d.pos[a], d.pos_b[a]);
-    std::swap(d.mass, d.mass_b);
+    swap_positions(d);
 }
 
 void launch_permute_rest(Device& d, hipStream_t st)
@@ -741,20 +798,22 @@ void launch_permute_rest(Device& d, hipStream_t st)
     permute_rest_kernel<<<blocks, 256, 0, st>>>(
         d.vals, d.n, d.vel[0], d.vel[1], d.vel[2], d.id, d.amag_live ? d.amag : nullptr,
         d.vel_b[0], d.vel_b[1], d.vel_b[2], d.id_b, d.amag_b);
-    for (int a = 0; a < 3; ++a)
-        std::swap(d.vel[a], d.vel_b[a]);
-    std::swap(d.id, d.id_b);
-    if (d.amag_live)
-        std::swap(d.amag, d.amag_b);
-    if (d.alevel) {
-        permute_adaptive_kernel<<<blocks, 256, 0, st>>>(
-            d.vals, d.n, d.aacc[0], d.aacc[1], d.aacc[2], d.alevel, d.atick, d.aacc_b[0],
-            d.aacc_b[1], d.aacc_b[2], d.alevel_b, d.atick_b);
-        for (int a = 0; a < 3; ++a)
-            std::swap(d.aacc[a], d.aacc_b[a]);
-        std::swap(d.alevel, d.alevel_b);
-        std::swap(d.atick, d.atick_b);
-    }
+    swap_rest(d);
+    permute_adaptive(d, blocks, st);
+}
+
+void launch_permute_all(Device& d, hipStream_t st)
+{
+    if (d.n == 0)
+        return;
+    const unsigned blocks = static_cast<unsigned>((d.n + 255) / 256);
+    permute_all_kernel<<<blocks, 256, 0, st>>>(
+        d.vals, d.n, d.pos[0], d.pos[1], d.pos[2], d.mass, d.vel[0], d.vel[1], d.vel[2], d.id,
+        d.amag_live ? d.amag : nullptr, d.pos_b[0], d.pos_b[1], d.pos_b[2], d.mass_b, d.vel_b[0],
+        d.vel_b[1], d.vel_b[2], d.id_b, d.amag_b);
+    swap_positions(d);
+    swap_rest(d);
+    permute_adaptive(d, blocks, st);
 }
 
 void launch_rank(Device& d)
