@@ -1308,77 +1308,111 @@ __device__ inline void node_moments_coop(CoopLds<OCT>& S, uint32_t node, int lev
     wave_lds_fence();  // the next call writes S
 }
 
-// The nodes that the lanes of one wavefront hold (has; node, meta each) on one
-// level: a few by 8 lanes each, many by a lane each.
+// The nodes that the threads of one workgroup of W wavefronts hold (has; node,
+// meta each) on one level, gathered in LDS and handed out again: a few by 8 lanes
+// each, so that all wavefronts have some, many by a lane each. S.n is 0 before the
+// first call; turn alternates.
 constexpr int kCoopMax = 16;
 
-template <bool OCT>
-__device__ inline void wave_nodes(CoopLds<OCT>& S, bool has, uint32_t node, int level,
-                                  const NodeMeta& meta, const RootGeom* __restrict__ geom,
-                                  WalkNode* __restrict__ wn, float* __restrict__ ext,
-                                  float* __restrict__ noct, int refit, int* err)
+template <bool OCT, int W>
+struct LevelLds {
+    CoopLds<OCT> coop[W];
+    uint64_t prefix[64 * W];
+    uint32_t node[64 * W], nchild[64 * W], first[64 * W], count[64 * W];
+    uint32_t n[2];
+};
+
+template <bool OCT, int W>
+__device__ inline void level_nodes(LevelLds<OCT, W>& S, int& turn, bool has, uint32_t node,
+                                   int level, const NodeMeta& meta,
+                                   const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn,
+                                   float* __restrict__ ext, float* __restrict__ noct, int refit,
+                                   int* err)
 {
-    unsigned long long m = __ballot(has);
-    if (__popcll(m) > kCoopMax) {
-        if (has)
-            node_moments<OCT, false>(static_cast<int>(node), level, meta, geom, wn, ext, noct,
-                                     refit, err, [](uint32_t, const double*) { return float4{}; });
-        return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned long long m = __ballot(has);
+    uint32_t base = 0u;
+    if (lane == 0 && m)
+        base = atomicAdd(&S.n[turn], static_cast<uint32_t>(__popcll(m)));
+    base = __shfl(base, 0, 64);
+    if (has) {
+        const uint32_t at = base + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
+        S.node[at] = node;
+        S.prefix[at] = meta.prefix;
+        S.nchild[at] = meta.nchild;
+        S.first[at] = meta.first;
+        S.count[at] = meta.count;
     }
-    while (m) {
-        // group g of lanes takes the g-th holder's node
-        const int g = (threadIdx.x & 63) >> 3;
-        unsigned long long k = m;
-        for (int i = 0; i < g; ++i)
-            k &= k - 1ull;
-        const int src = k ? __builtin_ctzll(k) : 0;
-        NodeMeta t;
-        t.nchild = __shfl(meta.nchild, src, 64);
-        t.first = __shfl(meta.first, src, 64);
-        t.count = __shfl(meta.count, src, 64);
-        const uint32_t at = __shfl(node, src, 64);
-        node_moments_coop<OCT>(S, k ? at : kNoNode, level, t, geom, wn, ext, noct, refit);
-        for (int i = 0; i < 8 && m; ++i)
-            m &= m - 1ull;
+    __syncthreads();
+    const uint32_t total = S.n[turn];
+    turn ^= 1;
+    if (threadIdx.x == 0)
+        S.n[turn] = 0u;  // its last readers passed the barrier that ended their call
+    const auto held = [&](uint32_t k) {
+        return NodeMeta{S.prefix[k], S.nchild[k], S.first[k], S.count[k]};
+    };
+    if (total > kCoopMax * W) {
+        if (threadIdx.x < total)
+            node_moments<OCT, false>(static_cast<int>(S.node[threadIdx.x]), level,
+                                     held(threadIdx.x), geom, wn, ext, noct, refit, err,
+                                     [](uint32_t, const double*) { return float4{}; });
+    } else {
+        for (uint32_t r = 8u * static_cast<uint32_t>(w); r < total; r += 8u * W) {
+            const uint32_t k = r + static_cast<uint32_t>(lane >> 3);
+            const uint32_t q = k < total ? k : r;
+            node_moments_coop<OCT>(S.coop[w], k < total ? S.node[k] : kNoNode, level, held(q), geom,
+                                   wn, ext, noct, refit);
+        }
     }
+    __syncthreads();  // the next level reads these nodes
 }
 
 // Internal nodes, after the leaves, of a tree from the one-pass topology, whose
-// scanned counts say which nodes of each level start in a tile. One wavefront per
-// tile sums, level by level, the internal nodes that lie whole inside the tile,
-// and leaves in cross[L][tile] the one node of each level (if any) that starts in
-// it and ends past it; cross_moments_kernel takes those. Bound: latency (about
-// 1.5 us a level; 4-6 levels of a tile hold internal nodes). One launch per level
-// for all internal nodes, 21 launches, took 62 us at 4,099 particles, 88 at
-// 65,536 and 254 at 8,388,608; the tiles and what they leave take 41, 61 and 210.
-template <bool OCT>
-__global__ __launch_bounds__(64, 3) void tile_moments_kernel(
+// scanned counts say which nodes of each level start in a tile. One workgroup of W
+// wavefronts per unit of `per` tiles sums, level by level, the internal nodes that
+// lie whole inside the unit, and leaves in cross[L][unit] the one node of each
+// level (if any) that starts in it and ends past it; cross_moments_kernel takes
+// those. Bound: latency (about 1.5 us a level; 4-6 levels of a tile hold internal
+// nodes). One launch per level for all internal nodes, 21 launches, took 62 us at
+// 4,099 particles, 88 at 65,536 and 254 at 8,388,608; the tiles and what they leave
+// take 24, 45 and 151 (39, 58 and 175 with one wavefront a tile, each taking the
+// nodes of its own lanes).
+template <bool OCT, int W>
+__global__ __launch_bounds__(64 * W) void tile_moments_kernel(
     const uint64_t* __restrict__ nprefix, const uint32_t* __restrict__ nstart,
     const uint32_t* __restrict__ ncount, const uint32_t* __restrict__ nchild,
     const uint32_t* __restrict__ nfirst, const int* __restrict__ info,
     const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn, float* __restrict__ ext,
     float* __restrict__ noct, int refit, int* err, const uint32_t* __restrict__ tilecnt,
-    uint32_t ntiles, uint32_t* __restrict__ cross)
+    uint32_t ntiles, uint32_t per, uint32_t* __restrict__ cross)
 {
-    __shared__ CoopLds<OCT> S;
+    __shared__ LevelLds<OCT, W> S;
     __shared__ uint32_t lvFirst[kLevels], lvEnd[kLevels];  // the tile's nodes per level
-    const uint32_t tile = blockIdx.x;
-    const uint32_t lim = (tile + 1u) * kTopoTile;
+    __shared__ uint32_t lvSet;
+    const uint32_t unit = blockIdx.x, units = gridDim.x;
+    const uint32_t tile = unit * per, last = min(tile + per, ntiles);
+    const uint64_t lim = static_cast<uint64_t>(last) * kTopoTile;
     bool any = false;
+    int turn = 0;
+    if (threadIdx.x < 2)
+        S.n[threadIdx.x] = 0u;
     if (threadIdx.x < kLevels) {
         const int L = threadIdx.x;
         const uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
         const uint32_t c0 = col[tile];
         const uint32_t c1 =
-            tile + 1 < ntiles ? col[tile + 1] : tilecnt[static_cast<size_t>(kLevels) * ntiles + L];
+            last < ntiles ? col[last] : tilecnt[static_cast<size_t>(kLevels) * ntiles + L];
         const bool kept = info[kLevels + L] > 0;  // levels past the node capacity were dropped
         any = kept && c1 > c0 && L < kMaxLevel;
         lvFirst[L] = static_cast<uint32_t>(info[L]) + c0;
         lvEnd[L] = static_cast<uint32_t>(info[L]) + (kept ? c1 : c0);
-        cross[static_cast<size_t>(L) * ntiles + tile] = kNoNode;
+        cross[static_cast<size_t>(L) * units + unit] = kNoNode;
     }
-    uint32_t levels = static_cast<uint32_t>(__ballot(any));  // those with nodes
+    const uint32_t mine = static_cast<uint32_t>(__ballot(any));
+    if (threadIdx.x == 0)
+        lvSet = mine;
     __syncthreads();
+    uint32_t levels = lvSet;  // those with nodes
     NodeMeta meta, next = {};
     uint32_t start = 0u, nextStart = 0u;
     const auto fetch = [&](uint32_t node, uint32_t end, NodeMeta& m, uint32_t& s) {
@@ -1390,10 +1424,10 @@ __global__ __launch_bounds__(64, 3) void tile_moments_kernel(
     };
     const auto sum = [&](uint32_t node, int L) {
         const bool in = meta.nchild != 0u;  // (else a leaf, or no node)
-        const bool past = in && start + meta.count > lim;
+        const bool past = in && static_cast<uint64_t>(start) + meta.count > lim;
         if (past)  // at most one node of a level
-            cross[static_cast<size_t>(L) * ntiles + tile] = node;
-        wave_nodes<OCT>(S, in && !past, node, L, meta, geom, wn, ext, noct, refit, err);
+            cross[static_cast<size_t>(L) * units + unit] = node;
+        level_nodes<OCT, W>(S, turn, in && !past, node, L, meta, geom, wn, ext, noct, refit, err);
     };
     int L = levels ? 31 - __builtin_clz(levels) : -1;
     if (L >= 0)
@@ -1408,21 +1442,20 @@ __global__ __launch_bounds__(64, 3) void tile_moments_kernel(
         if (above >= 0)  // the next level's fields while this one is summed
             fetch(lvFirst[above] + threadIdx.x, lvEnd[above], next, nextStart);
         sum(node, L);
-        for (uint32_t at = lvFirst[L] + 64u; at < e; at += 64u) {  // the whole wavefront
-            node += 64u;
+        for (uint32_t at = lvFirst[L] + 64u * W; at < e; at += 64u * W) {  // all threads
+            node += 64u * W;
             fetch(node, e, meta, start);
             sum(node, L);
         }
-        __syncthreads();  // the next level reads these nodes
         L = above;
     }
 }
 
-// The nodes the tiles left: unit u of this pass is kCrossUnits consecutive units of
-// the pass before (of tiles, in the first), held by one workgroup. cross_in[L * nin
-// + i] is the node of level L that starts in input unit i and ends past it;
-// the workgroup computes those inside its own unit and passes on the one per
-// level that ends past it. The last pass has one unit, which holds everything.
+// The nodes the units left: unit u of this pass is kCrossUnits consecutive units of
+// the pass before, held by one workgroup. cross_in[L * nin + i] is the node of
+// level L that starts in input unit i and ends past it; the workgroup computes those
+// inside its own unit and passes on the one per level that ends past it. The last
+// pass has one unit, which holds everything.
 constexpr int kCrossUnits = 512;
 
 template <bool OCT>
@@ -1434,11 +1467,14 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
     int* err, const uint32_t* __restrict__ cross_in, uint32_t nin, uint64_t unit,
     uint32_t* __restrict__ cross_out, uint32_t nout)
 {
-    __shared__ CoopLds<OCT> S[kCrossUnits / 64];
+    __shared__ LevelLds<OCT, kCrossUnits / 64> S;
     __shared__ uint32_t sNode[kMaxLevel][kCrossUnits];
     __shared__ uint32_t sLevels;  // bit L: this unit holds input nodes of level L
     const uint32_t i = blockIdx.x * kCrossUnits + threadIdx.x;
     const uint64_t lim = (static_cast<uint64_t>(blockIdx.x) + 1) * unit;
+    int turn = 0;
+    if (threadIdx.x < 2)
+        S.n[threadIdx.x] = 0u;
     if (threadIdx.x == 0)
         sLevels = 0u;
     uint32_t has = 0u;
@@ -1479,9 +1515,8 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
                           static_cast<uint64_t>(start) + meta.count > lim;
         if (past)
             cross_out[static_cast<size_t>(L) * nout + blockIdx.x] = node;
-        wave_nodes<OCT>(S[threadIdx.x >> 6], node != kNoNode && !past, node, L, meta, geom, wn,
-                        ext, noct, refit, err);
-        __syncthreads();
+        level_nodes<OCT>(S, turn, node != kNoNode && !past, node, L, meta, geom, wn, ext, noct,
+                         refit, err);
         L = above;
     }
 }
@@ -1721,6 +1756,15 @@ void launch_groups(Device& d, uint32_t gmax, hipStream_t s)
 
 namespace {
 
+// How the tiles are taken (tile and cross kernels, us). Up to 8 tiles in one unit
+// by one workgroup, which leaves nothing straddling: at 2,000 particles 16.8
+// against 14.6 + 11.7 as tiles, 4,099 24.2 / 14.7 + 17.1, 8,192 32.0 / 13.9 + 20.7,
+// 16,384 46.2 / 14.0 + 22.9. Up to 512 tiles by four wavefronts each, where the
+// card has room: 65,536 15.6 against 18.6 with one, 300,001 17.2 / 23.0, 1,048,576
+// 21.7 / 20.6, 8,388,608 123.8 / 86.1.
+constexpr uint32_t kOneUnitTiles = 8;
+constexpr uint32_t kWideTiles = 512;
+
 template <bool OCT>
 void launch_moments_t(Device& d, int rf)
 {
@@ -1735,9 +1779,21 @@ void launch_moments_t(Device& d, int rf)
         uint32_t* in = d.cross;
         uint32_t nin = topo_tiles(d.n);
         uint64_t unit = kTopoTile;
-        tile_moments_kernel<OCT><<<nin, 64, 0, d.stream>>>(
-            d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.level_info, d.geom, d.wnode,
-            d.next, noct, rf, d.err, d.topo_cnt, nin, in);
+        const uint32_t ntiles = nin;
+        const auto tiles = [&](auto waves, uint32_t per) {
+            constexpr int W = decltype(waves)::value;
+            nin = (ntiles + per - 1) / per;
+            unit = static_cast<uint64_t>(per) * kTopoTile;
+            tile_moments_kernel<OCT, W><<<nin, 64 * W, 0, d.stream>>>(
+                d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.level_info, d.geom, d.wnode,
+                d.next, noct, rf, d.err, d.topo_cnt, ntiles, per, in);
+        };
+        if (ntiles <= kOneUnitTiles)
+            tiles(std::integral_constant<int, 4>{}, ntiles);
+        else if (ntiles <= kWideTiles)
+            tiles(std::integral_constant<int, 4>{}, 1);
+        else
+            tiles(std::integral_constant<int, 1>{}, 1);
         while (nin > 1) {
             uint32_t* out = in + static_cast<size_t>(kLevels) * nin;
             const uint32_t nout = (nin + kCrossUnits - 1) / kCrossUnits;

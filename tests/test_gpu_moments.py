@@ -57,3 +57,17 @@ def test_internal_moments_follow_from_the_children(n, bucket):
         s.upload(pos, vel, mass)
         s.build_tree()
         _check(s.dump_tree())
+
+
+@pytest.mark.parametrize("bucket", [1, 16, 64])
+@pytest.mark.parametrize("n", [2048, 8192, 8193, 40000])
+def test_moments_of_units_of_several_tiles_and_full_levels(n, bucket):
+    # up to 8 tiles one workgroup takes the whole tree; bucket 1 gives levels of
+    # more nodes than its lanes; the coincident particles one deep chain
+    pos, vel, _ = B.plummer(n, seed=n + 1)
+    pos[: n // 50] = pos[0]
+    mass = np.random.default_rng(n).uniform(0.5, 1.5, n).astype(np.float32)
+    with B.OctreeHip(n, bucket_capacity=bucket) as s:
+        s.upload(pos, vel, mass)
+        s.build_tree()
+        _check(s.dump_tree())
