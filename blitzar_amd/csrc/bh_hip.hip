@@ -262,11 +262,11 @@ bool alloc_nodes(bh_hip_handle* h, size_t cap)
            dalloc(h, &d.scan_tmp, scan_n, "scan tmp") &&
            dalloc(h, &d.bnd_tmp, 8 * scan_n, "child bounds") &&
            dalloc(h, &d.big_list, scan_n, "large-node list") &&
-           dalloc(h, &d.topo_cnt, bh::topo_count_words(d.n), "tile node counts") &&
+           dalloc(h, &d.topo_cnt, 2 * bh::topo_count_words(d.n), "tile node counts") &&
            dalloc_zero(h, &d.scan_blocks, bh::scan_block_sums_words(scan_n), "scan blocks",
                        d.stream) &&
            dalloc(h, &d.nparent, cap, "node parent") && dalloc(h, &d.gscan, cap, "group scan") &&
-           dalloc_zero(h, &d.gscan_blocks, bh::scan_block_sums_words(cap), "group scan blocks",
+           dalloc_zero(h, &d.gscan_blocks, bh::group_scan_words(cap), "group scan blocks",
                        d.stream) &&
            (!oct || dalloc(h, &d.noct, 10 * cap, "node third moments"));
 }
@@ -636,8 +636,7 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
         rec(ev ? ev->j1 : nullptr, d.stream);
         if (h->p.key_mode == 0) {
             d.group_cap = group_max(h);
-            bh::launch_groups(d, d.group_cap, d.stream);
-            bh::launch_tree_moments(d);
+            bh::launch_tree_moments(d, false, true);
         }
         end_build(h, ev);
         return;

@@ -125,7 +125,8 @@ enum DeviceError : int {
 
 // One-pass tree topology (k_tree.hip): tiles of kTopoTile sorted keys; it
 // handles buckets of up to kTopoHalo particles (wider ones build level by
-// level). Its per-tile, per-level node counts need topo_count_words(n) words.
+// level). Its per-tile, per-level node counts need topo_count_words(n) words, and
+// as many again once scanned.
 constexpr int kTopoTile = 1024;
 constexpr int kTopoHalo = 64;
 inline uint32_t topo_tiles(size_t n) { return static_cast<uint32_t>((n + kTopoTile - 1) / kTopoTile); }
@@ -242,6 +243,7 @@ struct Device {
     uint32_t* bnd_tmp = nullptr;   // per-level child bounds (8 per node) from count to emit
     uint32_t* big_list = nullptr;  // per-level indices of nodes searched by a whole wavefront
     uint32_t* topo_cnt = nullptr;  // one-pass topology: node counts per tile and level
+    uint32_t* topo_scan = nullptr; // and their exclusive scans, level by level
     bool topo_tiled = false;       // the last topology came from the one-pass build
     uint32_t* cross = nullptr;     // moments: nodes that straddle tiles (cross_words)
     uint32_t* scan_blocks = nullptr;
@@ -356,12 +358,14 @@ void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s);
 // Moments, leaf packing and the walk's node records of the current
 // positions. refit: the topology is that of an earlier build (positions have
 // moved since); each node's level in the walk record is lowered until its
-// cell covers the node's particles.
-void launch_tree_moments(Device& d, bool refit = false);
+// cell covers the node's particles. groups: also the walk groups of d.group_cap
+// (launch_groups), in the leaves' launch.
+void launch_tree_moments(Device& d, bool refit = false, bool groups = false);
 // Walk groups: a partition of the sorted particles into spatially compact
 // runs of at most gmax <= kGroupMax particles (consecutive small children of
 // one node packed together; see node_groups in k_tree.hip).
 void launch_groups(Device& d, uint32_t gmax, hipStream_t s);
+size_t group_scan_words(size_t node_cap);  // of d.gscan_blocks, zeroed once when allocated
 // k_walk.hip
 // stats (optional, device): [0] particle-particle, [1] particle-cell interactions,
 // [3] node-group far-field interactions, [4] far-field target evaluations

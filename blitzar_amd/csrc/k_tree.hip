@@ -524,13 +524,14 @@ __global__ __launch_bounds__(kTopoThreads) void topo_count_kernel(
 }
 
 // Exclusive scan of each level's tile counts (one block per level, 4 tiles per
-// thread, in place); the level totals go to tilecnt[kLevels * ntiles + L].
-__global__ __launch_bounds__(kScanBlock) void topo_scan_kernel(uint32_t* __restrict__ tilecnt,
-                                                               uint32_t ntiles)
+// thread); the level totals go to scanned[kLevels * ntiles + L].
+__global__ __launch_bounds__(kScanBlock) void topo_scan_kernel(
+    const uint32_t* __restrict__ tilecnt, uint32_t* __restrict__ scanned, uint32_t ntiles)
 {
     __shared__ uint32_t tmp[kScanWaves];
     const int L = blockIdx.x;
-    uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
+    const uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
+    uint32_t* out = scanned + static_cast<size_t>(L) * ntiles;
     uint32_t carry = 0;
     for (uint32_t b = 0; b < ntiles; b += 4 * kScanBlock) {
         const uint32_t t = b + 4 * threadIdx.x;
@@ -543,35 +544,42 @@ __global__ __launch_bounds__(kScanBlock) void topo_scan_kernel(uint32_t* __restr
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
             if (t + k < ntiles)
-                col[t + k] = ex;
+                out[t + k] = ex;
             ex += v[k];
         }
         carry += total;
     }
     if (threadIdx.x == 0)
-        tilecnt[static_cast<size_t>(kLevels) * ntiles + L] = carry;
+        scanned[static_cast<size_t>(kLevels) * ntiles + L] = carry;
 }
 
 // The nodes that start in one tile, in breadth-first place, level by level
 // (a thread's nodes of one level take consecutive slots, so neighbouring
 // lanes write neighbouring slots). The first level whose nodes would not fit
 // in node_cap is dropped with every deeper one (the nodes above it that
-// would split stay leaves; flagged). Block 0 also writes the level table.
+// would split stay leaves; flagged). Block 0 also writes the level table. SCAN: of
+// up to kSelfScanTiles tiles, every workgroup sums the counts before its own
+// itself, which saves the launch of a scan (4,099 particles 11.0 us against 10.2 +
+// 3.1, 262,144 12.6 / 11.6 + 4.0).
+constexpr uint32_t kSelfScanTiles = 256;
+
+template <bool SCAN>
 __global__ __launch_bounds__(kTopoThreads) void topo_emit_kernel(
     const unsigned long long* __restrict__ keys, uint32_t n, const uint32_t* __restrict__ pinfo,
-    const uint32_t* __restrict__ tilecnt, uint32_t ntiles, int node_cap,
+    const uint32_t* __restrict__ tilecnt, uint32_t* __restrict__ scanned, uint32_t ntiles,
+    int node_cap,
     uint64_t* __restrict__ nprefix, uint8_t* __restrict__ nlevel, uint32_t* __restrict__ nstart,
     uint32_t* __restrict__ ncount, uint32_t* __restrict__ nchild, uint32_t* __restrict__ nfirst,
     uint32_t* __restrict__ nparent, int* __restrict__ info, int* __restrict__ err)
 {
     __shared__ uint32_t cnt[kLevels][kTopoThreads];
     __shared__ uint32_t sbase[kLevels];  // level base + this tile's offset
+    __shared__ uint32_t tot[kLevels];    // nodes per level
     __shared__ int slmax;
     const int tid = threadIdx.x;
     const uint32_t tile = blockIdx.x;
     const uint32_t t0 = tile * kTopoTile;
     const uint32_t i0 = t0 + static_cast<uint32_t>(tid * kTopoPer);
-    const uint32_t* tot = tilecnt + static_cast<size_t>(kLevels) * ntiles;
     // the thread's level ranges and keys, loaded together
     uint32_t pk[kTopoPer];
     unsigned long long kq[kTopoPer];
@@ -600,6 +608,35 @@ __global__ __launch_bounds__(kTopoThreads) void topo_emit_kernel(
             kq[q] = in ? keys[i0 + q] & kKeyMask : 0ull;
         }
     }
+    if (SCAN) {
+#pragma unroll
+        for (int k = 0; k < (kLevels + kTopoThreads / 64 - 1) / (kTopoThreads / 64); ++k) {
+            const int L = (tid >> 6) + k * (kTopoThreads / 64);
+            uint32_t all = 0u, before = 0u;
+            if (L < kLevels) {
+                const uint32_t* col = tilecnt + static_cast<size_t>(L) * ntiles;
+#pragma unroll
+                for (uint32_t q = 0; q < kSelfScanTiles / 64; ++q) {
+                    const uint32_t t = q * 64 + static_cast<uint32_t>(tid & 63);
+                    const uint32_t v = t < ntiles ? col[t] : 0u;
+                    all += v;
+                    before += t < tile ? v : 0u;
+                }
+                all = wave_total(all);
+                before = wave_total(before);
+                if ((tid & 63) == 0) {
+                    tot[L] = all;
+                    sbase[L] = before;
+                    scanned[static_cast<size_t>(L) * ntiles + tile] = before;
+                    if (tile == 0)
+                        scanned[static_cast<size_t>(kLevels) * ntiles + L] = all;
+                }
+            }
+        }
+    } else if (tid < kLevels) {
+        tot[tid] = scanned[static_cast<size_t>(kLevels) * ntiles + tid];
+        sbase[tid] = scanned[static_cast<size_t>(tid) * ntiles + tile];
+    }
     if (tid == 0)
         slmax = kMaxLevel;
     __syncthreads();
@@ -614,7 +651,7 @@ __global__ __launch_bounds__(kTopoThreads) void topo_emit_kernel(
     const int lmax = slmax;
     if (tid < kLevels) {
         const uint32_t base = static_cast<uint32_t>(below);
-        sbase[tid] = base + (tid <= lmax ? tilecnt[static_cast<size_t>(tid) * ntiles + tile] : 0u);
+        sbase[tid] = base + (tid <= lmax ? sbase[tid] : 0u);
         if (tile == 0) {
             const bool kept = tid <= lmax;
             uint64_t kept_total = 0;
@@ -1091,17 +1128,164 @@ __device__ inline void node_moments(int node, int level, const NodeMeta& meta,
     }
 }
 
+// Walk groups. Node i owns groups when
+//   * i is the root and holds <= G particles: one group;
+//   * i holds > G particles and is a leaf: ceil(count / G) chunks;
+//   * i holds > G particles and has children: its children holding <= G
+//     particles, packed greedily in octant order into runs of consecutive
+//     children with <= G particles in total (a child holding > G ends a run).
+//     A run also ends before a child that would stretch the run's box (the
+//     smallest box of octants covering it) over a sibling holding > G
+//     particles: octants 3 and 4, for instance, span the whole cell, and a
+//     group whose targets surround a dense sibling would open all of it.
+// Every particle lands in exactly one group; a group's particles are
+// contiguous in sorted order and lie inside node i's cell, whose lattice
+// centre is the group's reference point. G = gmax (at most kGroupMax, one
+// target per lane of the walk's wavefront).
+__device__ inline bool octant_box_holds(uint32_t ax, uint32_t ay, uint32_t az, uint32_t o)
+{
+    // ax/ay/az: bit v set when the box covers value v of that axis' octant bit
+    return ((ax >> ((o >> 2) & 1u)) & (ay >> ((o >> 1) & 1u)) & (az >> (o & 1u)) & 1u) != 0u;
+}
+
+template <bool EMIT>
+__device__ inline uint32_t node_groups(int i, const uint64_t* __restrict__ nprefix,
+                                       const uint32_t* __restrict__ nstart,
+                                       const uint32_t* __restrict__ ncount,
+                                       const uint32_t* __restrict__ nchild,
+                                       const uint32_t* __restrict__ nfirst,
+                                       const uint32_t* __restrict__ nparent, uint32_t base,
+                                       uint4* __restrict__ groups, uint32_t gmax)
+{
+    const uint32_t c = ncount[i];
+    if (c <= gmax) {
+        if (nparent[i] != 0xffffffffu)
+            return 0;
+        if (EMIT)
+            groups[base] = make_uint4(nstart[i], c, static_cast<uint32_t>(i), 0u);
+        return 1;
+    }
+    const uint32_t nc = nchild[i];
+    if (nc == 0) {
+        const uint32_t k = (c + gmax - 1) / gmax;
+        if (EMIT)
+            for (uint32_t j = 0; j < k; ++j) {
+                const uint32_t off = j * gmax;
+                const uint32_t cnt = c - off < gmax ? c - off : gmax;
+                groups[base + j] = make_uint4(nstart[i] + off, cnt, static_cast<uint32_t>(i), 0u);
+            }
+        return k;
+    }
+    const uint32_t f = nfirst[i];
+    uint32_t dense = 0;  // octants of the children holding > G particles
+    for (uint32_t j = f; j < f + nc; ++j)
+        if (ncount[j] > gmax)
+            dense |= 1u << static_cast<uint32_t>(nprefix[j] & 7u);
+    uint32_t ng = 0, run_start = 0, run_count = 0;
+    uint32_t bx = 0, by = 0, bz = 0;  // the run's octant box
+    for (uint32_t j = f; j < f + nc; ++j) {
+        const uint32_t cc = ncount[j];
+        const bool small = cc <= gmax;
+        const uint32_t o = static_cast<uint32_t>(nprefix[j] & 7u);
+        const uint32_t nx = bx | (1u << ((o >> 2) & 1u)), ny = by | (1u << ((o >> 1) & 1u)),
+                       nz = bz | (1u << (o & 1u));
+        bool covers_dense = false;
+        for (uint32_t q = 0; q < 8; ++q)
+            covers_dense = covers_dense || (((dense >> q) & 1u) && octant_box_holds(nx, ny, nz, q));
+        if (run_count > 0 && (!small || run_count + cc > gmax || covers_dense)) {
+            if (EMIT)
+                groups[base + ng] = make_uint4(run_start, run_count, static_cast<uint32_t>(i), 0u);
+            ++ng;
+            run_count = 0;
+            bx = by = bz = 0;
+        }
+        if (small) {
+            if (run_count == 0)
+                run_start = nstart[j];
+            run_count += cc;
+            bx |= 1u << ((o >> 2) & 1u);
+            by |= 1u << ((o >> 1) & 1u);
+            bz |= 1u << (o & 1u);
+        }
+    }
+    if (run_count > 0) {
+        if (EMIT)
+            groups[base + ng] = make_uint4(run_start, run_count, static_cast<uint32_t>(i), 0u);
+        ++ng;
+    }
+    return ng;
+}
+
+// Counting, scan and emission in one launch, a thread per node, 256 nodes a
+// workgroup: the groups before a workgroup's come by look-back (the workspace is
+// scan_lookback.h's, one status word per workgroup).
+constexpr int kGroupBlock = 256;
+
+struct GroupArgs {
+    const uint32_t* nparent;
+    uint32_t* ws;
+    uint4* groups;
+    int* info;
+    int* err;
+    uint32_t gmax, blocks;
+};
+
+__device__ inline void groups_block(const GroupArgs& a, uint32_t b,
+                                    const uint64_t* __restrict__ nprefix,
+                                    const uint32_t* __restrict__ nstart,
+                                    const uint32_t* __restrict__ ncount,
+                                    const uint32_t* __restrict__ nchild,
+                                    const uint32_t* __restrict__ nfirst)
+{
+    __shared__ uint32_t red[kScanWaves];
+    __shared__ uint32_t s_epoch, s_excl;
+    const int total = a.info[kInfoTotal];
+    const uint32_t nblocks = static_cast<uint32_t>((total + kGroupBlock - 1) / kGroupBlock);
+    if (b >= nblocks)
+        return;
+    if (threadIdx.x == 0)
+        s_epoch = __hip_atomic_load(&a.ws[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int i = static_cast<int>(b * kGroupBlock + threadIdx.x);
+    const uint32_t ng =
+        i < total ? node_groups<false>(i, nprefix, nstart, ncount, nchild, nfirst, a.nparent, 0u,
+                                       nullptr, a.gmax)
+                  : 0u;
+    uint32_t agg;
+    const uint32_t off = block_exclusive256(ng, red, &agg);  // its barriers also publish s_epoch
+    if (threadIdx.x < 64) {
+        const uint32_t epoch = s_epoch;
+        const uint32_t excl = scan_lookback_prefix(
+            b, agg, epoch, reinterpret_cast<unsigned long long*>(a.ws + kScanHeaderWords), a.err,
+            kErrScan);
+        if (threadIdx.x == 0) {
+            s_excl = excl;
+            if (b == nblocks - 1) {
+                a.info[kInfoGroups] = static_cast<int>(excl + agg);
+                __hip_atomic_store(&a.ws[0], epoch + 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    __syncthreads();
+    if (ng > 0u)
+        node_groups<true>(i, nprefix, nstart, ncount, nchild, nfirst, a.nparent, s_excl + off,
+                          a.groups, a.gmax);
+}
+
 // Leaves of every level. Particles in chunks of kLeafChunk (kLeafPer per
 // thread, coalesced): each stores its offset from its leaf's lattice centre
 // (spart) and keeps it in LDS. The chunk's leaf starts are then listed and
 // summed by consecutive threads (full wavefronts, not one lane in six),
 // reading the chunk's offsets from LDS and recomputing those past the chunk
-// (the same arithmetic, so the same bits). sleaf must be set.
+// (the same arithmetic, so the same bits). sleaf must be set. GROUPS: the first
+// ga.blocks workgroups make the walk groups, which need the topology too and
+// nothing of the leaves (4,099 particles 12.4 us against 16.1 for the groups in three
+// launches and 11.9, 65,536 17.3 / 19.8 + 14.0, 200,000 20.0 / 20.6 + 14.7).
 constexpr int kLeafThreads = 256;
 constexpr int kLeafPer = 4;
 constexpr int kLeafChunk = kLeafThreads * kLeafPer;
 
-template <bool OCT>
+template <bool OCT, bool GROUPS>
 __global__ __launch_bounds__(kLeafThreads) void leaf_moments_kernel(
     const uint64_t* __restrict__ nprefix, const uint8_t* __restrict__ nlevel,
     const uint32_t* __restrict__ nstart, const uint32_t* __restrict__ ncount,
@@ -1110,12 +1294,16 @@ __global__ __launch_bounds__(kLeafThreads) void leaf_moments_kernel(
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
     const float* __restrict__ pm, const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn,
     float4* __restrict__ spart, float* __restrict__ ext, float* __restrict__ noct, int refit,
-    int* err)
+    int* err, GroupArgs ga)
 {
     __shared__ float4 sp[kLeafChunk];
     __shared__ uint32_t starts[kLeafChunk];  // chunk-relative first particle of each leaf
     __shared__ uint32_t nstarts;
-    const uint32_t b0 = blockIdx.x * kLeafChunk;
+    if (GROUPS && blockIdx.x < ga.blocks) {
+        groups_block(ga, blockIdx.x, nprefix, nstart, ncount, nchild, nfirst);
+        return;
+    }
+    const uint32_t b0 = (blockIdx.x - (GROUPS ? ga.blocks : 0u)) * kLeafChunk;
     const uint32_t total = static_cast<uint32_t>(info[kInfoTotal]);
     if (threadIdx.x == 0)
         nstarts = 0u;
@@ -1563,94 +1751,6 @@ __global__ __launch_bounds__(256) void tree_moments_kernel(
 }
 
 
-// Walk groups. Node i owns groups when
-//   * i is the root and holds <= G particles: one group;
-//   * i holds > G particles and is a leaf: ceil(count / G) chunks;
-//   * i holds > G particles and has children: its children holding <= G
-//     particles, packed greedily in octant order into runs of consecutive
-//     children with <= G particles in total (a child holding > G ends a run).
-//     A run also ends before a child that would stretch the run's box (the
-//     smallest box of octants covering it) over a sibling holding > G
-//     particles: octants 3 and 4, for instance, span the whole cell, and a
-//     group whose targets surround a dense sibling would open all of it.
-// Every particle lands in exactly one group; a group's particles are
-// contiguous in sorted order and lie inside node i's cell, whose lattice
-// centre is the group's reference point. G = gmax (at most kGroupMax, one
-// target per lane of the walk's wavefront).
-__device__ inline bool octant_box_holds(uint32_t ax, uint32_t ay, uint32_t az, uint32_t o)
-{
-    // ax/ay/az: bit v set when the box covers value v of that axis' octant bit
-    return ((ax >> ((o >> 2) & 1u)) & (ay >> ((o >> 1) & 1u)) & (az >> (o & 1u)) & 1u) != 0u;
-}
-
-template <bool EMIT>
-__device__ inline uint32_t node_groups(int i, const uint64_t* __restrict__ nprefix,
-                                       const uint32_t* __restrict__ nstart,
-                                       const uint32_t* __restrict__ ncount,
-                                       const uint32_t* __restrict__ nchild,
-                                       const uint32_t* __restrict__ nfirst,
-                                       const uint32_t* __restrict__ nparent, uint32_t base,
-                                       uint4* __restrict__ groups, uint32_t gmax)
-{
-    const uint32_t c = ncount[i];
-    if (c <= gmax) {
-        if (nparent[i] != 0xffffffffu)
-            return 0;
-        if (EMIT)
-            groups[base] = make_uint4(nstart[i], c, static_cast<uint32_t>(i), 0u);
-        return 1;
-    }
-    const uint32_t nc = nchild[i];
-    if (nc == 0) {
-        const uint32_t k = (c + gmax - 1) / gmax;
-        if (EMIT)
-            for (uint32_t j = 0; j < k; ++j) {
-                const uint32_t off = j * gmax;
-                const uint32_t cnt = c - off < gmax ? c - off : gmax;
-                groups[base + j] = make_uint4(nstart[i] + off, cnt, static_cast<uint32_t>(i), 0u);
-            }
-        return k;
-    }
-    const uint32_t f = nfirst[i];
-    uint32_t dense = 0;  // octants of the children holding > G particles
-    for (uint32_t j = f; j < f + nc; ++j)
-        if (ncount[j] > gmax)
-            dense |= 1u << static_cast<uint32_t>(nprefix[j] & 7u);
-    uint32_t ng = 0, run_start = 0, run_count = 0;
-    uint32_t bx = 0, by = 0, bz = 0;  // the run's octant box
-    for (uint32_t j = f; j < f + nc; ++j) {
-        const uint32_t cc = ncount[j];
-        const bool small = cc <= gmax;
-        const uint32_t o = static_cast<uint32_t>(nprefix[j] & 7u);
-        const uint32_t nx = bx | (1u << ((o >> 2) & 1u)), ny = by | (1u << ((o >> 1) & 1u)),
-                       nz = bz | (1u << (o & 1u));
-        bool covers_dense = false;
-        for (uint32_t q = 0; q < 8; ++q)
-            covers_dense = covers_dense || (((dense >> q) & 1u) && octant_box_holds(nx, ny, nz, q));
-        if (run_count > 0 && (!small || run_count + cc > gmax || covers_dense)) {
-            if (EMIT)
-                groups[base + ng] = make_uint4(run_start, run_count, static_cast<uint32_t>(i), 0u);
-            ++ng;
-            run_count = 0;
-            bx = by = bz = 0;
-        }
-        if (small) {
-            if (run_count == 0)
-                run_start = nstart[j];
-            run_count += cc;
-            bx |= 1u << ((o >> 2) & 1u);
-            by |= 1u << ((o >> 1) & 1u);
-            bz |= 1u << (o & 1u);
-        }
-    }
-    if (run_count > 0) {
-        if (EMIT)
-            groups[base + ng] = make_uint4(run_start, run_count, static_cast<uint32_t>(i), 0u);
-        ++ng;
-    }
-    return ng;
-}
-
 __global__ __launch_bounds__(256) void group_count_kernel(
     const uint64_t* __restrict__ nprefix, const uint32_t* __restrict__ nstart,
     const uint32_t* __restrict__ ncount, const uint32_t* __restrict__ nchild,
@@ -1706,10 +1806,14 @@ void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s)
         else
             topo_count_kernel<0><<<ntiles, kTopoThreads, 0, s>>>(
                 sorted, n, bucket, leaf_depth, pinfo, d.topo_cnt, ntiles);
-        topo_scan_kernel<<<kLevels, kScanBlock, 0, s>>>(d.topo_cnt, ntiles);
-        topo_emit_kernel<<<ntiles, kTopoThreads, 0, s>>>(
-            sorted, n, pinfo, d.topo_cnt, ntiles, static_cast<int>(d.node_cap), d.nprefix,
-            d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.nparent, d.level_info, d.err);
+        d.topo_scan = d.topo_cnt + topo_count_words(d.n);
+        const auto emit = ntiles <= kSelfScanTiles ? topo_emit_kernel<true> : topo_emit_kernel<false>;
+        if (ntiles > kSelfScanTiles)
+            topo_scan_kernel<<<kLevels, kScanBlock, 0, s>>>(d.topo_cnt, d.topo_scan, ntiles);
+        emit<<<ntiles, kTopoThreads, 0, s>>>(
+            sorted, n, pinfo, d.topo_cnt, d.topo_scan, ntiles, static_cast<int>(d.node_cap),
+            d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.nparent, d.level_info,
+            d.err);
         topo_link_kernel<<<level_grid(std::min<size_t>(d.node_cap, 2 * d.n + 64)), 256, 0,
                            s>>>(sorted, n, d.nprefix, d.nlevel, d.nstart, d.ncount,
                                        d.nchild, d.nfirst, d.nparent, d.sleaf, d.level_info,
@@ -1743,6 +1847,8 @@ void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s)
                        s>>>(d.nstart, d.ncount, d.nchild, d.level_info, n, d.sleaf);
 }
 
+size_t group_scan_words(size_t node_cap) { return scan_workspace_words(node_cap, kGroupBlock); }
+
 void launch_groups(Device& d, uint32_t gmax, hipStream_t s)
 {
     const unsigned g = level_grid(d.node_cap);
@@ -1766,15 +1872,19 @@ constexpr uint32_t kOneUnitTiles = 8;
 constexpr uint32_t kWideTiles = 512;
 
 template <bool OCT>
-void launch_moments_t(Device& d, int rf)
+void launch_moments_t(Device& d, int rf, bool groups)
 {
     const uint32_t n = static_cast<uint32_t>(d.n);
     float* noct = OCT ? d.noct : nullptr;
-    leaf_moments_kernel<OCT>
-        <<<(n + kLeafChunk - 1) / kLeafChunk, kLeafThreads, 0, d.stream>>>(
-            d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.sleaf, n, d.level_info,
-            d.pos[0], d.pos[1], d.pos[2], d.mass, d.geom, d.wnode, d.spart, d.next, noct, rf,
-            d.err);
+    GroupArgs ga{};
+    if (groups)
+        ga = GroupArgs{d.nparent, d.gscan_blocks, d.groups, d.level_info, d.err, d.group_cap,
+                       static_cast<uint32_t>((d.node_cap + kGroupBlock - 1) / kGroupBlock)};
+    const auto leaves = groups ? leaf_moments_kernel<OCT, true> : leaf_moments_kernel<OCT, false>;
+    leaves<<<ga.blocks + (n + kLeafChunk - 1) / kLeafChunk, kLeafThreads, 0, d.stream>>>(
+        d.nprefix, d.nlevel, d.nstart, d.ncount, d.nchild, d.nfirst, d.sleaf, n, d.level_info,
+        d.pos[0], d.pos[1], d.pos[2], d.mass, d.geom, d.wnode, d.spart, d.next, noct, rf, d.err,
+        ga);
     if (d.topo_tiled) {
         uint32_t* in = d.cross;
         uint32_t nin = topo_tiles(d.n);
@@ -1786,7 +1896,7 @@ void launch_moments_t(Device& d, int rf)
             unit = static_cast<uint64_t>(per) * kTopoTile;
             tile_moments_kernel<OCT, W><<<nin, 64 * W, 0, d.stream>>>(
                 d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.level_info, d.geom, d.wnode,
-                d.next, noct, rf, d.err, d.topo_cnt, ntiles, per, in);
+                d.next, noct, rf, d.err, d.topo_scan, ntiles, per, in);
         };
         if (ntiles <= kOneUnitTiles)
             tiles(std::integral_constant<int, 4>{}, ntiles);
@@ -1815,14 +1925,14 @@ void launch_moments_t(Device& d, int rf)
 
 }  // namespace
 
-void launch_tree_moments(Device& d, bool refit)
+void launch_tree_moments(Device& d, bool refit, bool groups)
 {
     if (d.n == 0)
         return;
     if (d.noct)
-        launch_moments_t<true>(d, refit ? 1 : 0);
+        launch_moments_t<true>(d, refit ? 1 : 0, groups);
     else
-        launch_moments_t<false>(d, refit ? 1 : 0);
+        launch_moments_t<false>(d, refit ? 1 : 0, groups);
 }
 
 }  // namespace bh

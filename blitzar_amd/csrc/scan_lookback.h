@@ -39,9 +39,9 @@ constexpr int kScanHeaderWords = 64;
 // error and stops waiting (results of that scan are then wrong, not hung).
 constexpr uint32_t kScanMaxPolls = 1u << 22;
 
-inline size_t scan_workspace_words(size_t capacity)
+inline size_t scan_workspace_words(size_t capacity, size_t chunk = kScanChunk)
 {
-    const size_t nb = (capacity + kScanChunk - 1) / kScanChunk + 1;
+    const size_t nb = (capacity + chunk - 1) / chunk + 1;
     return kScanHeaderWords + 2 * nb;
 }
 
@@ -85,6 +85,60 @@ __device__ inline unsigned long long scan_status(uint32_t epoch, uint32_t flag, 
            (static_cast<unsigned long long>(flag) << 32) | value;
 }
 
+// Block b's exclusive prefix, from its own sum and the blocks before it (one
+// wavefront, every lane; status words of the launch's epoch). Publishes both.
+__device__ inline uint32_t scan_lookback_prefix(uint32_t b, uint32_t agg, uint32_t epoch,
+                                                unsigned long long* status, int* err, int err_bit)
+{
+    const int lane = threadIdx.x & 63;
+    uint32_t excl = 0;
+    if (b == 0) {
+        if (lane == 0)
+            __hip_atomic_store(&status[0], scan_status(epoch, 2u, agg), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        return excl;
+    }
+    if (lane == 0)
+        __hip_atomic_store(&status[b], scan_status(epoch, 1u, agg), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    long long p = static_cast<long long>(b) - 1;  // nearest predecessor in this step
+    uint32_t polls = 0;
+    for (;;) {
+        const long long idx = p - lane;
+        uint32_t flag = 2u, val = 0u;  // before block 0: an inclusive zero
+        if (idx >= 0) {
+            const unsigned long long st = __hip_atomic_load(&status[idx], __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT);
+            const bool cur = static_cast<uint32_t>(st >> 34) == (epoch & 0x3fffffffu);
+            flag = cur ? static_cast<uint32_t>(st >> 32) & 3u : 0u;
+            val = static_cast<uint32_t>(st);
+        }
+        const unsigned long long incl = __ballot(flag == 2u);
+        const unsigned long long empty = __ballot(flag == 0u);
+        const int first = incl ? __builtin_ctzll(incl) : 64;
+        const unsigned long long need = first >= 63 ? ~0ull : ((2ull << first) - 1ull);
+        if (empty & need) {
+            if (++polls > kScanMaxPolls) {
+                if (lane == 0)
+                    atomicOr(err, err_bit);
+                break;
+            }
+            continue;
+        }
+        uint32_t part = lane <= first ? val : 0u;
+        for (int o = 32; o > 0; o >>= 1)
+            part += __shfl_xor(part, o, 64);
+        excl += part;
+        if (first < 64)
+            break;
+        p -= 64;
+    }
+    if (lane == 0)
+        __hip_atomic_store(&status[b], scan_status(epoch, 2u, excl + agg), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    return excl;
+}
+
 struct ScanBlockResult {
     bool last;       // this block holds the scan's last word (or, when n == 0, block 0)
     uint32_t total;  // sum of all n words (valid in the last block)
@@ -125,53 +179,8 @@ __device__ inline ScanBlockResult scan_lookback_block(uint32_t* __restrict__ dat
     const uint32_t epoch = s_epoch;
 
     if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        uint32_t excl = 0;
-        if (b == 0) {
-            if (lane == 0)
-                __hip_atomic_store(&status[0], scan_status(epoch, 2u, agg), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            if (lane == 0)
-                __hip_atomic_store(&status[b], scan_status(epoch, 1u, agg), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            long long p = static_cast<long long>(b) - 1;  // nearest predecessor in this step
-            uint32_t polls = 0;
-            for (;;) {
-                const long long idx = p - lane;
-                uint32_t flag = 2u, val = 0u;  // before block 0: an inclusive zero
-                if (idx >= 0) {
-                    const unsigned long long st = __hip_atomic_load(
-                        &status[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    const bool cur = static_cast<uint32_t>(st >> 34) == (epoch & 0x3fffffffu);
-                    flag = cur ? static_cast<uint32_t>(st >> 32) & 3u : 0u;
-                    val = static_cast<uint32_t>(st);
-                }
-                const unsigned long long incl = __ballot(flag == 2u);
-                const unsigned long long empty = __ballot(flag == 0u);
-                const int first = incl ? __builtin_ctzll(incl) : 64;
-                const unsigned long long need = first >= 63 ? ~0ull : ((2ull << first) - 1ull);
-                if (empty & need) {
-                    if (++polls > kScanMaxPolls) {
-                        if (lane == 0)
-                            atomicOr(err, err_bit);
-                        break;
-                    }
-                    continue;
-                }
-                uint32_t part = lane <= first ? val : 0u;
-                for (int o = 32; o > 0; o >>= 1)
-                    part += __shfl_xor(part, o, 64);
-                excl += part;
-                if (first < 64)
-                    break;
-                p -= 64;
-            }
-            if (lane == 0)
-                __hip_atomic_store(&status[b], scan_status(epoch, 2u, excl + agg),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane == 0) {
+        const uint32_t excl = scan_lookback_prefix(b, agg, epoch, status, err, err_bit);
+        if (threadIdx.x == 0) {
             s_excl = excl;
             if (b == nblocks - 1)
                 __hip_atomic_store(&ws[0], epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
