@@ -21,42 +21,134 @@
 // (TpmCosmology.inl:52); this is the split form of the same mesh.
 #include "bh_internal.h"
 
+#include <climits>
+
 namespace bh {
 namespace {
 
-__device__ inline void cic_split(double x, double cells_per_len, int N, int& i0, float& f)
+__device__ inline void cic_cell(double x, double cells_per_len, int& i, float& f)
 {
     const double u = x * cells_per_len - 0.5;
     const double fl = floor(u);
     f = static_cast<float>(u - fl);
-    int i = static_cast<int>(fl) % N;
-    i0 = i < 0 ? i + N : i;
+    i = static_cast<int>(fl);
 }
 
-__global__ __launch_bounds__(256) void pm_deposit_kernel(
+__device__ inline int wrap_cell(int i, int N)
+{
+    i %= N;
+    return i < 0 ? i + N : i;
+}
+
+__device__ inline void cic_split(double x, double cells_per_len, int N, int& i0, float& f)
+{
+    cic_cell(x, cells_per_len, i0, f);
+    i0 = wrap_cell(i0, N);
+}
+
+// Cloud-in-cell deposit. The particles are in Morton order, so kDepositChunk
+// consecutive ones cover a compact block of cells: a workgroup sums them in an LDS
+// window over the cells they touch and adds the window's nonzero cells to the mesh.
+// Chunks whose window exceeds the LDS (they straddle a jump of the curve, or their
+// cells hold less than a particle) add to the mesh directly. Bound: the rate of
+// atomics at the L2 (8 per particle directly, about 2 through the window).
+// 128^3 particles and cells: @DEPOSIT@.
+constexpr int kDepositThreads = 512;
+constexpr int kDepositChunk = 2 * kDepositThreads;
+constexpr int kDepositCells = 9984;  // 39 KB: four workgroups per CU; holds 17 x 17 x 33
+
+__global__ __launch_bounds__(kDepositThreads) void pm_deposit_kernel(
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
     const float* __restrict__ m, size_t n, int N, double cells_per_len, float inv_cell_vol,
     float* __restrict__ rho)
 {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    int ix, iy, iz;
-    float fx, fy, fz;
-    cic_split(px[i], cells_per_len, N, ix, fx);
-    cic_split(py[i], cells_per_len, N, iy, fy);
-    cic_split(pz[i], cells_per_len, N, iz, fz);
-    const float w = m[i] * inv_cell_vol;
-    const int jx = ix + 1 == N ? 0 : ix + 1, jy = iy + 1 == N ? 0 : iy + 1,
-              jz = iz + 1 == N ? 0 : iz + 1;
+    __shared__ float win[kDepositCells];
+    __shared__ int lim[kDepositThreads / 64][6];
+    constexpr int kPer = kDepositChunk / kDepositThreads;
+    int cell[kPer][3];  // not yet wrapped into the box
+    float frac[kPer][3], w[kPer];
+    // (minima of cell and of -cell: the chunk's first and last cells per axis)
+    int lo[6] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const size_t i = static_cast<size_t>(blockIdx.x) * kDepositChunk +
+                         static_cast<size_t>(k * kDepositThreads) + threadIdx.x;
+        w[k] = 0.0f;
+        if (i < n) {
+            cic_cell(px[i], cells_per_len, cell[k][0], frac[k][0]);
+            cic_cell(py[i], cells_per_len, cell[k][1], frac[k][1]);
+            cic_cell(pz[i], cells_per_len, cell[k][2], frac[k][2]);
+            w[k] = m[i] * inv_cell_vol;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                lo[a] = min(lo[a], cell[k][a]);
+                lo[a + 3] = min(lo[a + 3], -cell[k][a]);
+            }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+        for (int o = 32; o > 0; o >>= 1)
+            lo[a] = min(lo[a], __shfl_xor(lo[a], o, 64));
+        if ((threadIdx.x & 63) == 0)
+            lim[threadIdx.x >> 6][a] = lo[a];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 6; ++a)
+        for (int v = 0; v < kDepositThreads / 64; ++v)
+            lo[a] = min(lo[a], lim[v][a]);
+    // extents in 64 bits: a chunk may span any range of cells
+    const long long ex = -static_cast<long long>(lo[3]) - lo[0] + 2;
+    const long long ey = -static_cast<long long>(lo[4]) - lo[1] + 2;
+    const long long ez = -static_cast<long long>(lo[5]) - lo[2] + 2;
+    const bool fits = ex <= kDepositCells && ey <= kDepositCells && ez <= kDepositCells &&
+                      ex * ey <= kDepositCells && ex * ey * ez <= kDepositCells;
+    const int wy = static_cast<int>(ey), wz = static_cast<int>(ez);
+    const int cells = fits ? static_cast<int>(ex * ey * ez) : 0;
+    for (int c = threadIdx.x; c < cells; c += kDepositThreads)
+        win[c] = 0.0f;
+    __syncthreads();
     const size_t NN = static_cast<size_t>(N);
-    const int xs[2] = {ix, jx}, ys[2] = {iy, jy}, zs[2] = {iz, jz};
-    const float wx[2] = {1.0f - fx, fx}, wy[2] = {1.0f - fy, fy}, wz[2] = {1.0f - fz, fz};
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b)
-            for (int c = 0; c < 2; ++c)
-                atomicAdd(&rho[(static_cast<size_t>(xs[a]) * NN + ys[b]) * NN + zs[c]],
-                          w * wx[a] * wy[b] * wz[c]);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const size_t i = static_cast<size_t>(blockIdx.x) * kDepositChunk +
+                         static_cast<size_t>(k * kDepositThreads) + threadIdx.x;
+        if (i >= n)
+            continue;
+        const float fx[2] = {1.0f - frac[k][0], frac[k][0]};
+        const float fy[2] = {1.0f - frac[k][1], frac[k][1]};
+        const float fz[2] = {1.0f - frac[k][2], frac[k][2]};
+        if (fits) {
+            float* at = win + ((cell[k][0] - lo[0]) * wy + cell[k][1] - lo[1]) * wz +
+                        cell[k][2] - lo[2];
+            for (int a = 0; a < 2; ++a)
+                for (int b = 0; b < 2; ++b)
+                    for (int c = 0; c < 2; ++c)
+                        unsafeAtomicAdd(at + (a * wy + b) * wz + c, w[k] * fx[a] * fy[b] * fz[c]);
+        } else {
+            const int ix = wrap_cell(cell[k][0], N), iy = wrap_cell(cell[k][1], N),
+                      iz = wrap_cell(cell[k][2], N);
+            const int xs[2] = {ix, ix + 1 == N ? 0 : ix + 1};
+            const int ys[2] = {iy, iy + 1 == N ? 0 : iy + 1};
+            const int zs[2] = {iz, iz + 1 == N ? 0 : iz + 1};
+            for (int a = 0; a < 2; ++a)
+                for (int b = 0; b < 2; ++b)
+                    for (int c = 0; c < 2; ++c)
+                        atomicAdd(&rho[(static_cast<size_t>(xs[a]) * NN + ys[b]) * NN + zs[c]],
+                                  w[k] * fx[a] * fy[b] * fz[c]);
+        }
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < cells; c += kDepositThreads) {
+        const float v = win[c];
+        if (v == 0.0f)
+            continue;
+        const int xy = c / wz, x = xy / wy;
+        atomicAdd(&rho[(static_cast<size_t>(wrap_cell(lo[0] + x, N)) * NN +
+                        wrap_cell(lo[1] + xy - x * wy, N)) * NN +
+                       wrap_cell(lo[2] + c - xy * wz, N)], v);
+    }
 }
 
 __device__ inline float sincf_half(float kh)  // sin(kh/2) / (kh/2)
@@ -211,7 +303,8 @@ bool launch_pm_accel(Device& d, PmState& pm, double L, float rs, float max_acc)
     const double cpl = static_cast<double>(N) / L;
     const double h = L / N;
     launch_fill_u32(reinterpret_cast<uint32_t*>(pm.rho), 0u, cells, d.stream);
-    pm_deposit_kernel<<<grid_for(d.n), 256, 0, d.stream>>>(
+    pm_deposit_kernel<<<static_cast<unsigned>((d.n + kDepositChunk - 1) / kDepositChunk),
+                        kDepositThreads, 0, d.stream>>>(
         d.pos[0], d.pos[1], d.pos[2], d.mass, d.n, N, cpl, static_cast<float>(1.0 / (h * h * h)),
         pm.rho);
     void* in[1] = {pm.rho};

@@ -143,23 +143,21 @@ __constant__ float kTpmQ[14] = {
     1.174437930e-04f,  -1.865963713e-05f, 2.218408781e-06f, -1.821118900e-07f,
     9.095778353e-09f,  -2.065529969e-10f};
 
-// w(x) and E(x) = exp(-x^2 / 4), x = r / rs
-__device__ inline float tpm_weight_e(float x, float& E)
+// w(x) and E(x) = exp(-x^2 / 4), x = r / rs. The exponent comes from r^2 (r2, with
+// e2 = -log2(e) / 4 rs^2) instead of x: one product less and one rounding less (w
+// errs by at most 1.6e-7 instead of 2.2e-7, r and x rounded to FP32 included).
+__device__ inline float tpm_weight_e(float x, float r2, float e2, float& E)
 {
     const float xc = fminf(x, 8.0f);
     float q = kTpmQ[13];
 #pragma unroll
     for (int k = 12; k >= 0; --k)
         q = fmaf(q, xc, kTpmQ[k]);
-    E = __builtin_amdgcn_exp2f(-(x * x) * 0.3606737554f);  // log2(e) / 4
+    E = __builtin_amdgcn_exp2f(r2 * e2);
     return q * E;
 }
 
-__device__ inline float tpm_weight(float r, float inv_rs)
-{
-    float E;
-    return tpm_weight_e(r * inv_rs, E);
-}
+__device__ inline float tpm_e2(float inv_rs) { return -0.3606737554f * (inv_rs * inv_rs); }
 
 // An accepted node in the cell list: (COM, mass), (qxx, qxy, qxz, qyy),
 // (qyz, trs term, qzz, -). The trs term is eps^2 trs in the open walk, trs in the
@@ -176,9 +174,14 @@ struct Cell {
 // share (DJ = 1) starts at entry 0: every lane makes the same number of turns, and
 // the loop is counted in scalar registers. Counted per lane it took 2.2 VALU
 // instructions of 36 per cell and 0.75 of 13.75 per particle.
+constexpr uint32_t kHalfBox = 1u << 31;  // beside a wave's count of accepted cells
 constexpr float kPadFar = 1.0e18f;  // its square is finite in FP32, its force zero
 
-template <int ORDER, bool TPM, int DJ>
+// WRAP: pairs take their nearest image (a periodic TreePM box). The walk shifts every
+// node to the image nearest to the group, so a pair needs its own only where an entry
+// lies half a box from some target (far_image in walk_kernel); elsewhere rounding the
+// separation to whole boxes gives 0, and the loops without it sum the same bits.
+template <int ORDER, bool TPM, bool WRAP, int DJ>
 __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int j0, float tx,
                                      float ty, float tz, const WalkParams& P, float& ax, float& ay,
                                      float& az)
@@ -187,13 +190,16 @@ __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int
     const int turns = DJ == 1 || !TPM ? (ncell + DJ - 1) / DJ : (ncell - j0 + DJ - 1) / DJ;
     const Cell* p = DJ == 1 ? cl : cl + j0;
     const float inv_rs = TPM ? 1.0f / P.rs : 0.0f;
-    const float box = TPM ? P.box : 0.0f;
-    const float ib = box > 0.0f ? 1.0f / box : 0.0f;
+    const float e2 = TPM ? tpm_e2(inv_rs) : 0.0f;
+    const float cE = 0.28209479177387814f * inv_rs * inv_rs * inv_rs;  // 1 / (2 sqrt(pi) rs^3)
+    const float cE2 = 0.25f * inv_rs * inv_rs * cE;
+    const float box = WRAP ? P.box : 0.0f;
+    const float ib = WRAP ? 1.0f / box : 0.0f;
 #pragma unroll 2
     for (int k = 0; k < turns; ++k, p += DJ) {
         const float4 a = p->a;
         float dx = a.x - tx, dy = a.y - ty, dz = a.z - tz;
-        if (TPM && box > 0.0f) {  // nearest image of this pair
+        if (WRAP) {  // nearest image of this pair
             dx -= box * rintf(dx * ib);
             dy -= box * rintf(dy * ib);
             dz -= box * rintf(dz * ib);
@@ -202,9 +208,9 @@ __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int
         const float ri = __frsqrt_rn(r2);
         const float ri2 = ri * ri;
         const float ri3 = ri * ri2;
-        float wgt = 1.0f;
+        float wgt = 1.0f, E;
         if (TPM && ORDER < 2)
-            wgt = tpm_weight(r2 * ri, inv_rs);
+            wgt = tpm_weight_e(r2 * ri * inv_rs, r2, e2, E);
         if (TPM && ORDER >= 2) {
             // Second-order expansion of the short-range kernel g(R) d,
             // g = w(R) / R^3, about the COM (S = (Q + trs I) / 3 the raw
@@ -212,33 +218,27 @@ __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int
             //   a = [M g + G2 (dQd + trs |d|^2) / 6 + 5/6 G1 trs] d + G1 / 3 Q d
             // with G1 = g'(R) / R, G2 = G1'(R) / R. For the erfc weight,
             // w'(R) = -R^2 E / (2 sqrt(pi) rs^3), E = exp(-R^2 / 4 rs^2), so
-            //   G1 = -c / R^2 - 3 w / R^5,
-            //   G2 = c (1 / (2 rs^2 R^2) + 5 / R^4) + 15 w / R^7,
-            // c = E / (2 sqrt(pi) rs^3). With w = 1, c = 0 it is the softened
-            // Newtonian expansion of the open walk.
+            // with c = E / (2 sqrt(pi) rs^3)
+            //   u = -G1 = (c + 3 g) / R^2,
+            //   G2 = (c / (2 rs^2) + 5 u) / R^2.
+            // With w = 1, c = 0 it is the softened Newtonian expansion of the open
+            // walk. The list holds Q / 3, trs / 3 and 5/6 trs, so that no factor is
+            // left over: 56 VALU instructions a cell against 66.
             const float4 b = p->b;
-            const float4 c = p->c;  // (qyz, trs, qzz)
+            const float4 c = p->c;  // (qyz, trs, qzz) / 3, 5/6 trs
             const float qx = fmaf(b.z, dz, fmaf(b.y, dy, b.x * dx));
             const float qy = fmaf(c.x, dz, fmaf(b.w, dy, b.y * dx));
             const float qz = fmaf(c.z, dz, fmaf(c.x, dy, b.z * dx));
-            const float dqd = fmaf(dz, qz, fmaf(dy, qy, dx * qx));
-            const float R = r2 * ri;
-            float E;
-            const float w = tpm_weight_e(R * inv_rs, E);
-            const float cE = E * (0.28209479177387814f * inv_rs * inv_rs * inv_rs);
-            const float ri4 = ri2 * ri2;
-            const float wr5 = w * ri4 * ri;
+            const float w = tpm_weight_e(r2 * ri * inv_rs, r2, e2, E);
             const float g = w * ri3;
-            const float G1 = fmaf(-cE, ri2, -3.0f * wr5);
-            const float G2 = fmaf(cE, fmaf(0.5f * inv_rs * inv_rs, ri2, 5.0f * ri4),
-                                  15.0f * wr5 * ri2);
+            const float u = fmaf(3.0f, g, E * cE) * ri2;
+            const float h = fmaf(2.5f, u, E * cE2) * ri2;  // G2 / 2
             const float d2 = r2 - P.eps2;
-            const float s = fmaf(G2 * (1.0f / 6.0f), fmaf(c.y, d2, dqd),
-                                 fmaf(a.w, g, (5.0f / 6.0f) * G1 * c.y));
-            const float t = G1 * (1.0f / 3.0f);
-            ax = fmaf(t, qx, fmaf(s, dx, ax));
-            ay = fmaf(t, qy, fmaf(s, dy, ay));
-            az = fmaf(t, qz, fmaf(s, dz, az));
+            const float q2 = fmaf(dz, qz, fmaf(dy, qy, fmaf(dx, qx, c.y * d2)));
+            const float s = fmaf(h, q2, fmaf(a.w, g, -(c.w * u)));
+            ax = fmaf(-u, qx, fmaf(s, dx, ax));
+            ay = fmaf(-u, qy, fmaf(s, dy, ay));
+            az = fmaf(-u, qz, fmaf(s, dz, az));
         } else if (ORDER >= 2) {
             const float4 b = p->b;
             const float4 c = p->c;
@@ -263,7 +263,7 @@ __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int
     }
 }
 
-template <bool TPM, int DJ>
+template <bool TPM, bool WRAP, int DJ>
 __device__ inline void eval_parts_dj(const float4* __restrict__ pl, int np, int j0, float tx,
                                      float ty, float tz, const WalkParams& P, float& ax, float& ay,
                                      float& az)
@@ -288,27 +288,32 @@ __device__ inline void eval_parts_dj(const float4* __restrict__ pl, int np, int 
         return;
     }
     const float inv_rs = TPM ? 1.0f / P.rs : 0.0f;
-    const float box = TPM ? P.box : 0.0f;
-    const float ib = box > 0.0f ? 1.0f / box : 0.0f;
+    const float e2 = TPM ? tpm_e2(inv_rs) : 0.0f;
+    const float box = WRAP ? P.box : 0.0f;
+    const float ib = WRAP ? 1.0f / box : 0.0f;
+    const float cut2 = TPM && P.rcut2 > 0.0f ? P.rcut2 : __builtin_inff();
 #pragma unroll 4
     for (int k = 0; k < turns; ++k, p += DJ) {
         const float4 a = *p;
         float dx = a.x - tx, dy = a.y - ty, dz = a.z - tz;
-        if (TPM && box > 0.0f) {  // nearest image of this pair
+        if (WRAP) {  // nearest image of this pair
             dx -= box * rintf(dx * ib);
             dy -= box * rintf(dy * ib);
             dz -= box * rintf(dz * ib);
         }
-        const float d2 = dx * dx + dy * dy + dz * dz;
+        // (the order of the sum is that of every loop here: a pair at the cutoff is
+        // in or out by its last bit)
+        const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
         const float r2 = d2 + P.eps2;
         const float ri = __frsqrt_rn(r2);
-        bool use = r2 > P.min_d2;
-        float wgt = 1.0f;
+        // (both tests without a branch: a wavefront hardly ever drops all of a pair)
+        const bool use = (r2 > P.min_d2) & (!TPM || d2 <= cut2);
+        float s = a.w * ri * ri * ri;
         if (TPM) {
-            wgt = tpm_weight(r2 * ri, inv_rs);
-            use = use && (P.rcut2 <= 0.0f || d2 <= P.rcut2);
+            float E;
+            s *= tpm_weight_e(r2 * ri * inv_rs, r2, e2, E);
         }
-        const float s = use ? a.w * ri * ri * ri * wgt : 0.0f;
+        s = use ? s : 0.0f;
         ax += s * dx;
         ay += s * dy;
         az += s * dz;
@@ -341,32 +346,54 @@ __device__ inline void pad_parts(float4* pl, int n, int dj)
     __syncthreads();
 }
 
+template <int ORDER, bool TPM, bool WRAP, int W>
+__device__ inline void eval_cells_w(const Cell* __restrict__ cl, int ncell, int j0, int dj,
+                                    float tx, float ty, float tz, const WalkParams& P, float& ax,
+                                    float& ay, float& az)
+{
+    if (dj == 1)
+        eval_cells_dj<ORDER, TPM, WRAP, W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
+    else if (dj == 2)
+        eval_cells_dj<ORDER, TPM, WRAP, 2 * W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
+    else
+        eval_cells_dj<ORDER, TPM, WRAP, 4 * W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
+}
+
 template <int ORDER, bool TPM, int W>
-__device__ inline void eval_cells(Cell* __restrict__ cl, int ncell, int j0, int dj, float tx,
-                                  float ty, float tz, const WalkParams& P, float& ax, float& ay,
-                                  float& az)
+__device__ inline void eval_cells(Cell* __restrict__ cl, int ncell, int j0, int dj, bool wrap,
+                                  float tx, float ty, float tz, const WalkParams& P, float& ax,
+                                  float& ay, float& az)
 {
     pad_cells<TPM, W>(cl, ncell, dj);
-    if (dj == 1)
-        eval_cells_dj<ORDER, TPM, W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
-    else if (dj == 2)
-        eval_cells_dj<ORDER, TPM, 2 * W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
+    if (TPM && wrap)
+        eval_cells_w<ORDER, TPM, TPM, W>(cl, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
     else
-        eval_cells_dj<ORDER, TPM, 4 * W>(cl, ncell, j0, tx, ty, tz, P, ax, ay, az);
+        eval_cells_w<ORDER, TPM, false, W>(cl, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
+}
+
+template <bool TPM, bool WRAP, int W>
+__device__ inline void eval_parts_w(const float4* __restrict__ pl, int np, int j0, int dj,
+                                    float tx, float ty, float tz, const WalkParams& P, float& ax,
+                                    float& ay, float& az)
+{
+    if (dj == 1)
+        eval_parts_dj<TPM, WRAP, W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+    else if (dj == 2)
+        eval_parts_dj<TPM, WRAP, 2 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+    else
+        eval_parts_dj<TPM, WRAP, 4 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
 }
 
 template <bool TPM, int W>
-__device__ inline void eval_parts(float4* __restrict__ pl, int np, int j0, int dj, float tx,
-                                  float ty, float tz, const WalkParams& P, float& ax, float& ay,
-                                  float& az)
+__device__ inline void eval_parts(float4* __restrict__ pl, int np, int j0, int dj, bool wrap,
+                                  float tx, float ty, float tz, const WalkParams& P, float& ax,
+                                  float& ay, float& az)
 {
     pad_parts<TPM, W>(pl, np, dj);
-    if (dj == 1)
-        eval_parts_dj<TPM, W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
-    else if (dj == 2)
-        eval_parts_dj<TPM, 2 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+    if (TPM && wrap)
+        eval_parts_w<TPM, TPM, W>(pl, np, j0, dj, tx, ty, tz, P, ax, ay, az);
     else
-        eval_parts_dj<TPM, 4 * W>(pl, np, j0, tx, ty, tz, P, ax, ay, az);
+        eval_parts_w<TPM, false, W>(pl, np, j0, dj, tx, ty, tz, P, ax, ay, az);
 }
 
 // Group far field: the local (Taylor) expansion about the group centre of an
@@ -651,6 +678,8 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             fsum[lane] = 0.0f;
         int ncell = 0, npart = 0;
         int nrec = 0;
+        // TreePM: some entry lies half a box or more from some target (uniform)
+        bool far_image = false;
         int sp = 1;
         if (threadIdx.x == 0) {
             if (W > 1)
@@ -774,6 +803,14 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
                     }
                 }
             }
+            bool half_box = false;  // of what this wave adds
+            if (TPM && P.box > 0.0f) {
+                const float reach = fmaxf(fmaxf(fabsf(px - gcx) + ghx, fabsf(py - gcy) + ghy),
+                                          fabsf(pz - gcz) + ghz) + w.bmax;
+                half_box = __ballot((accept || direct) && reach >= 0.49f * P.box) != 0ull;
+                if (W == 1)
+                    far_image = far_image || half_box;
+            }
 
             if (REC) {
                 near = near && accept;
@@ -852,7 +889,7 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             if (W > 1) {
                 if (lane == 0) {
                     wtot[wv][0] = static_cast<uint32_t>(nm);
-                    wtot[wv][1] = static_cast<uint32_t>(na);
+                    wtot[wv][1] = static_cast<uint32_t>(na) | (half_box ? kHalfBox : 0u);
                     wtot[wv][2] = static_cast<uint32_t>(nd);
                     wtot[wv][3] = static_cast<uint32_t>(ctot);
                     wtot[wv][4] = ltot;
@@ -864,12 +901,14 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
                 for (int k = 0; k < W; ++k) {
                     const bool prior = k < wv;
                     om += prior ? static_cast<int>(wtot[k][0]) : 0;
-                    oa += prior ? static_cast<int>(wtot[k][1]) : 0;
+                    const uint32_t nak = wtot[k][1];
+                    far_image = far_image || (TPM && (nak & kHalfBox) != 0u);
+                    oa += prior ? static_cast<int>(nak & ~kHalfBox) : 0;
                     od += prior ? static_cast<int>(wtot[k][2]) : 0;
                     oc += prior ? static_cast<int>(wtot[k][3]) : 0;
                     ol += prior ? wtot[k][4] : 0u;
                     nm += static_cast<int>(wtot[k][0]);
-                    na += static_cast<int>(wtot[k][1]);
+                    na += static_cast<int>(nak & ~kHalfBox);
                     nd += static_cast<int>(wtot[k][2]);
                     ctot += static_cast<int>(wtot[k][3]);
                     ltot += wtot[k][4];
@@ -879,7 +918,7 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             // 1) accepted nodes -> LDS cell list (point masses -> particle list)
             if (CRIT == 3 && nm > 0) {
                 if (npart + nm >= kPartCap) {  // uniform; keeps npart < kPartCap
-                    eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+                    eval_parts<TPM, W>(pl, npart, j0, dj, far_image, tx, ty, tz, P, ax, ay, az);
                     npp += static_cast<unsigned long long>(npart);
                     npart = 0;
                     __syncthreads();
@@ -893,10 +932,18 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             if (accept) {
                 const int slot = ncell + oa + static_cast<int>(__popcll(am & lt));
                 cl[slot].a = make_float4(px, py, pz, w.mass);
-                cl[slot].b = make_float4(w.qxx, w.qxy, w.qxz, w.qyy);
-                // the open walk's expansion needs eps^2 trs, the TreePM one trs
-                cl[slot].c = make_float4(w.qyz, TPM ? w.trs : P.eps2 * w.trs,
-                                         -(w.qxx + w.qyy), 0.0f);
+                // the open walk's expansion needs eps^2 trs, the TreePM one Q / 3, trs / 3
+                // and 5/6 trs
+                constexpr float third = 1.0f / 3.0f;
+                if (TPM) {
+                    cl[slot].b = make_float4(third * w.qxx, third * w.qxy, third * w.qxz,
+                                             third * w.qyy);
+                    cl[slot].c = make_float4(third * w.qyz, third * w.trs,
+                                             -third * (w.qxx + w.qyy), (2.5f * third) * w.trs);
+                } else {
+                    cl[slot].b = make_float4(w.qxx, w.qxy, w.qxz, w.qyy);
+                    cl[slot].c = make_float4(w.qyz, P.eps2 * w.trs, -(w.qxx + w.qyy), 0.0f);
+                }
             }
             ncell += na;
 
@@ -935,7 +982,7 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             }
 
             if (ncell > kCellCap - kThreads) {
-                eval_cells<ORDER, TPM, W>(cl, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
+                eval_cells<ORDER, TPM, W>(cl, ncell, j0, dj, far_image, tx, ty, tz, P, ax, ay, az);
                 npc += static_cast<unsigned long long>(ncell);
                 ncell = 0;
                 __syncthreads();
@@ -963,15 +1010,15 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
                 npart += static_cast<int>(chunk);
                 done += chunk;
                 if (npart == kPartCap) {
-                    eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+                    eval_parts<TPM, W>(pl, npart, j0, dj, far_image, tx, ty, tz, P, ax, ay, az);
                     npp += static_cast<unsigned long long>(npart);
                     npart = 0;
                     __syncthreads();
                 }
             }
         }
-        eval_cells<ORDER, TPM, W>(cl, ncell, j0, dj, tx, ty, tz, P, ax, ay, az);
-        eval_parts<TPM, W>(pl, npart, j0, dj, tx, ty, tz, P, ax, ay, az);
+        eval_cells<ORDER, TPM, W>(cl, ncell, j0, dj, far_image, tx, ty, tz, P, ax, ay, az);
+        eval_parts<TPM, W>(pl, npart, j0, dj, far_image, tx, ty, tz, P, ax, ay, az);
         npc += static_cast<unsigned long long>(ncell);
         npp += static_cast<unsigned long long>(npart);
         for (int o = 32; o >= tw; o >>= 1) {  // the list shares of one target
