@@ -510,6 +510,31 @@ __device__ inline void far_flush(const uint32_t* __restrict__ fl, int nfl,
     }
 }
 
+// Pushes nodes first, first + 1, ... (1 to 8 of them) by at most three stores. One store
+// per child took as many turns as the wavefront's largest nc, of 6 VALU instructions.
+__device__ inline void push_children(int* __restrict__ to, int first, uint32_t nc)
+{
+    typedef int int4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef int int2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+    if (nc >= 4u) {
+        *reinterpret_cast<int4_a4*>(to) = int4_a4{first, first + 1, first + 2, first + 3};
+        to += 4;
+        first += 4;
+        nc -= 4u;
+    }
+    if (nc == 4u) {
+        *reinterpret_cast<int4_a4*>(to) = int4_a4{first, first + 1, first + 2, first + 3};
+        return;
+    }
+    if (nc & 2u) {
+        *reinterpret_cast<int2_a4*>(to) = int2_a4{first, first + 1};
+        to += 2;
+        first += 2;
+    }
+    if (nc & 1u)
+        *to = first;
+}
+
 // W waves walk one group together (W > 1: small walks, see walk_waves). They
 // pop up to 64 W nodes per step, share the lists in LDS, take every W-th
 // entry of them each and add their shares of a target's force in wave order at
@@ -952,11 +977,14 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
                 if (threadIdx.x == 0)
                     atomicOr(err, kErrStackOverflow);
             } else {
-                if (open) {
-                    const int base = sp + oc + static_cast<int>(cinc - nc);
+                const int base = sp + oc + static_cast<int>(cinc - nc);
+                if (W == 1) {
+                    if (open)
+                        push_children(stk + base, w.first, nc);
+                } else if (open) {
                     for (uint32_t j = 0; j < nc; ++j) {
                         const int at = base + static_cast<int>(j);
-                        if (W > 1 && at < kLdsStack)
+                        if (at < kLdsStack)
                             lstk[W > 1 ? at : 0] = w.first + static_cast<int>(j);
                         else
                             stk[at] = w.first + static_cast<int>(j);
@@ -974,6 +1002,8 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
                 lfSy[slot] = sy;
                 lfSz[slot] = sz;
             }
+            if (static_cast<int>(threadIdx.x) >= nd)
+                lfPre[threadIdx.x] = ~0u;  // past the last leaf, for the search below
             __syncthreads();
 
             if (FAR && nfl > kFarCap - 64) {
@@ -989,19 +1019,17 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
             }
 
             uint32_t done = 0;
+            const int top = nd > 1 ? 1 << (31 - __builtin_clz(static_cast<unsigned>(nd - 1))) : 0;
             while (done < ltot) {
                 const uint32_t room = static_cast<uint32_t>(kPartCap - npart);
                 const uint32_t chunk = ltot - done < room ? ltot - done : room;
                 for (uint32_t f = threadIdx.x; f < chunk; f += static_cast<uint32_t>(kThreads)) {
                     const uint32_t gi = done + f;
-                    int lo = 0, hi = nd - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (lfPre[mid] <= gi)
-                            lo = mid;
-                        else
-                            hi = mid - 1;
-                    }
+                    // the last leaf that starts at gi or before: a step per bit of nd - 1,
+                    // the same for all lanes, 3 VALU instructions each (7 with two bounds)
+                    int lo = 0;
+                    for (int step = top; step > 0; step >>= 1)
+                        lo += lfPre[lo + step] <= gi ? step : 0;
                     const float4 q = spart[lfFirst[lo] + static_cast<int>(gi - lfPre[lo])];
                     pl[npart + static_cast<int>(f)] =
                         make_float4(q.x + lfSx[lo], q.y + lfSy[lo], q.z + lfSz[lo], q.w);
