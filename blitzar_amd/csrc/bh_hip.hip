@@ -597,10 +597,12 @@ uint32_t group_max(const bh_hip_handle* h)
     return g;
 }
 
-void end_build(bh_hip_handle* h, StepEvents* ev)
+// ended: the moments' last kernel has done launch_end_build's work
+void end_build(bh_hip_handle* h, StepEvents* ev, bool ended)
 {
     rec(ev ? ev->b1 : nullptr, h->d.stream);
-    bh::launch_end_build(h->d);
+    if (!ended)
+        bh::launch_end_build(h->d);
     (void)hipEventRecord(h->built, h->d.stream);
     h->rank_valid = false;
     h->have_tree = true;
@@ -627,20 +629,21 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
         bh::launch_radix_sort(d, d.n, h->p.key_mode == 1 ? 30 : 63);
     }
     rec(ev ? ev->s1 : nullptr, d.stream);
-    bh::launch_tie_fix(d);
     if (d.n <= kOneStreamMax) {
         bh::launch_tree_build(d, h->leaf_depth, h->p.bucket_capacity, d.stream);
         rec(ev ? ev->t1 : nullptr, d.stream);
         bh::launch_permute_all(d, d.stream);
         rec(ev ? ev->p1 : nullptr, d.stream);
         rec(ev ? ev->j1 : nullptr, d.stream);
+        bool ended = false;
         if (h->p.key_mode == 0) {
             d.group_cap = group_max(h);
-            bh::launch_tree_moments(d, false, true);
+            ended = bh::launch_tree_moments(d, false, true, true);
         }
-        end_build(h, ev);
+        end_build(h, ev, ended);
         return;
     }
+    bh::launch_tie_fix(d);
     // The topology needs only the sorted keys: it runs on the side stream
     // while the main stream permutes the positions and masses. The rest of
     // the store (velocities, ids, |a|) and the walk groups follow the
@@ -663,7 +666,7 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
     if (h->p.key_mode == 0)
         bh::launch_tree_moments(d);
     (void)hipStreamWaitEvent(d.stream, h->ev_groups, 0);
-    end_build(h, ev);
+    end_build(h, ev, false);
 }
 
 // Moments of the current positions on the topology of the last build (block
@@ -674,9 +677,10 @@ void queue_refit(bh_hip_handle* h, StepEvents* ev)
     for (hipEvent_t e : {ev ? ev->b0 : nullptr, ev ? ev->s0 : nullptr, ev ? ev->s1 : nullptr,
                          ev ? ev->p1 : nullptr, ev ? ev->t1 : nullptr, ev ? ev->j1 : nullptr})
         rec(e, d.stream);
-    bh::launch_tree_moments(d, true);
+    const bool ended = bh::launch_tree_moments(d, true, false, true);
     rec(ev ? ev->b1 : nullptr, d.stream);
-    bh::launch_end_build(d);
+    if (!ended)
+        bh::launch_end_build(d);
     (void)hipEventRecord(h->built, d.stream);
 }
 

@@ -187,6 +187,22 @@ struct HostReport {
     int info[2 * kLevels + 4];
 };
 
+// A build's end, by one workgroup whose kernel starts after all others of the build:
+// the walk's tickets cleared and the error word to the host. report null: not here.
+struct EndBuild {
+    unsigned int* tickets = nullptr;
+    HostReport* report = nullptr;
+};
+__device__ inline void end_build(const int* err, const EndBuild& end)
+{
+    for (int i = threadIdx.x; i < kTicketWords; i += blockDim.x)
+        end.tickets[i] = 0u;
+    __syncthreads();  // the workgroup's own errors are raised by now
+    if (threadIdx.x == 0)
+        end.report->err_build =
+            __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Device buffers of one solver instance. The particle store is kept in the
 // order of the last sort (Morton order); `id` maps a store slot to the
 // caller's particle index and `rank` maps back.
@@ -351,7 +367,8 @@ void launch_tie_fix(Device& d);
 // then velocities, ids, |a| and the block time-step arrays, each on its stream
 void launch_permute_store(Device& d, hipStream_t s);
 void launch_permute_rest(Device& d, hipStream_t s);
-void launch_permute_all(Device& d, hipStream_t s);  // both in one launch
+// Both in one launch, equal keys ordered by particle id on the way (no launch_tie_fix).
+void launch_permute_all(Device& d, hipStream_t s);
 void launch_rank(Device& d);  // rebuild rank from id
 // k_tree.hip
 void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s);
@@ -360,7 +377,9 @@ void launch_tree_build(Device& d, int leaf_depth, int bucket, hipStream_t s);
 // moved since); each node's level in the walk record is lowered until its
 // cell covers the node's particles. groups: also the walk groups of d.group_cap
 // (launch_groups), in the leaves' launch.
-void launch_tree_moments(Device& d, bool refit = false, bool groups = false);
+// end: the build ends with these kernels (nothing of it runs beside them), so that the
+// last of them may do the work of launch_end_build; true where it did.
+bool launch_tree_moments(Device& d, bool refit = false, bool groups = false, bool end = false);
 // Walk groups: a partition of the sorted particles into spatially compact
 // runs of at most gmax <= kGroupMax particles (consecutive small children of
 // one node packed together; see node_groups in k_tree.hip).

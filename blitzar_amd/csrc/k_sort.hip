@@ -486,9 +486,13 @@ __global__ __launch_bounds__(256) void permute_rest_kernel(
         oam[s] = am[j];
 }
 
-// Both parts in one launch, where they run one after the other anyway.
+// Both parts in one launch, where they run one after the other anyway. It also orders
+// equal keys by particle id (tie_fix_kernel's launch, 4 us of a small build's 170): the
+// thread at place s moves its source to the run's start plus the ids of the run below
+// its own. src_out takes the fixed order.
 __global__ __launch_bounds__(256) void permute_all_kernel(
-    const uint32_t* __restrict__ src, size_t n, const double* __restrict__ px,
+    const unsigned long long* __restrict__ keys, const uint32_t* __restrict__ src,
+    uint32_t* __restrict__ src_out, size_t n, const double* __restrict__ px,
     const double* __restrict__ py, const double* __restrict__ pz, const float* __restrict__ m,
     const double* __restrict__ vx, const double* __restrict__ vy, const double* __restrict__ vz,
     const uint32_t* __restrict__ id, const float* __restrict__ am, double* __restrict__ opx,
@@ -496,10 +500,21 @@ __global__ __launch_bounds__(256) void permute_all_kernel(
     double* __restrict__ ovx, double* __restrict__ ovy, double* __restrict__ ovz,
     uint32_t* __restrict__ oid, float* __restrict__ oam)
 {
-    const size_t s = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    size_t s = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (s >= n)
         return;
     const uint32_t j = src[s];
+    const uint32_t jid = id[j];
+    const unsigned long long k = keys[s];
+    if ((s > 0 && keys[s - 1] == k) || (s + 1 < n && keys[s + 1] == k)) {
+        size_t at = s, below = 0;
+        for (; at > 0 && keys[at - 1] == k; --at)
+            below += id[src[at - 1]] < jid ? 1 : 0;
+        for (size_t e = s + 1; e < n && keys[e] == k; ++e)
+            below += id[src[e]] < jid ? 1 : 0;
+        s = at + below;
+    }
+    src_out[s] = j;
     opx[s] = px[j];
     opy[s] = py[j];
     opz[s] = pz[j];
@@ -507,7 +522,7 @@ __global__ __launch_bounds__(256) void permute_all_kernel(
     ovx[s] = vx[j];
     ovy[s] = vy[j];
     ovz[s] = vz[j];
-    oid[s] = id[j];
+    oid[s] = jid;
     if (am)
         oam[s] = am[j];
 }
@@ -555,13 +570,9 @@ __global__ void begin_call_kernel(int* err, unsigned long long* stats)
         stats[threadIdx.x] = 0ull;
 }
 
-__global__ __launch_bounds__(256) void end_build_kernel(const int* err, unsigned int* tickets,
-                                                        HostReport* rep)
+__global__ __launch_bounds__(256) void end_build_kernel(const int* err, EndBuild end)
 {
-    for (int i = threadIdx.x; i < kTicketWords; i += blockDim.x)
-        tickets[i] = 0u;
-    if (threadIdx.x == 0)
-        rep->err_build = *err;
+    end_build(err, end);
 }
 
 __global__ void report_kernel(const int* err, const unsigned long long* stats, const int* info,
@@ -808,9 +819,10 @@ void launch_permute_all(Device& d, hipStream_t st)
         return;
     const unsigned blocks = static_cast<unsigned>((d.n + 255) / 256);
     permute_all_kernel<<<blocks, 256, 0, st>>>(
-        d.vals, d.n, d.pos[0], d.pos[1], d.pos[2], d.mass, d.vel[0], d.vel[1], d.vel[2], d.id,
+        reinterpret_cast<const unsigned long long*>(d.keys), d.vals, d.vals_b, d.n, d.pos[0], d.pos[1], d.pos[2], d.mass, d.vel[0], d.vel[1], d.vel[2], d.id,
         d.amag_live ? d.amag : nullptr, d.pos_b[0], d.pos_b[1], d.pos_b[2], d.mass_b, d.vel_b[0],
         d.vel_b[1], d.vel_b[2], d.id_b, d.amag_b);
+    std::swap(d.vals, d.vals_b);
     swap_positions(d);
     swap_rest(d);
     permute_adaptive(d, blocks, st);
@@ -830,7 +842,7 @@ void launch_begin_call(Device& d, unsigned long long* stats)
 
 void launch_end_build(Device& d)
 {
-    end_build_kernel<<<1, 256, 0, d.stream>>>(d.err, d.work_counter, d.report);
+    end_build_kernel<<<1, 256, 0, d.stream>>>(d.err, EndBuild{d.work_counter, d.report});
     d.tickets_zero = true;
 }
 

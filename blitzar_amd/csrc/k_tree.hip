@@ -1572,7 +1572,7 @@ __global__ __launch_bounds__(64 * W) void tile_moments_kernel(
     const uint32_t* __restrict__ nfirst, const int* __restrict__ info,
     const RootGeom* __restrict__ geom, WalkNode* __restrict__ wn, float* __restrict__ ext,
     float* __restrict__ noct, int refit, int* err, const uint32_t* __restrict__ tilecnt,
-    uint32_t ntiles, uint32_t per, uint32_t* __restrict__ cross)
+    uint32_t ntiles, uint32_t per, uint32_t* __restrict__ cross, EndBuild end)
 {
     __shared__ LevelLds<OCT, W> S;
     __shared__ uint32_t lvFirst[kLevels], lvEnd[kLevels];  // the tile's nodes per level
@@ -1637,6 +1637,8 @@ __global__ __launch_bounds__(64 * W) void tile_moments_kernel(
         }
         L = above;
     }
+    if (end.report)
+        end_build(err, end);
 }
 
 // The nodes the units left: unit u of this pass is kCrossUnits consecutive units of
@@ -1653,7 +1655,7 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
     const uint32_t* __restrict__ nfirst, const RootGeom* __restrict__ geom,
     WalkNode* __restrict__ wn, float* __restrict__ ext, float* __restrict__ noct, int refit,
     int* err, const uint32_t* __restrict__ cross_in, uint32_t nin, uint64_t unit,
-    uint32_t* __restrict__ cross_out, uint32_t nout)
+    uint32_t* __restrict__ cross_out, uint32_t nout, EndBuild end)
 {
     __shared__ LevelLds<OCT, kCrossUnits / 64> S;
     __shared__ uint32_t sNode[kMaxLevel][kCrossUnits];
@@ -1707,6 +1709,8 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
                          refit, err);
         L = above;
     }
+    if (end.report)
+        end_build(err, end);
 }
 
 // sleaf[s] = the leaf holding particle s (topology built level by level).
@@ -1872,7 +1876,7 @@ constexpr uint32_t kOneUnitTiles = 8;
 constexpr uint32_t kWideTiles = 512;
 
 template <bool OCT>
-void launch_moments_t(Device& d, int rf, bool groups)
+bool launch_moments_t(Device& d, int rf, bool groups, bool end)
 {
     const uint32_t n = static_cast<uint32_t>(d.n);
     float* noct = OCT ? d.noct : nullptr;
@@ -1890,13 +1894,17 @@ void launch_moments_t(Device& d, int rf, bool groups)
         uint32_t nin = topo_tiles(d.n);
         uint64_t unit = kTopoTile;
         const uint32_t ntiles = nin;
+        // the last launch is one workgroup: it ends the build (a launch of 4 us less)
+        const auto ending = [&](bool last) {
+            return end && last ? EndBuild{d.work_counter, d.report} : EndBuild{};
+        };
         const auto tiles = [&](auto waves, uint32_t per) {
             constexpr int W = decltype(waves)::value;
             nin = (ntiles + per - 1) / per;
             unit = static_cast<uint64_t>(per) * kTopoTile;
             tile_moments_kernel<OCT, W><<<nin, 64 * W, 0, d.stream>>>(
                 d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.level_info, d.geom, d.wnode,
-                d.next, noct, rf, d.err, d.topo_scan, ntiles, per, in);
+                d.next, noct, rf, d.err, d.topo_scan, ntiles, per, in, ending(nin == 1));
         };
         if (ntiles <= kOneUnitTiles)
             tiles(std::integral_constant<int, 4>{}, ntiles);
@@ -1910,29 +1918,29 @@ void launch_moments_t(Device& d, int rf, bool groups)
             unit *= kCrossUnits;
             cross_moments_kernel<OCT><<<nout, kCrossUnits, 0, d.stream>>>(
                 d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.geom, d.wnode, d.next, noct,
-                rf, d.err, in, nin, unit, out, nout);
+                rf, d.err, in, nin, unit, out, nout, ending(nout == 1));
             in = out;
             nin = nout;
         }
-        return;
+        d.tickets_zero = d.tickets_zero || end;
+        return end;
     }
     // level kMaxLevel holds leaves only
     for (int L = kMaxLevel - 1; L >= 0; --L)
         tree_moments_kernel<OCT><<<level_grid(level_bound(L, d.n, d.node_cap)), 256, 0, d.stream>>>(
             d.nprefix, d.ncount, d.nchild, d.nfirst, d.level_info, L, d.geom, d.wnode, d.next,
             noct, rf, d.err);
+    return false;
 }
 
 }  // namespace
 
-void launch_tree_moments(Device& d, bool refit, bool groups)
+bool launch_tree_moments(Device& d, bool refit, bool groups, bool end)
 {
     if (d.n == 0)
-        return;
-    if (d.noct)
-        launch_moments_t<true>(d, refit ? 1 : 0, groups);
-    else
-        launch_moments_t<false>(d, refit ? 1 : 0, groups);
+        return false;
+    return d.noct ? launch_moments_t<true>(d, refit ? 1 : 0, groups, end)
+                  : launch_moments_t<false>(d, refit ? 1 : 0, groups, end);
 }
 
 }  // namespace bh

@@ -45,3 +45,25 @@ def test_every_particle_is_in_one_walk_group(n, bucket):
     assert np.isfinite(a).all()
     assert (err <= 0.05 * np.maximum(scale, np.median(scale))).all()
     assert n == 1 or (np.linalg.norm(a, axis=1) > 0).all()
+
+
+# Equal keys leave in particle order whatever order the store had: runs of 2, 3 and
+# many, at the array's ends and across workgroups of 256; beyond 200,000 a launch of
+# its own does it. The positions come in a second upload, so that the slots of a run
+# are not in particle order.
+@pytest.mark.parametrize("n, cells", [(2, 1), (3, 1), (300, 1), (5000, 1), (5000, 40),
+                                      (200000, 20000), (200001, 20000)])
+def test_ties_follow_the_particle_index(oracle, n, cells):
+    rng = np.random.default_rng(n + cells)
+    first = rng.standard_normal((n, 3))
+    pos = rng.standard_normal((cells, 3))[rng.integers(0, cells, n)]
+    m = np.full(n, 1.0 / n, np.float32)
+    with B.OctreeHip(n, leaf_capacity=16, bucket_capacity=16) as s:
+        s.upload(first, None, m)
+        s.build_tree()
+        s.upload(pos, None, m)
+        s.build_tree()
+        t = s.dump_tree()
+    sk, order = oracle.stable_sort(oracle.keys(pos, 0))
+    assert np.array_equal(t["sorted_keys"], sk)
+    assert np.array_equal(t["sorted_ids"], order)
