@@ -79,7 +79,7 @@ struct bh_hip_handle {
     // (default priority), beside the store permutation and the moments:
     // sorted -> topology (side), topo -> moments (main), groups -> walk (main).
     hipStream_t side = nullptr;
-    hipEvent_t ev_sorted = nullptr, ev_topo = nullptr, ev_groups = nullptr;
+    hipEvent_t ev_sorted = nullptr, ev_topo = nullptr, ev_groups = nullptr, ev_due = nullptr;
     int err_carry = 0;      // error bits of this call kept across a node regrow
     int steps_done = -1;    // bh_hip_step: steps completed before an error stopped it
     // pinned ring of copy_out (allocated at the first copy, sized for it)
@@ -929,15 +929,19 @@ bool alloc_adaptive(bh_hip_handle* h)
 }
 
 // Build (or refit) + walk of one block-step force evaluation, regrown and
-// repeated on a node-capacity overflow (a refit makes no nodes).
-bool build_and_walk(bh_hip_handle* h, StepEvents* ev, const bh::WalkParams& wp,
-                    bool refit = false)
+// repeated on a node-capacity overflow (a refit makes no nodes). ready(), called with
+// the build queued, waits for what the walk's parameters need and sets them.
+template <class Ready>
+bool build_and_walk(bh_hip_handle* h, StepEvents* ev, const bh::WalkParams& wp, bool refit,
+                    const Ready& ready)
 {
     for (int attempt = 0; attempt < 8; ++attempt) {
         if (refit)
             queue_refit(h, ev);
         else
             queue_build(h, ev);
+        if (!ready())
+            return false;
         // A build permutes the block time-step levels with the store (the
         // buffer pointers swap): the walk must read the permuted ones.
         bh::WalkParams w = wp;
@@ -979,7 +983,7 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
         // ticks start at 0 so that every cadence 2^(L - level) divides the
         // start of each global step
         h->ad_tick = 0;
-        if (!build_and_walk(h, next_events(h), wp0))
+        if (!build_and_walk(h, next_events(h), wp0, false, [] { return true; }))
             return fail();
         bh::launch_adaptive_init(d, a, 0u);
         h->ad_primed = true;
@@ -989,7 +993,11 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
     // due is found on the device; the slices in between have no force
     // evaluation, so one predictor spans them (constant acceleration makes k
     // single-slice predictors one predictor over k q).
+    // The predictor takes the tick from the device, and it and the build or refit are
+    // queued before the host knows it; the host waits (for the predictor's report)
+    // only to give the walk its tick, while the moments run.
     uint32_t* due = reinterpret_cast<uint32_t*>(d.err + 1);
+    uint32_t* next_due = due + 1;
     bool due_known = false;  // the last correction found the next due tick
     const uint64_t slices = 1ull << a.levels;
     // The tree is built at the first force evaluation of each global step
@@ -1006,21 +1014,25 @@ bh_hip_result_t step_adaptive(bh_hip_handle* h, double dt, int32_t nsteps)
         while (h->ad_tick < end) {
             if (!due_known)
                 bh::launch_adaptive_next_due(d, a, static_cast<uint32_t>(h->ad_tick), due);
-            bh::launch_due_report(d, due);
-            if (!check(h, hipStreamSynchronize(d.stream), "adaptive schedule"))
-                return fail();
-            const uint64_t t = std::min<uint64_t>(end, h->ad_tick + d.report->due);
-            bh::launch_adaptive_drift(d, a, static_cast<double>(t - h->ad_tick) * a.quantum);
-            h->ad_tick = t;
-            const uint32_t tt = static_cast<uint32_t>(t);
+            const uint64_t from = h->ad_tick;
+            bh::launch_adaptive_drift(d, a, due, static_cast<uint32_t>(end - from), next_due);
+            (void)hipEventRecord(h->ev_due, d.stream);
             bh::WalkParams wp = wp0;
             wp.alevel = d.alevel;
-            wp.atick = tt;
             wp.alevels = a.levels;
-            if (!build_and_walk(h, next_events(h), wp, !first_slice && !rebuild_each))
+            const auto ready = [&] {
+                if (!check(h, hipEventSynchronize(h->ev_due), "adaptive schedule"))
+                    return false;
+                h->ad_tick = std::min<uint64_t>(end, from + d.report->due);
+                wp.atick = static_cast<uint32_t>(h->ad_tick);
+                return true;
+            };
+            if (!build_and_walk(h, next_events(h), wp, !first_slice && !rebuild_each, ready))
                 return fail();
+            const uint32_t tt = wp.atick;
             first_slice = false;
-            bh::launch_adaptive_correct(d, a, tt, h->stats + 2, due);
+            bh::launch_adaptive_correct(d, a, tt, h->stats + 2, next_due);
+            std::swap(due, next_due);
             due_known = true;
             if (bits_at_build(h) & kFatalBits) {
                 stop = true;
@@ -1129,7 +1141,7 @@ bh_hip_result_t bh_hip_create(const bh_hip_params_t* params, uint64_t n, bh_hip_
     h->leaf_depth = reference_leaf_depth(n, h->p.leaf_capacity);
     bool ok = check(h, hipStreamCreateWithFlags(&h->d.stream, hipStreamNonBlocking), "stream") &&
               check(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking), "stream");
-    for (hipEvent_t* x : {&h->ev_sorted, &h->ev_topo, &h->ev_groups})
+    for (hipEvent_t* x : {&h->ev_sorted, &h->ev_topo, &h->ev_groups, &h->ev_due})
         ok = ok && check(h, hipEventCreateWithFlags(x, hipEventDisableTiming), "event");
     ok = ok && alloc_all(h, n);
     ok = ok && check(h, hipEventCreateWithFlags(&h->built, hipEventDisableTiming), "event") &&
@@ -1178,7 +1190,7 @@ void bh_hip_destroy(bh_hip_handle_t* h)
     }
     if (h->built)
         (void)hipEventDestroy(h->built);
-    for (hipEvent_t x : {h->ev_sorted, h->ev_topo, h->ev_groups})
+    for (hipEvent_t x : {h->ev_sorted, h->ev_topo, h->ev_groups, h->ev_due})
         if (x)
             (void)hipEventDestroy(x);
     if (h->d.report)

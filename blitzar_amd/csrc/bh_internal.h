@@ -445,15 +445,17 @@ void pm_release(PmState& pm);
 bool launch_pm_accel(Device& d, PmState& pm, double L, float rs, float max_acc);
 // block time steps
 void launch_adaptive_init(Device& d, const AdaptiveParams& a, uint32_t tick);
-// Predictor over `span` (k slices of constant acceleration: x += v s + a s^2/2,
-// v += a s, the same as k single-slice predictors).
-void launch_adaptive_drift(Device& d, const AdaptiveParams& a, double span);
+// Predictor to the next due tick, *due ticks away and at most `left` (k slices of
+// constant acceleration: x += v s + a s^2/2, v += a s, the same as k single-slice
+// predictors). It also reports *due to the host and clears *next_due, which the next
+// correction lowers.
+void launch_adaptive_drift(Device& d, const AdaptiveParams& a, const uint32_t* due, uint32_t left,
+                           uint32_t* next_due);
 // *out = the first tick after t at which some particle is due.
 void launch_adaptive_next_due(Device& d, const AdaptiveParams& a, uint32_t t, uint32_t* out);
 // count (optional, device): += number of particles corrected
 void launch_adaptive_correct(Device& d, const AdaptiveParams& a, uint32_t tick,
                              unsigned long long* count, uint32_t* due);
-void launch_due_report(Device& d, uint32_t* due);
 void launch_gather_u32(Device& d, const uint32_t* src_by_slot, uint32_t* out_by_caller);
 
 }  // namespace bh

@@ -561,11 +561,17 @@ __global__ __launch_bounds__(256) void adaptive_drift_kernel(
     double* __restrict__ px, double* __restrict__ py, double* __restrict__ pz,
     double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz,
     const float* __restrict__ ax, const float* __restrict__ ay, const float* __restrict__ az,
-    size_t n, double q, double vmax, double box)
+    size_t n, const uint32_t* __restrict__ due, uint32_t left, double quantum, double vmax,
+    double box, uint32_t* __restrict__ next_due, HostReport* __restrict__ rep)
 {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        rep->due = *due;
+        *next_due = 0xffffffffu;
+    }
     if (i >= n)
         return;
+    const double q = static_cast<double>(min(*due, left)) * quantum;
     const double hq = 0.5 * q * q;
     const double gx = ax[i], gy = ay[i], gz = az[i];
     double x = vx[i], y = vy[i], z = vz[i];
@@ -616,15 +622,6 @@ __device__ inline uint32_t ticks_to_due(uint32_t level, int L, uint32_t t)
 {
     const uint32_t c = 1u << (static_cast<uint32_t>(L) - level);
     return (t / c + 1u) * c - t;
-}
-
-// The next due tick to the report, and the word cleared for the next minimum.
-__global__ void due_report_kernel(uint32_t* due, HostReport* rep)
-{
-    if (threadIdx.x == 0) {
-        rep->due = *due;
-        *due = 0xffffffffu;
-    }
 }
 
 // Corrector for the particles active at `tick` (their new force is in acc).
@@ -721,14 +718,15 @@ void launch_adaptive_init(Device& d, const AdaptiveParams& a, uint32_t tick)
         d.aacc[2], d.alevel, d.atick, d.n, a, tick);
 }
 
-void launch_adaptive_drift(Device& d, const AdaptiveParams& a, double span)
+void launch_adaptive_drift(Device& d, const AdaptiveParams& a, const uint32_t* due, uint32_t left,
+                           uint32_t* next_due)
 {
     d.aabb_parts = 0;
     if (d.n == 0)
         return;
     adaptive_drift_kernel<<<blocks_for(d.n), 256, 0, d.stream>>>(
         d.pos[0], d.pos[1], d.pos[2], d.vel[0], d.vel[1], d.vel[2], d.aacc[0], d.aacc[1],
-        d.aacc[2], d.n, span, a.max_speed, a.box);
+        d.aacc[2], d.n, due, left, a.quantum, a.max_speed, a.box, next_due, d.report);
 }
 
 void launch_adaptive_next_due(Device& d, const AdaptiveParams& a, uint32_t t, uint32_t* out)
@@ -750,11 +748,6 @@ void launch_adaptive_correct(Device& d, const AdaptiveParams& a, uint32_t tick,
     adaptive_correct_kernel<<<reduce_blocks(d.n), 256, 0, d.stream>>>(
         d.pos[0], d.pos[1], d.pos[2], d.vel[0], d.vel[1], d.vel[2], d.acc[0], d.acc[1], d.acc[2],
         d.aacc[0], d.aacc[1], d.aacc[2], d.alevel, d.atick, d.n, a, tick, count, due);
-}
-
-void launch_due_report(Device& d, uint32_t* due)
-{
-    due_report_kernel<<<1, 64, 0, d.stream>>>(due, d.report);
 }
 
 void launch_gather_u32(Device& d, const uint32_t* src_by_slot, uint32_t* out_by_caller)
