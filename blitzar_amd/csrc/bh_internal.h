@@ -132,11 +132,11 @@ constexpr int kTopoHalo = 64;
 inline uint32_t topo_tiles(size_t n) { return static_cast<uint32_t>((n + kTopoTile - 1) / kTopoTile); }
 inline size_t topo_count_words(size_t n) { return static_cast<size_t>(kLevels) * (topo_tiles(n) + 1); }
 // Nodes left over by the moments' passes over tiles (kLevels words per unit of
-// each pass, see cross_moments_kernel; the passes' units shrink 512-fold).
+// each pass, see cross_moments_kernel; the passes' units shrink 64-fold or more).
 inline size_t cross_words(size_t n)
 {
     const size_t t = topo_tiles(n);
-    return static_cast<size_t>(kLevels) * (t + t / 512 + t / 262144 + 4);
+    return static_cast<size_t>(kLevels) * (t + t / 32 + 8);
 }
 
 // Parameters the walk needs (by value into the kernel).

@@ -1641,12 +1641,19 @@ __global__ __launch_bounds__(64 * W) void tile_moments_kernel(
         end_build(err, end);
 }
 
-// The nodes the units left: unit u of this pass is kCrossUnits consecutive units of
-// the pass before, held by one workgroup. cross_in[L * nin + i] is the node of
-// level L that starts in input unit i and ends past it; the workgroup computes those
-// inside its own unit and passes on the one per level that ends past it. The last
-// pass has one unit, which holds everything.
+// The nodes the units left: unit u of this pass is `per` consecutive units of the pass
+// before, held by one workgroup. cross_in[L * nin + i] is the node of level L that
+// starts in input unit i and ends past it; the workgroup computes those inside its own
+// unit and passes on the one per level that ends past it. The last pass has one unit,
+// which holds everything.
+//
+// A pass lasts as long as its levels, about 20, and a level of many nodes takes them one
+// a lane, 2.5 us: many units go through a pass of kCrossSplit a workgroup first, whose
+// levels 8 lanes a node take. All passes, us, with kCrossUnits / kCrossSplit first:
+// 300,001 particles (293 tiles) 47 / 56, 1,048,576 87 / 60, 2,097,152 66 / 40, 8,388,608
+// 102 / 80; with third moments 524,288 (512 tiles) 92 / 70.
 constexpr int kCrossUnits = 512;
+constexpr int kCrossSplit = 64;
 
 template <bool OCT>
 __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
@@ -1655,12 +1662,13 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
     const uint32_t* __restrict__ nfirst, const RootGeom* __restrict__ geom,
     WalkNode* __restrict__ wn, float* __restrict__ ext, float* __restrict__ noct, int refit,
     int* err, const uint32_t* __restrict__ cross_in, uint32_t nin, uint64_t unit,
-    uint32_t* __restrict__ cross_out, uint32_t nout, EndBuild end)
+    uint32_t* __restrict__ cross_out, uint32_t nout, uint32_t per, EndBuild end)
 {
     __shared__ LevelLds<OCT, kCrossUnits / 64> S;
     __shared__ uint32_t sNode[kMaxLevel][kCrossUnits];
     __shared__ uint32_t sLevels;  // bit L: this unit holds input nodes of level L
-    const uint32_t i = blockIdx.x * kCrossUnits + threadIdx.x;
+    const uint32_t i = blockIdx.x * per + threadIdx.x;
+    const bool held = threadIdx.x < per && i < nin;
     const uint64_t lim = (static_cast<uint64_t>(blockIdx.x) + 1) * unit;
     int turn = 0;
     if (threadIdx.x < 2)
@@ -1670,7 +1678,7 @@ __global__ __launch_bounds__(kCrossUnits) void cross_moments_kernel(
     uint32_t has = 0u;
 #pragma unroll
     for (int L = 0; L < kMaxLevel; ++L) {
-        const uint32_t v = i < nin ? cross_in[static_cast<size_t>(L) * nin + i] : kNoNode;
+        const uint32_t v = held ? cross_in[static_cast<size_t>(L) * nin + i] : kNoNode;
         sNode[L][threadIdx.x] = v;
         has |= v != kNoNode ? 1u << L : 0u;
     }
@@ -1914,11 +1922,12 @@ bool launch_moments_t(Device& d, int rf, bool groups, bool end)
             tiles(std::integral_constant<int, 1>{}, 1);
         while (nin > 1) {
             uint32_t* out = in + static_cast<size_t>(kLevels) * nin;
-            const uint32_t nout = (nin + kCrossUnits - 1) / kCrossUnits;
-            unit *= kCrossUnits;
+            const uint32_t per_cross = nin > (OCT ? 384u : 512u) ? kCrossSplit : kCrossUnits;
+            const uint32_t nout = (nin + per_cross - 1) / per_cross;
+            unit *= per_cross;
             cross_moments_kernel<OCT><<<nout, kCrossUnits, 0, d.stream>>>(
                 d.nprefix, d.nstart, d.ncount, d.nchild, d.nfirst, d.geom, d.wnode, d.next, noct,
-                rf, d.err, in, nin, unit, out, nout, ending(nout == 1));
+                rf, d.err, in, nin, unit, out, nout, per_cross, ending(nout == 1));
             in = out;
             nin = nout;
         }

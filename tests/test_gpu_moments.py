@@ -71,3 +71,15 @@ def test_moments_of_units_of_several_tiles_and_full_levels(n, bucket):
         s.upload(pos, vel, mass)
         s.build_tree()
         _check(s.dump_tree())
+
+
+# With third moments (learned correction) 385 tiles go through two passes of straddling
+# nodes, 384 through one.
+@pytest.mark.parametrize("n", [393216, 393217])
+def test_moments_with_third_order(n):
+    pos, vel, m = B.plummer(n, seed=n)
+    with B.OctreeHip(n, theta=0.9, softening=0.01) as s:
+        s.lff_configure(theta=0.9, band=0.75, min_count=64)
+        s.upload(pos, vel, m)
+        s.build_tree()
+        _check(s.dump_tree())
