@@ -180,7 +180,9 @@ constexpr float kPadFar = 1.0e18f;  // its square is finite in FP32, its force z
 // WRAP: pairs take their nearest image (a periodic TreePM box). The walk shifts every
 // node to the image nearest to the group, so a pair needs its own only where an entry
 // lies half a box from some target (far_image in walk_kernel); elsewhere rounding the
-// separation to whole boxes gives 0, and the loops without it sum the same bits.
+// separation to whole boxes gives 0, and the loops without it sum the same terms (9 of
+// 45 VALU instructions a particle less). With the shorter cells below: VALU instructions
+// per 128^3 walk 1.77e9 -> 1.37e9, 2.42 -> 2.02 ms, still bound by VALU issue.
 template <int ORDER, bool TPM, bool WRAP, int DJ>
 __device__ inline void eval_cells_dj(const Cell* __restrict__ cl, int ncell, int j0, float tx,
                                      float ty, float tz, const WalkParams& P, float& ax, float& ay,
@@ -512,6 +514,8 @@ __device__ inline void far_flush(const uint32_t* __restrict__ fl, int nfl,
 
 // Pushes nodes first, first + 1, ... (1 to 8 of them) by at most three stores. One store
 // per child took as many turns as the wavefront's largest nc, of 6 VALU instructions.
+// With the leaf search below 44 of about 190 VALU instructions per traversal step: a
+// 65,536-particle step 624 -> 613 us, 128^3 TreePM forces 3.62 -> 3.52 ms.
 __device__ inline void push_children(int* __restrict__ to, int first, uint32_t nc)
 {
     typedef int int4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -1139,6 +1143,7 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
 //   relative        100,000: 374 / 286 / 296 / 616 260,000: 557 / 502 / 668 / -
 //                   500,000: 578 / 587 / 756 / -
 //   periodic TreePM  64^3:   492 / 450 / 541 / 881  128^3: 2250 / 2274 / 2505 / -
+//   (with every pair's image rounded; 1 wave at 128^3 now 1990)
 // The relative and TreePM walks, whose lists take longer per entry or flush
 // more often, gain from 2 waves up to 3.5 groups per slot. COM runs keep one
 // wave from 0.47 groups per slot on and under block time steps: adding a
