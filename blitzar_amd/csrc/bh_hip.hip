@@ -1259,7 +1259,8 @@ bh_hip_result_t bh_hip_upload(bh_hip_handle_t* h, const double* pos3, const doub
     // The store keeps its current order; each slot picks its caller index. One
     // staging buffer serves the three arrays in stream order (each copy lands
     // after the kernel that read the buffer before it); the call waits for the
-    // stream before it returns, so the caller's arrays are free then.
+    // stream before it returns, after a failed copy too, so the caller's arrays
+    // are free then.
     bool ok = zero_err(h) && stage_to_device(h, pos3, 3 * d.n * sizeof(double));
     if (ok) {
         bh::launch_from_caller(d, 0);
@@ -1279,8 +1280,10 @@ bh_hip_result_t bh_hip_upload(bh_hip_handle_t* h, const double* pos3, const doub
     h->ad_primed = false;
     h->have_tree = false;
     h->amag_valid = false;
-    if (!ok)
+    if (!ok) {
+        (void)hipStreamSynchronize(d.stream);
         return BH_HIP_INTERNAL_ERROR;
+    }
     return finish(h, "upload");
 }
 

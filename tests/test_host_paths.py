@@ -1,0 +1,60 @@
+"""Host side of the library's calls on a double of the HIP runtime (fake_hip.cpp):
+what they leave behind when a copy or an allocation fails, what they allocate and
+wait for, and how the events of a build add up. No GPU: kernels do nothing, so no
+result is looked at."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+fake.fake_extra_memory.restype = C.c_size_t
+import numpy as np
+import blitzar_amd as B
+def cube(n):
+    rng = np.random.default_rng(n)
+    return rng.random((n, 3)), rng.random((n, 3)), np.full(n, 1.0 / n, np.float32)
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake") / "libfake_hip.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-pthread", "-o", str(so),
+                    os.path.join(HERE, "fake_hip.cpp")], check=True)
+    return str(so)
+
+
+def run(fake, body):
+    """The body in a process of its own (the library binds to the double there)."""
+    p = subprocess.run([sys.executable, "-c", PRELUDE + body, fake], cwd=ROOT, timeout=120,
+                       capture_output=True, text=True)
+    assert p.returncode == 0, (p.returncode, p.stdout, p.stderr)
+    return p.stdout
+
+
+@pytest.mark.parametrize("copy", [0, 1, 2])
+def test_failed_upload_leaves_nothing_in_flight(fake, copy):
+    """The caller's arrays are free when bh_hip_upload returns, also where one of
+    its three copies failed; a later upload works."""
+    run(fake, f"""
+state = cube(1000)
+with B.OctreeHip(1000) as s:
+    fake.fake_fail_copy({copy})
+    try:
+        s.upload(*state)
+    except B.BhHipError as e:
+        assert "stage upload" in str(e), e
+    else:
+        raise SystemExit("the upload did not fail")
+    assert fake.fake_uploads() == 0
+    fake.fake_fail_copy(-1)
+    s.upload(*state)
+""")
