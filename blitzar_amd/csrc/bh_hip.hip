@@ -18,7 +18,6 @@
 #include <numeric>
 #include <random>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -399,8 +398,9 @@ bool copy_out(bh_hip_handle* h, void* dst, const void* src, size_t bytes, const 
         try {
             for (; nthreads < kCopyThreads; ++nthreads)
                 pool[nthreads] = std::thread(worker);
-        } catch (const std::system_error&) {
-            // no (more) threads: those that started do it, or the caller alone
+        } catch (...) {
+            // no (more) threads, or no memory for one: those that started do it, or
+            // the caller alone (nothing may leave here with threads running)
         }
     }
     bool ok = true;

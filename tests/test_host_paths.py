@@ -58,3 +58,19 @@ with B.OctreeHip(1000) as s:
     fake.fake_fail_copy(-1)
     s.upload(*state)
 """)
+
+
+@pytest.mark.parametrize("started", [0, 1, 3])
+def test_download_without_memory_for_its_threads(fake, started):
+    """A large copy out whose helper threads cannot all be started (no memory for
+    the next one) is emptied by those that were, or by the caller alone."""
+    run(fake, f"""
+n = 200000
+with B.OctreeHip(n) as s:
+    s.upload(*cube(n))
+    s.download()  # the ring and its events are there
+    fake.fake_fail_new({started})
+    pos, vel = s.download()
+    fake.fake_fail_new(-1)
+    assert np.isfinite(pos).all() and np.isfinite(vel).all()
+""")
