@@ -441,6 +441,15 @@ bool copy_out(bh_hip_handle* h, void* dst, const void* src, size_t bytes, const 
     return ok;
 }
 
+// copy_out behind kernels that may run for long: its helper threads spin until the
+// first chunk lands, so the kernels are waited for before they start (a copy without
+// helpers needs no wait of its own).
+bool copy_result(bh_hip_handle* h, void* dst, const void* src, size_t bytes, const char* what)
+{
+    return (bytes < kCopyThreadsMin || check(h, hipStreamSynchronize(h->d.stream), what)) &&
+           copy_out(h, dst, src, bytes, what);
+}
+
 // Device errors that no retry repairs (a node-capacity overflow is repaired
 // inside the force evaluation, see check_build).
 constexpr int kFatalBits =
@@ -1556,7 +1565,8 @@ bh_hip_result_t bh_hip_direct_forces_fp64(bh_hip_handle_t* h, const uint32_t* ta
         if (ok) {
             bh::launch_direct_fp64(d, dt, nt, h->p.softening, h->p.min_distance2, ws);
             ok = check(h, hipGetLastError(), "direct launch") &&
-                 copy_out(h, acc3, ws, 3 * static_cast<size_t>(nt) * sizeof(double), "direct out");
+                 copy_result(h, acc3, ws, 3 * static_cast<size_t>(nt) * sizeof(double),
+                             "direct out");
         }
         (void)hipStreamSynchronize(d.stream);
     }
@@ -2039,7 +2049,7 @@ bh_hip_result_t bh_hip_lff_forward(bh_hip_handle_t* h, const float* X, uint32_t 
     bh::launch_lff_forward(h->d, h->lff, h->lff_rows, n, dY);
     const bool ok =
         check(h, hipGetLastError(), "fwd") &&
-        copy_out(h, Y, dY, static_cast<size_t>(n) * bh::kLffOutputs * sizeof(float), "fwd Y");
+        copy_result(h, Y, dY, static_cast<size_t>(n) * bh::kLffOutputs * sizeof(float), "fwd Y");
     if (!ok)
         (void)hipStreamSynchronize(h->d.stream);
     return ok ? BH_HIP_OK : BH_HIP_INTERNAL_ERROR;

@@ -74,3 +74,18 @@ with B.OctreeHip(n) as s:
     fake.fake_fail_new(-1)
     assert np.isfinite(pos).all() and np.isfinite(vel).all()
 """)
+
+
+def test_kernels_are_done_before_their_copy_starts_threads(fake):
+    """The helper threads of a large copy out spin until its first chunk lands, so
+    they start only once the direct sum, or the network, has run."""
+    run(fake, """
+n = 200000
+with B.OctreeHip(n) as s:
+    s.upload(*cube(n))
+    alone = fake.fake_threads()
+    s.direct_forces_fp64(np.arange(n, dtype=np.uint32))  # 4.8 MB of results
+    assert fake.fake_waiting_threads() <= alone, (fake.fake_waiting_threads(), alone)
+    s.lff_forward(np.zeros((400000, 32), np.float32))
+    assert fake.fake_waiting_threads() <= alone, (fake.fake_waiting_threads(), alone)
+""")
