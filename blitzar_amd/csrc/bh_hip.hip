@@ -32,6 +32,8 @@ constexpr size_t kRingChunk = 2u << 20;
 constexpr size_t kRingChunkMin = 256u << 10;
 constexpr int kCopyThreads = 4;
 constexpr size_t kCopyThreadsMin = 4u << 20;
+// direct_forces_fp64: doubles of a workspace of its own (8 MB: about 38,000 targets)
+constexpr size_t kDirectWords = 1u << 20;
 
 // b0 build start, s0 sort start (after AABB + keys), s1 sort end, p1 after
 // the tie fix and permutation, t1 after the tree levels, b1 build end (after
@@ -1549,24 +1551,34 @@ bh_hip_result_t bh_hip_direct_forces_fp64(bh_hip_handle_t* h, const uint32_t* ta
             h->last_error = "direct_forces_fp64: target index out of range";
             return BH_HIP_INVALID_ARGUMENT;
         }
-    // workspace and targets in the staging buffer when they fit
+    // Workspace and targets in the staging buffer when they fit. Else in a buffer of
+    // at most kDirectWords, the targets in pieces of what the larger of the two
+    // holds (the workspace of all of them is 216 bytes per target, 1.8 GB for
+    // 8,388,608). A target's sum does not depend on the piece it is in.
     bh::Device& d = h->d;
-    const size_t words = bh::direct_fp64_words(d.n, nt);
-    const size_t need = words + (static_cast<size_t>(nt) + 1) / 2;
+    const uint32_t splits = bh::direct_fp64_splits(d.n, nt);
+    const auto need = [&](size_t k) { return bh::direct_fp64_words(k, splits) + (k + 1) / 2; };
+    const size_t room = std::max(3 * d.n, kDirectWords);
+    size_t piece = nt;
+    if (need(piece) > room)
+        piece = (room - 1) / need(8) * 8;
     double* ws = d.stage;
-    const bool own = need > 3 * d.n;
-    bool ok = !own || dalloc(h, &ws, need, "direct sum");
+    const bool own = need(piece) > 3 * d.n;
+    bool ok = !own || dalloc(h, &ws, need(piece), "direct sum");
     if (ok) {
-        uint32_t* dt = reinterpret_cast<uint32_t*>(ws + words);
         ensure_rank(h);
-        ok = check(h, hipMemcpyAsync(dt, targets, nt * sizeof(uint32_t), hipMemcpyHostToDevice,
-                                     d.stream),
-                   "targets");
-        if (ok) {
-            bh::launch_direct_fp64(d, dt, nt, h->p.softening, h->p.min_distance2, ws);
-            ok = check(h, hipGetLastError(), "direct launch") &&
-                 copy_result(h, acc3, ws, 3 * static_cast<size_t>(nt) * sizeof(double),
-                             "direct out");
+        uint32_t* dt = reinterpret_cast<uint32_t*>(ws + bh::direct_fp64_words(piece, splits));
+        for (size_t at = 0; ok && at < nt; at += piece) {
+            const uint32_t k = static_cast<uint32_t>(std::min(piece, nt - at));
+            ok = check(h, hipMemcpyAsync(dt, targets + at, k * sizeof(uint32_t),
+                                         hipMemcpyHostToDevice, d.stream),
+                       "targets");
+            if (ok) {
+                bh::launch_direct_fp64(d, dt, k, splits, h->p.softening, h->p.min_distance2, ws);
+                ok = check(h, hipGetLastError(), "direct launch") &&
+                     copy_result(h, acc3 + 3 * at, ws, 3 * static_cast<size_t>(k) * sizeof(double),
+                                 "direct out");
+            }
         }
         (void)hipStreamSynchronize(d.stream);
     }

@@ -423,11 +423,13 @@ void launch_from_caller(Device& d, int which);
 // (to: another buffer, pinned host memory included)
 void launch_to_caller(Device& d, int which, void* to = nullptr);
 void launch_init_ids(Device& d);
-// FP64 direct sum; ws_dev holds direct_fp64_words(n, nt) doubles, the result
-// (3 per target) first.
-size_t direct_fp64_words(size_t n, uint32_t nt);
-void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, double eps,
-                        double min_d2, double* ws_dev);
+// FP64 direct sum in `splits` ranges of sources, direct_fp64_splits of n and all
+// targets of the call; ws_dev holds direct_fp64_words(nt, splits) doubles, the
+// result (3 per target) first.
+uint32_t direct_fp64_splits(size_t n, uint32_t nt);
+size_t direct_fp64_words(size_t nt, uint32_t splits);
+void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, uint32_t splits,
+                        double eps, double min_d2, double* ws_dev);
 void launch_energy(Device& d, double* out_dev);
 void launch_potential(Device& d, const uint32_t* slots_dev, uint32_t ns, double eps,
                       double min_d2, double* out_dev);

@@ -462,29 +462,26 @@ void launch_to_caller(Device& d, int which, void* to)
         static_cast<double*>(to), d.id, src[0], src[1], src[2], d.n);
 }
 
-namespace {
 // Source ranges per target block: enough blocks for 8 per CU, in multiples of 8
 // (one range per XCD), at least 1,024 sources each.
-uint32_t direct_splits(size_t n, uint32_t nt)
+uint32_t direct_fp64_splits(size_t n, uint32_t nt)
 {
     const uint32_t tiles = (nt + kDirectTargets - 1) / kDirectTargets;
     const uint32_t want = 8u * ((256u + tiles - 1) / tiles);
     const uint32_t most = static_cast<uint32_t>(n / 1024);
     return std::max(1u, most >= 8u ? std::min(want, most / 8u * 8u) : most);
 }
-}  // namespace
 
-size_t direct_fp64_words(size_t n, uint32_t nt)
+size_t direct_fp64_words(size_t nt, uint32_t splits)
 {
-    return 3 * static_cast<size_t>(nt) * (direct_splits(n, nt) + 1);
+    return 3 * nt * (static_cast<size_t>(splits) + 1);
 }
 
-void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, double eps,
-                        double min_d2, double* ws_dev)
+void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, uint32_t splits,
+                        double eps, double min_d2, double* ws_dev)
 {
     if (nt == 0 || d.n == 0)
         return;
-    const uint32_t splits = direct_splits(d.n, nt);
     const uint32_t tiles = (nt + kDirectTargets - 1) / kDirectTargets;
     double* part = ws_dev + 3 * static_cast<size_t>(nt);
     const double eps2 = eps * eps;

@@ -36,3 +36,19 @@ def test_direct_sum_matches_oracle(oracle, n, nt, eps):
         S = (w * np.linalg.norm(d, axis=1)).sum()
         # a few FP64 roundings a term and at most n / 256 additions in a row
         assert np.abs(a[k] - ref[k]).max() <= 1e-13 * S, (k, i)
+
+
+# more targets than the workspace takes at once: two pieces and a ragged last one,
+# with ranges of sources below 8 and of 8
+@pytest.mark.parametrize("n, nt", [(3000, 200001), (20000, 60003)])
+def test_pieces_of_targets_sum_the_same(n, nt):
+    rng = np.random.default_rng(n)
+    pos = rng.standard_normal((n, 3))
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    t = rng.integers(0, n, nt).astype(np.uint32)
+    with B.OctreeHip(n, softening=0.01) as s:
+        s.upload(pos, None, m)
+        s.build_tree()
+        # (all n of them in one piece, in as many ranges)
+        one = s.direct_forces_fp64(np.arange(n, dtype=np.uint32))
+        assert np.array_equal(s.direct_forces_fp64(t), one[t])

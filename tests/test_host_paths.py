@@ -89,3 +89,16 @@ with B.OctreeHip(n) as s:
     s.lff_forward(np.zeros((400000, 32), np.float32))
     assert fake.fake_waiting_threads() <= alone, (fake.fake_waiting_threads(), alone)
 """)
+
+
+@pytest.mark.parametrize("n, nt", [(2000000, 2000000), (1000, 2000000), (300000, 300001)])
+def test_direct_sum_workspace_is_bounded(fake, n, nt):
+    """Many targets are worked through in pieces: nothing above 8 MB is allocated."""
+    run(fake, f"""
+with B.OctreeHip({n}) as s:
+    s.upload(*cube({n}))
+    s.direct_forces_fp64([0])
+    fake.fake_mark_memory()
+    s.direct_forces_fp64(np.arange({nt}, dtype=np.uint32) % {n})
+    assert fake.fake_extra_memory() <= 8 << 20, fake.fake_extra_memory()
+""")
