@@ -233,8 +233,10 @@ __device__ inline double rsqrt_fp64(double x)
 // (whose coordinates are scalars), so a source is loaded once per 8 pairs, and
 // block b takes range b mod splits: with splits a multiple of 8 the blocks of
 // one XCD share a range in its L2. Bound: FP64 VALU, about 18 instructions per
-// pair. SOFT (the softening keeps every pair finite and above min_d2): no
-// pair needs skipping, a coincident one adds exactly zero.
+// pair. SOFT (the softening keeps every pair finite and above min_d2): no pair
+// needs skipping, a coincident one adds exactly zero, and so does the target
+// itself, unless its mass is not finite (its block then skips pairs as without
+// softening).
 // 4,096 targets of 1,048,576: 2.8 ms against 10.8 ms with one block per target,
 // a division and a square root per pair.
 constexpr int kDirectTargets = 8;
@@ -254,31 +256,37 @@ __global__ __launch_bounds__(256) void direct_fp64_kernel(
     const uint32_t hi = static_cast<uint32_t>(static_cast<uint64_t>(n) * (split + 1) / splits);
     uint32_t self[T];
     double x[T], y[T], z[T], ax[T], ay[T], az[T];
+    bool finite = true;
 #pragma unroll
     for (int k = 0; k < T; ++k) {
         self[k] = rank[targets[min(t0 + k, nt - 1)]];
         x[k] = px[self[k]];
         y[k] = py[self[k]];
         z[k] = pz[self[k]];
+        finite = finite && isfinite(pm[self[k]]);
         ax[k] = ay[k] = az[k] = 0.0;
     }
-    for (uint32_t j = lo + threadIdx.x; j < hi; j += 256u) {
-        const double sx = px[j], sy = py[j], sz = pz[j];
-        const double m = static_cast<double>(pm[j]);
+    const auto sum = [&](auto all) {  // all: every pair counts
+        for (uint32_t j = lo + threadIdx.x; j < hi; j += 256u) {
+            const double sx = px[j], sy = py[j], sz = pz[j];
+            const double m = static_cast<double>(pm[j]);
 #pragma unroll
-        for (int k = 0; k < T; ++k) {
-            const double dx = sx - x[k], dy = sy - y[k], dz = sz - z[k];
-            const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, eps2)));
-            const double inv = rsqrt_fp64(r2);
-            double s = m * inv * (inv * inv);
-            if (!SOFT)
-                s = j != self[k] && !(r2 <= min_d2) ? s : 0.0;
-            const bool use = SOFT || s != 0.0;  // a skipped pair's dx may be infinite
-            ax[k] = use ? fma(dx, s, ax[k]) : ax[k];
-            ay[k] = use ? fma(dy, s, ay[k]) : ay[k];
-            az[k] = use ? fma(dz, s, az[k]) : az[k];
+            for (int k = 0; k < T; ++k) {
+                const double dx = sx - x[k], dy = sy - y[k], dz = sz - z[k];
+                const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, eps2)));
+                const double inv = rsqrt_fp64(r2);
+                const double s = m * inv * (inv * inv);
+                const bool use = all || (j != self[k] && !(r2 <= min_d2));
+                ax[k] = use ? fma(dx, s, ax[k]) : ax[k];
+                ay[k] = use ? fma(dy, s, ay[k]) : ay[k];
+                az[k] = use ? fma(dz, s, az[k]) : az[k];
+            }
         }
-    }
+    };
+    if (SOFT && finite)
+        sum(std::true_type{});
+    else
+        sum(std::false_type{});
     const int w = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < T; ++k) {
@@ -485,15 +493,12 @@ void launch_direct_fp64(Device& d, const uint32_t* targets_dev, uint32_t nt, uin
     const uint32_t tiles = (nt + kDirectTargets - 1) / kDirectTargets;
     double* part = ws_dev + 3 * static_cast<size_t>(nt);
     const double eps2 = eps * eps;
-    // (the softened kernel: m / eps^3 stays finite for any FP32 mass)
-    if (eps >= 1e-60 && min_d2 <= eps2)
-        direct_fp64_kernel<true><<<tiles * splits, 256, 0, d.stream>>>(
-            targets_dev, nt, d.rank, d.pos[0], d.pos[1], d.pos[2], d.mass,
-            static_cast<uint32_t>(d.n), eps2, min_d2, splits, part);
-    else
-        direct_fp64_kernel<false><<<tiles * splits, 256, 0, d.stream>>>(
-            targets_dev, nt, d.rank, d.pos[0], d.pos[1], d.pos[2], d.mass,
-            static_cast<uint32_t>(d.n), eps2, min_d2, splits, part);
+    // (the softened kernel: m / eps^3 stays finite for any finite FP32 mass)
+    const auto kernel = eps >= 1e-60 && min_d2 <= eps2 ? direct_fp64_kernel<true>
+                                                       : direct_fp64_kernel<false>;
+    kernel<<<tiles * splits, 256, 0, d.stream>>>(
+        targets_dev, nt, d.rank, d.pos[0], d.pos[1], d.pos[2], d.mass, static_cast<uint32_t>(d.n),
+        eps2, min_d2, splits, part);
     direct_sum_kernel<<<(nt + 3) / 4, 256, 0, d.stream>>>(part, nt, splits, ws_dev);
 }
 

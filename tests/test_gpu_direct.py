@@ -52,3 +52,34 @@ def test_pieces_of_targets_sum_the_same(n, nt):
         # (all n of them in one piece, in as many ranges)
         one = s.direct_forces_fp64(np.arange(n, dtype=np.uint32))
         assert np.array_equal(s.direct_forces_fp64(t), one[t])
+
+
+# a target's own mass is no part of its force, whatever it is; a pair that is
+# neither the target itself nor below min_distance2 counts, at infinity too
+@pytest.mark.parametrize("eps", [0.01, 0.0])
+@pytest.mark.parametrize("odd", [np.inf, -np.inf, np.nan])
+def test_direct_sum_of_values_that_are_not_finite(oracle, eps, odd):
+    n, k = 3001, 1234
+    rng = np.random.default_rng(5)
+    pos = rng.standard_normal((n, 3))
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    t = np.array([k - 1, k, k + 1, 7, n - 1], np.uint32)
+    far = pos.copy()
+    far[k, 0] = odd
+    heavy = m.copy()
+    heavy[k] = odd
+    with B.OctreeHip(n, softening=eps, min_softening=0.0, min_distance2=0.0) as s:
+        s.upload(pos, None, heavy)
+        a = s.direct_forces_fp64(t)
+        s.upload(far, None, m)
+        f = s.direct_forces_fp64(t)
+    light = m.astype(np.float64)
+    light[k] = 0.0
+    e = float(np.float32(eps))
+    ref = oracle.direct_fp64(pos, light, np.array([k], np.int32), e, 0.0)[0]
+    # (the target with the mass that is not finite: FP64 roundings of a sum of |terms|)
+    d = pos - pos[k]
+    w = light * np.maximum((d * d).sum(1) + e * e, 1e-100) ** -1.5
+    assert np.abs(a[1] - ref).max() <= 1e-13 * (w * np.linalg.norm(d, axis=1)).sum()
+    assert not np.isfinite(a[[0, 2, 3, 4]]).any()
+    assert np.isnan(f[:, 0]).all()
