@@ -36,13 +36,14 @@ constexpr size_t kCopyThreadsMin = 4u << 20;
 constexpr size_t kDirectWords = 1u << 20;
 
 // b0 build start, s0 sort start (after AABB + keys), s1 sort end, p1 after
-// the tie fix and permutation, t1 after the tree levels, b1 build end (after
-// moments and groups), w1 walk end.
+// the tie fix and permutation, t1 after the topology, j1 after both, b1 build end
+// (after moments and groups), w1 walk end.
 struct StepEvents {
     hipEvent_t b0 = nullptr, s0 = nullptr, s1 = nullptr, p1 = nullptr, t1 = nullptr,
                j1 = nullptr, b1 = nullptr, w1 = nullptr;
     hipEvent_t l0 = nullptr;  // learned correction start (after its walk)
     bool l0_used = false;
+    bool one_stream = false;  // the permutation starts at t1, not beside the topology at s1
 };
 
 // Start and end of one kick / kick-drift launch (read at the end of the call,
@@ -640,7 +641,10 @@ void queue_build(bh_hip_handle* h, StepEvents* ev)
         bh::launch_radix_sort(d, d.n, h->p.key_mode == 1 ? 30 : 63);
     }
     rec(ev ? ev->s1 : nullptr, d.stream);
-    if (d.n <= kOneStreamMax) {
+    const bool one_stream = d.n <= kOneStreamMax;
+    if (ev)
+        ev->one_stream = one_stream;
+    if (one_stream) {
         bh::launch_tree_build(d, h->leaf_depth, h->p.bucket_capacity, d.stream);
         rec(ev ? ev->t1 : nullptr, d.stream);
         bh::launch_permute_all(d, d.stream);
@@ -861,7 +865,7 @@ void end_call(bh_hip_handle* h)
             span(e.b0, e.b1, t.build_ms);
             span(e.b0, e.s0, t.keys_ms);
             span(e.s0, e.s1, t.sort_ms);
-            span(e.s1, e.p1, t.permute_ms);
+            span(e.one_stream ? e.t1 : e.s1, e.p1, t.permute_ms);
             span(e.s1, e.t1, t.tree_ms);
             span(e.j1, e.b1, t.moments_ms);
             span(e.b1, e.w1, t.walk_ms);

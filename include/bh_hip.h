@@ -134,7 +134,8 @@ typedef struct bh_hip_handle bh_hip_handle_t;
  * bh_hip_set_timing) and walk interaction counts. */
 typedef struct bh_hip_timings {
     double build_ms;      /* AABB + keys + sort + permute + tree + moments */
-    double sort_ms;       /* radix sort alone */
+    double sort_ms;       /* sort of the keys, which also makes them on builds of up to
+                             4,194,304 particles (part of build_ms) */
     double walk_ms;       /* tree walk */
     double integrate_ms;  /* kick/drift kernels */
     uint64_t pp_interactions; /* particle-particle interactions (sum over timed walks) */
@@ -152,11 +153,14 @@ typedef struct bh_hip_timings {
     /* parts of build_ms */
     double keys_ms;     /* AABB, and the Morton keys unless the sort makes them
                            (builds of up to 4,194,304 particles) */
-    double permute_ms;  /* equal-key tie order + store permutation */
-    double tree_ms;     /* topology, from the end of the sort (it runs beside the
-                           permutation, on a second stream) */
-    double moments_ms;  /* moments and leaf packing, after the topology, until the
-                           walk groups (second stream, beside them) are done */
+    /* builds of up to 200,000 particles run on one stream: there the parts follow one
+     * another and add up to build_ms */
+    double permute_ms;  /* equal-key tie order + store permutation (beyond 200,000
+                           particles positions and masses only, beside the topology) */
+    double tree_ms;     /* topology, from the end of the sort */
+    double moments_ms;  /* moments, leaf packing and walk groups (beyond 200,000
+                           particles until the rest of the store and the groups, on
+                           the second stream, are done too) */
     uint64_t lff_pairs; /* learned correction: (target, node) pairs evaluated */
     uint64_t lff_tiles; /* learned correction: 16-pair MFMA tiles run */
     double lff_ms;      /* learned correction: the MLP pass (part of walk_ms) */

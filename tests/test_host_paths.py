@@ -102,3 +102,19 @@ with B.OctreeHip({n}) as s:
     s.direct_forces_fp64(np.arange({nt}, dtype=np.uint32) % {n})
     assert fake.fake_extra_memory() <= 8 << 20, fake.fake_extra_memory()
 """)
+
+
+@pytest.mark.parametrize("n", [1000, 150000])
+def test_parts_of_a_one_stream_build_add_up(fake, n):
+    """The parts of a build whose kernels run one after the other sum to the whole
+    (the double's events count kernels)."""
+    run(fake, f"""
+with B.OctreeHip({n}) as s:
+    s.upload(*cube({n}))
+    B.lib().bh_hip_set_timing(s._h, 1)
+    s.build_tree()
+    t = s.timings()
+    parts = [t[k] for k in ("keys_ms", "sort_ms", "permute_ms", "tree_ms", "moments_ms")]
+    assert min(parts) > 0 and sum(parts) == t["build_ms"], (parts, t["build_ms"])
+    assert t["permute_ms"] == 1, t  # one launch
+""")
