@@ -62,3 +62,32 @@ def test_periodic_short_range_walk(oracle, n):
     # the split weight errs by 1.6e-7, separations of neighbours by FP32 rounding
     assert np.abs(a[t] - ref).max() <= 2e-5 * scale
 
+
+
+# The extent criterion, on either side of the lines where it takes 8, 4 and 1 waves
+# per group on a 256-CU GPU. The particles lie in 216 clumps of radius 1e-3 on a
+# lattice of spacing 0.2: a cell of several clumps has bmax >= 0.1 and is opened
+# (theta R <= 0.05 x 1.74), a clump is accepted whole from outside, where its
+# expansion is exact to (1e-3 / 0.2)^3. So the lists hold one cell or the particles of
+# every clump, and what is left is FP32 rounding: of the terms, as above, and of
+# positions up to 1, 2.4e-7 times the gradient 1 / R^3 of each term.
+@pytest.mark.parametrize("n", [1009, 35001, 36001, 311001, 313001])
+def test_extent_walk_of_clumps_matches_direct_sum(n):
+    rng = np.random.default_rng(n)
+    k = np.arange(n) % 216
+    eps = float(np.float32(0.05))
+    pos = 0.2 * np.stack([k // 36, k // 6 % 6, k % 6], 1)
+    v = rng.standard_normal((n, 3))
+    pos += 1e-3 * v / np.maximum(np.linalg.norm(v, axis=1, keepdims=True), 1.0)
+    mass = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    t = np.unique(np.linspace(0, n - 1, 48).astype(np.uint32))
+    with B.OctreeHip(n, theta=0.05, softening=0.05, criterion="extent", multipole_order=2) as s:
+        s.upload(pos, None, mass)
+        a = s.compute_accelerations()
+        assert np.array_equal(s.compute_accelerations(), a)
+        ref = s.direct_forces_fp64(t)
+    for j, i in enumerate(t):
+        d = pos - pos[i]
+        r3 = ((d * d).sum(1) + eps * eps) ** -1.5
+        S = (mass * np.linalg.norm(d, axis=1) * r3).sum()
+        assert np.linalg.norm(a[i] - ref[j]) <= 1e-5 * S + 2.4e-7 * (mass * r3).sum(), (n, i)
