@@ -43,6 +43,7 @@ struct StepEvents {
                j1 = nullptr, b1 = nullptr, w1 = nullptr;
     hipEvent_t l0 = nullptr;  // learned correction start (after its walk)
     bool l0_used = false;
+    bool walked = false;      // w1 is recorded (a build alone, or one that failed, has no walk)
     bool one_stream = false;  // the permutation starts at t1, not beside the topology at s1
 };
 
@@ -558,7 +559,7 @@ StepEvents* next_events(bh_hip_handle* h)
         h->events.push_back(e);
     }
     StepEvents* ev = &h->events[h->events_used++];
-    ev->l0_used = false;
+    ev->l0_used = ev->walked = false;
     return ev;
 }
 
@@ -583,6 +584,14 @@ void rec(hipEvent_t e, hipStream_t s)
 {
     if (e)
         (void)hipEventRecord(e, s);
+}
+
+void end_walk(bh_hip_handle* h, StepEvents* ev)
+{
+    if (!ev)
+        return;
+    rec(ev->w1, h->d.stream);
+    ev->walked = true;
 }
 
 // Walk-group size. A walk keeps about cu_count * 24 waves resident and
@@ -831,7 +840,7 @@ bool queue_force(bh_hip_handle* h)
             return false;
         }
     }
-    rec(ev ? ev->w1 : nullptr, h->d.stream);
+    end_walk(h, ev);
     h->primed = true;
     return true;
 }
@@ -868,8 +877,9 @@ void end_call(bh_hip_handle* h)
             span(e.one_stream ? e.t1 : e.s1, e.p1, t.permute_ms);
             span(e.s1, e.t1, t.tree_ms);
             span(e.j1, e.b1, t.moments_ms);
-            span(e.b1, e.w1, t.walk_ms);
-            if (e.l0_used)
+            if (e.walked)
+                span(e.b1, e.w1, t.walk_ms);
+            if (e.walked && e.l0_used)
                 span(e.l0, e.w1, t.lff_ms);
         }
         for (size_t k = 0; k < h->int_used; ++k) {
@@ -965,7 +975,7 @@ bool build_and_walk(bh_hip_handle* h, StepEvents* ev, const bh::WalkParams& wp, 
         launch_force_walk(h, w);
         const Built b = check_build(h);
         if (b == Built::kOk) {
-            rec(ev ? ev->w1 : nullptr, h->d.stream);
+            end_walk(h, ev);
             return true;
         }
         if (b == Built::kFatal)

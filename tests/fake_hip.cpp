@@ -53,6 +53,7 @@ struct Launch {
     void* stream;
 };
 thread_local Launch pending_launch;
+thread_local int last_error = kOk;
 }  // namespace
 
 void* operator new(size_t n)
@@ -99,7 +100,12 @@ int hipGetDeviceCount(int* n) { return *n = 1, kOk; }
 int hipGetDevice(int* d) { return *d = 0, kOk; }
 int hipGetDevicePropertiesR0600(void*, int) { return kError; }
 const char* hipGetErrorString(int) { return "injected"; }
-int hipGetLastError() { return kOk; }
+int hipGetLastError()
+{
+    const int e = last_error;
+    last_error = kOk;
+    return e;
+}
 int hipMalloc(void** p, size_t n)
 {
     size_t* q = static_cast<size_t*>(std::calloc(n + 64, 1));
@@ -139,9 +145,9 @@ int hipStreamCreateWithFlags(void** s, unsigned) { return *s = std::malloc(1), k
 int hipStreamDestroy(void* s) { return std::free(s), kOk; }
 int hipStreamSynchronize(void*) { return wait(); }
 int hipStreamWaitEvent(void*, void*, unsigned) { return kOk; }
-int hipEventCreate(void** e) { return *e = std::calloc(1, sizeof(long)), kOk; }
+int hipEventCreate(void** e) { return *e = new long(-1), kOk; }  // not recorded
 int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
-int hipEventDestroy(void* e) { return std::free(e), kOk; }
+int hipEventDestroy(void* e) { return delete static_cast<long*>(e), kOk; }
 int hipEventRecord(void* e, void*) { return *static_cast<long*>(e) = ticks, kOk; }
 int hipEventSynchronize(void*)
 {
@@ -151,7 +157,10 @@ int hipEventSynchronize(void*)
 }
 int hipEventElapsedTime(float* ms, void* a, void* b)
 {
-    *ms = static_cast<float>(*static_cast<long*>(b) - *static_cast<long*>(a));
+    const long x = *static_cast<long*>(a), y = *static_cast<long*>(b);
+    if (x < 0 || y < 0)
+        return last_error = kError;  // and the thread's last error, as the runtime keeps it
+    *ms = static_cast<float>(y - x);
     return kOk;
 }
 }

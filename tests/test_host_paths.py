@@ -118,3 +118,22 @@ with B.OctreeHip({n}) as s:
     assert min(parts) > 0 and sum(parts) == t["build_ms"], (parts, t["build_ms"])
     assert t["permute_ms"] == 1, t  # one launch
 """)
+
+
+@pytest.mark.parametrize("n", [1000, 300000])
+def test_timed_builds_without_a_walk(fake, n):
+    """bh_hip_build_tree with timing on: no walk ends, so none is read (an event never
+    recorded left an error that failed the next call; one of an earlier call gave a
+    negative time)."""
+    run(fake, f"""
+with B.OctreeHip({n}) as s:
+    s.upload(*cube({n}))
+    B.lib().bh_hip_set_timing(s._h, 1)
+    for k in range(3):
+        s.build_tree()
+        assert s.timings()["walk_ms"] == 0 and s.timings()["build_ms"] > 0
+    s.compute_accelerations(to_host=False)
+    assert s.timings()["walk_ms"] > 0
+    s.build_tree()
+    assert s.timings()["walk_ms"] == 0
+""")
