@@ -2,10 +2,12 @@
 // management and the per-step orchestration of the HIP kernels.
 //
 // Step structure (leapfrog), after the first force evaluation:
-//   kick_drift(dt/2, dt) -> AABB -> keys -> radix sort -> tie fix -> permute
-//   -> tree levels -> moments -> walk -> kick(dt/2)
-// All of it is queued on the handle's stream without host synchronisation;
-// the host synchronises once per API call to report device-side errors.
+//   kick_drift(dt/2, dt) -> AABB -> keys and sort -> topology, tie order and
+//   permutation -> moments and walk groups -> walk -> kick(dt/2)
+// queued on the handle's stream; above 200,000 particles the topology, the rest of
+// the store and the groups run on a second stream beside the permutation and the
+// moments (queue_build). The host waits for a build's error word, while the walk
+// behind it runs, and for the stream at the end of each API call.
 #include "../../include/bh_hip.h"
 #include "bh_internal.h"
 

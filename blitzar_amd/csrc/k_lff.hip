@@ -369,9 +369,9 @@ __global__ __launch_bounds__(64) void lff_tuple_kernel(
 //     LDS as [unit][sample] rows, and wave w sums its 16 rows (of W2 and W3) or
 //     columns (of W1) over the chunk's 64 samples, so the workgroup holds one
 //     copy of the gradient in registers (28 per lane).
-// Bound: FP32 matrix issue, 292 MFMA of 32 cycles per 16 samples (15 us for
-// 65,536 samples on the card), one wave per SIMD by LDS (127 KB). The
-// lane-per-sample vector form took 503 us for 65,536 samples, this one 46 us.
+// Bound: latency of a chunk, with one wave per SIMD by LDS (127 KB) and the barriers
+// between a chunk's parts: 46 us for 65,536 samples, of which FP32 matrix issue (292
+// MFMA of 32 cycles per 16 samples) is 15. The lane-per-sample vector form took 503.
 constexpr int kGradChunk = 64;
 constexpr int kGradRow = kGradChunk + 4;  // float4-aligned rows, banks spread
 

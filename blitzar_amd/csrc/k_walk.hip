@@ -13,17 +13,19 @@
 // (pair force engine/physics/octree/force/OctreeForce.cpp:23-57); the sum is
 // clamped to max_acceleration (engine/physics/octree/force/OctForces.cpp:128-133).
 //
-// MI355X mapping. One 64-lane workgroup (one wavefront) owns a group of at
-// most 64 targets (one target per lane) -- the particles of one tree node, so
-// the group is spatially compact -- and walks the tree once for the whole
-// group. A node is accepted only when the criterion holds for every
+// MI355X mapping. One workgroup owns a group of at most 64 targets (one target
+// per lane) -- the particles of one tree node, so the group is spatially compact
+// -- and walks the tree once for the whole group: one wavefront where there are
+// groups enough to fill the chip, 2, 4 or 8 that share the lists and the stack
+// where there are not (walk_waves). A node is accepted only when the criterion holds for every
 // point of the group's bounding box (distance measured from the box, which is
 // conservative), and only when no target lies within the node's bounding
 // sphere (bmax) -- the group form of the reference's "contains self" test.
 // Accepted nodes (monopole + traceless quadrupole) and the particles of opened
-// leaves are staged in LDS lists and evaluated by all 64 lanes with broadcast
-// LDS reads. Traversal keeps a LIFO of node indices in global memory, popped
-// 64 at a time. Groups are handed out by an atomic ticket; every workgroup
+// leaves are staged in LDS lists and evaluated by all lanes with broadcast LDS
+// reads. Traversal keeps a LIFO of node indices, popped 64 per wavefront at a
+// time, in global memory (its top in LDS where several wavefronts share it).
+// Groups are handed out by an atomic ticket; every workgroup
 // exits when the ticket passes the group count.
 //
 // Precision: positions in the walk are FP32 offsets from the exact lattice
@@ -46,9 +48,9 @@ namespace {
 
 // LDS list capacities (cells flush at kCellCap - 64, particles at kPartCap);
 // together with the leaf descriptors they set the LDS per wavefront and so
-// the walk's residency: 96 and 96 take 6.5 KB (24 waves per CU by LDS, 20 by
-// VGPRs) where 128 and 128 took 8.3 KB (18 waves per CU); the relative walk
-// is 2 % faster at 8M.
+// the walk's residency: 96 and 96, cells of 48 bytes, take 7.4 KB (22 waves per
+// CU by LDS, 20 by VGPRs in the relative walk). Chosen with cells of 40 bytes: 6.5 KB
+// against 8.3 KB (18 waves per CU) for 128 and 128, the relative walk 2 % faster at 8M.
 #ifndef BH_WALK_CELL_CAP
 #define BH_WALK_CELL_CAP 96
 #endif
@@ -1146,8 +1148,9 @@ __global__ __launch_bounds__(64 * W, FAR ? 1 : W > 1 ? 4 : BH_WALK_MIN_WAVES) vo
 //   (with every pair's image rounded; 1 wave at 128^3 now 1990)
 // The relative and TreePM walks, whose lists take longer per entry or flush
 // more often, gain from 2 waves up to 3.5 groups per slot. COM runs keep one
-// wave from 0.47 groups per slot on and under block time steps: adding a
-// target's terms in another order moves its FP32 force by 2e-7 (4,096
+// wave from 0.47 groups per slot on and under block time steps. That is a choice,
+// no limit (against FP64 either order errs the same): adding a target's terms in
+// another order moves its FP32 force by 2e-7 (4,096
 // particles) to 5e-7 (65,536), which an FP64 state integrated over tens of steps
 // shows (1.6e-9 of the velocities after 20 steps at 65,536), for 7 % of the walk
 // there. The count depends on n, the criterion and the GPU only; the recording

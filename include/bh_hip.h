@@ -265,7 +265,9 @@ bh_hip_result_t bh_hip_get_last_error(bh_hip_handle_t* h, char* buf, size_t cap)
 typedef struct bh_hip_lff_config {
     float theta;       /* opening angle of the corrected walk (e.g. 0.9) */
     float band;        /* near nodes: size / distance >= band */
-    int32_t list_cap;  /* nodes recorded per target group (0 = default 192) */
+    int32_t list_cap;  /* nodes recorded per target group (0 = default 192); a group
+                          whose list is full opens its further near nodes, and which
+                          those are follows the order of the walk */
     int32_t enabled;   /* 1: force evaluations and steps use the corrected walk */
     int32_t min_count; /* near nodes with fewer particles are opened (summed at
                           the angle `band`) instead of corrected (default 32) */
@@ -310,8 +312,8 @@ bh_hip_result_t bh_hip_pm_accelerations(bh_hip_handle_t* h, float* acc3);
  * adaptive step. */
 bh_hip_result_t bh_hip_adaptive_levels(bh_hip_handle_t* h, int32_t* levels);
 
-/* Standalone stable radix sort of (key, value) pairs on the device, the
- * building block behind thrust::sort_by_key at OctBuild.inl:96. Sorts by the
+/* Standalone stable sort of (key, value) pairs on the device, the building
+ * block behind thrust::sort_by_key at OctBuild.inl:96. Sorts by the
  * low key_bits bits (1..64); host arrays in and out. */
 bh_hip_result_t bh_hip_sort_pairs(const uint64_t* keys, const uint32_t* vals, uint64_t n,
                                   int32_t key_bits, uint64_t* keys_out, uint32_t* vals_out,
